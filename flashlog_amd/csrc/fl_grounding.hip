@@ -199,26 +199,32 @@ __device__ __forceinline__ GrOpts gr_side_reg(const GrSide &s, int32_t off, int6
 struct GrScratch {
     uint64_t *skey;
     int32_t *sgrp;
-    int32_t *oop, *ostart, *otake;
+    int4 *oopt;     // {operator, first position, edges taken, 0}
     double *omass;
 };
 
 // Hub cache: per (head slot, step, rank) combination c and hub h, the
-// node's option lists (fw options, then inv options) with cumulative masses
-// at c * nopt + hub_off[h], and the header {fw count, inv count, total}.
-struct GrHubHdr {
-    int32_t nf, ni;
+// node's options (forward ones, then inverse ones) with cumulative masses at
+// c * nopt + hub_off[h], and a header that one load fetches: hub_off[h], the
+// number of options with the identity's presence in the top bit, and the
+// total mass.
+struct __align__(16) GrHubHdr {
+    uint32_t off;
+    uint32_t n;
     double total;
-    int64_t off;  // first option slot in the pool
 };
+constexpr uint32_t GR_HDR_ID = 0x80000000u;
 
 struct GrHubPool {
     GrHubHdr *hdr;                // [combos][nhub]
-    int32_t *op, *start, *take;   // [combos][nopt]
+    int4 *opt;                    // [combos][nopt]
     double *cum;                  // [combos][nopt]
     const int32_t *hub_id, *hub_node;
     const int64_t *hub_off;
     int64_t nhub, nopt;
+    // hubs of at most GR_SMALL groups a side, then (from the end) the others,
+    // and how many of each there are
+    int32_t *list, *nlist;
 };
 
 // Options of a side of up to 64*RR groups (RR keys per lane, element
@@ -299,9 +305,7 @@ __device__ __forceinline__ int gr_side_regsort(const GrSide &s, int32_t off, int
         take = take > 0 ? take : 0;
         if (take > 0) {
             const int32_t op = (int32_t)(key[r] & 0xFFFFFFFFull);
-            sc.oop[o + n + lane] = op;
-            sc.ostart[o + n + lane] = s.start[g];
-            sc.otake[o + n + lane] = (int32_t)take;
+            sc.oopt[o + n + lane] = make_int4(op, s.start[g], (int32_t)take, 0);
             sc.omass[o + n + lane] = __dmul_rn(gr_proposal(w[op], temp), (double)take);
         }
         n += __popcll(__ballot(take > 0));
@@ -365,9 +369,7 @@ __device__ __forceinline__ int gr_side_mem(const GrSide &s, int32_t off, int64_t
         take = take > 0 ? take : 0;
         if (take > 0) {
             const int32_t op = (int32_t)(key & 0xFFFFFFFFull);
-            sc.oop[o + n + lane] = op;
-            sc.ostart[o + n + lane] = s.start[g];
-            sc.otake[o + n + lane] = (int32_t)take;
+            sc.oopt[o + n + lane] = make_int4(op, s.start[g], (int32_t)take, 0);
             sc.omass[o + n + lane] = __dmul_rn(gr_proposal(w[op], temp), (double)take);
         }
         n += __popcll(__ballot(take > 0));
@@ -459,19 +461,133 @@ __device__ __forceinline__ void gr_option(const GrOpts &o, const GrScratch &sc, 
         *start = __shfl(o.start, i, FL_WAVE);
         *take = __shfl(o.take, i, FL_WAVE);
     } else {
-        *op = sc.oop[obase + i];
-        *start = sc.ostart[obase + i];
-        *take = sc.otake[obase + i];
+        const int4 x = sc.oopt[obase + i];
+        *op = x.x;
+        *start = x.y;
+        *take = x.z;
     }
 }
 
 constexpr int GR_NT = 64;
 constexpr int64_t GR_LDS_SORT_MAX = 4096;  // groups per side sorted in LDS (48 KB)
 
-// Hub cache fill, wave per (combination, hub) (grid-stride): the hub's
-// options ranked and their masses accumulated exactly as a walk step does
-// (no excluded operator), written to the pool; the sort scratch of large
-// sides is the block's walk scratch.
+// The hubs by size: those whose two sides fit a row of 16 lanes each, and the
+// others (in any order within a kind: each is filled by itself).
+constexpr int GR_SMALL = 16;
+
+__global__ void k_gr_kinds(GrGraph gg, GrHubPool hp) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= hp.nhub) return;
+    const int32_t node = hp.hub_node[i];
+    const bool small = gg.fw.ptr[node + 1] - gg.fw.ptr[node] <= GR_SMALL &&
+                       gg.inv.ptr[node + 1] - gg.inv.ptr[node] <= GR_SMALL;
+    const unsigned long long sm = __ballot(small), all = __ballot(true);
+    const unsigned long long mine = small ? sm : all & ~sm;
+    const int lane = fl_lane(), lead = __ffsll((long long)mine) - 1;
+    int at = 0;
+    if (lane == lead) at = atomicAdd(&hp.nlist[small ? 0 : 1], __popcll(mine));
+    at = __shfl(at, lead, FL_WAVE) + __popcll(mine & ((1ull << lane) - 1));
+    hp.list[small ? at : hp.nhub - 1 - at] = (int32_t)i;
+}
+
+// Small hubs, two (combination, hub) pairs a wave: lanes 0..15 of a half hold
+// the forward groups, 16..31 the inverse ones.  A group's place is the number
+// of keys of its row below its own (15 row rotations: a third of the
+// instructions of a wave-wide network on keys that mostly do not exist);
+// takes, masses and the sequential sum of masses as in a walk step.  C3,
+// 16 heads x 3 ranks: all 2.1 M lists 5.8 ms by k_gr_hubs alone.
+__global__ __launch_bounds__(256) void k_gr_small(GrGraph gg, GrHubPool hp, const float *__restrict__ att,
+                                                 int64_t ranks, int64_t vocab, int64_t ncombo, int64_t topk,
+                                                 double temp) {
+    __shared__ double mass_all[256];
+    const int lane = fl_lane();
+    const int l16 = lane & 15, side = (lane >> 4) & 1, row0 = lane & 48;
+    double *mass_lds = mass_all + (threadIdx.x & ~31);
+    const int64_t nsmall = hp.nlist[0];
+    const int64_t pairs = ncombo * nsmall;
+    const int32_t R = gg.R;
+    const int32_t tk = (int32_t)(topk < 0x7FFFFFFF ? topk : 0x7FFFFFFF);
+    const int64_t halves = (int64_t)gridDim.x * (256 / 32);
+    for (int64_t u = (int64_t)blockIdx.x * (256 / 32) + (threadIdx.x >> 5); __ballot(u < pairs) != 0; u += halves) {
+        const bool live = u < pairs;
+        const int64_t uu = live ? u : 0;
+        const int64_t combo = uu / nsmall;
+        const int32_t hid = hp.list[uu - combo * nsmall];
+        const int32_t node = hp.hub_node[hid];
+        const int64_t hslot = combo / (3 * ranks), step = (combo / ranks) % 3, rank = combo % ranks;
+        const float *w = att + hslot * 3 * ranks * vocab + (step * ranks + rank) * vocab;
+        const GrSide &s = side ? gg.inv : gg.fw;
+        const int32_t g0 = s.ptr[node], G = s.ptr[node + 1] - g0;
+        int32_t op = 0, start = 0, cnt = 0;
+        float wv = 0.0f;
+        if (l16 < G) {
+            op = (int32_t)s.rel[g0 + l16] + (side ? R : 0);
+            start = s.start[g0 + l16];
+            cnt = s.count[g0 + l16];
+            wv = w[op];
+        }
+        // weight descending, then group order (operators ascend with it);
+        // groups without a say last
+        const bool el = wv > 0.0f && cnt > 0;
+        const uint64_t key = ((uint64_t)(el ? ~fl_order_key(wv) : 0xFFFFFFFFu) << 32) | (uint32_t)l16;
+        int place = 0;
+#define GR_ROT(n)                                                                                  \
+    {                                                                                              \
+        const uint32_t lo = (uint32_t)fl_dpp<0x120 + n>((int)(uint32_t)key);                        \
+        const uint32_t hi = (uint32_t)fl_dpp<0x120 + n>((int)(uint32_t)(key >> 32));                \
+        place += ((((uint64_t)hi << 32) | lo) < key) ? 1 : 0;                                      \
+    }
+        GR_ROT(1) GR_ROT(2) GR_ROT(3) GR_ROT(4) GR_ROT(5) GR_ROT(6) GR_ROT(7) GR_ROT(8)
+        GR_ROT(9) GR_ROT(10) GR_ROT(11) GR_ROT(12) GR_ROT(13) GR_ROT(14) GR_ROT(15)
+#undef GR_ROT
+        const int to = (row0 | place) << 2;  // every lane of a row to another one of it
+        op = __builtin_amdgcn_ds_permute(to, op);
+        start = __builtin_amdgcn_ds_permute(to, start);
+        cnt = __builtin_amdgcn_ds_permute(to, el ? cnt : 0);
+        wv = __int_as_float(__builtin_amdgcn_ds_permute(to, __float_as_int(wv)));
+        // edges before the group's in the row (at most the side's edges)
+        int incl = cnt;
+        incl += fl_dpp<0x111>(incl);
+        incl += fl_dpp<0x112>(incl);
+        incl += fl_dpp<0x114>(incl);
+        incl += fl_dpp<0x118>(incl);
+        const int take = max(min(tk - (incl - cnt), cnt), 0);
+        const double mass = take > 0 ? __dmul_rn(gr_proposal(wv, temp), (double)take) : 0.0;
+        const uint64_t taken = __ballot(take > 0) >> (lane & 32);
+        const int nf = __popcll(taken & 0xFFFFull), ni = __popcll(taken & 0xFFFF0000ull);
+        const int at = side ? nf + l16 : l16;  // the option's place in the node's list
+        fl_wave_sync();
+        if (take > 0) mass_lds[at] = mass;
+        fl_wave_sync();
+        double acc = 0.0, total = 0.0;
+        const int n = nf + ni;
+        for (int i = 0; __ballot(i < n) != 0; ++i) {
+            const double m = mass_lds[i & 31];
+            if (i < n) total = __dadd_rn(total, m);
+            if (i == at) acc = total;
+        }
+        if (!live) continue;
+        const int64_t ob = combo * hp.nopt + hp.hub_off[hid];
+        if (take > 0) {
+            hp.opt[ob + at] = make_int4(op, start, take, 0);
+            hp.cum[ob + at] = acc;
+        }
+        if ((lane & 31) == 0) {
+            const float wid = w[2 * R];
+            if (wid > 0.0f) total = __dadd_rn(total, gr_proposal(wid, temp));
+            GrHubHdr hd;
+            hd.off = (uint32_t)hp.hub_off[hid];
+            hd.n = (uint32_t)n | (wid > 0.0f ? GR_HDR_ID : 0u);
+            hd.total = total;
+            hp.hdr[combo * hp.nhub + hid] = hd;
+        }
+    }
+}
+
+// Hub cache fill of the other hubs, wave per (combination, hub)
+// (grid-stride): the hub's options ranked and their masses accumulated
+// exactly as a walk step does (no excluded operator), written to the pool;
+// the sort scratch of large sides is the block's walk scratch.
 __global__ __launch_bounds__(GR_NT) void k_gr_hubs(GrGraph gg, GrHubPool hp, const float *__restrict__ att,
                                                   int64_t ranks, int64_t vocab, int64_t ncombo, int64_t topk,
                                                   double temp, int64_t pmax, int64_t ocap, char *__restrict__ scratch,
@@ -480,8 +596,9 @@ __global__ __launch_bounds__(GR_NT) void k_gr_hubs(GrGraph gg, GrHubPool hp, con
     const int lane = fl_lane();
     char *ws = scratch + (size_t)blockIdx.x * stride;
     const int32_t R = gg.R;
-    for (int64_t u = blockIdx.x; u < ncombo * hp.nhub; u += gridDim.x) {
-        const int64_t combo = u / hp.nhub, hid = u - combo * hp.nhub;
+    const int64_t nlarge = hp.nlist[1];
+    for (int64_t u = blockIdx.x; u < ncombo * nlarge; u += gridDim.x) {
+        const int64_t combo = u / nlarge, hid = hp.list[hp.nhub - 1 - (u - combo * nlarge)];
         const int32_t node = hp.hub_node[hid];
         const int64_t hslot = combo / (3 * ranks), step = (combo / ranks) % 3, rank = combo % ranks;
         const float *w = att + hslot * 3 * ranks * vocab + (step * ranks + rank) * vocab;
@@ -489,9 +606,7 @@ __global__ __launch_bounds__(GR_NT) void k_gr_hubs(GrGraph gg, GrHubPool hp, con
         GrScratch sc;
         sc.skey = (uint64_t *)ws;
         sc.sgrp = (int32_t *)(sc.skey + pmax);
-        sc.oop = hp.op + ob;
-        sc.ostart = hp.start + ob;
-        sc.otake = hp.take + ob;
+        sc.oopt = hp.opt + ob;
         sc.omass = hp.cum + ob;
         (void)ocap;
         const int64_t fg0 = gg.fw.ptr[node], fG = gg.fw.ptr[node + 1] - fg0;
@@ -500,9 +615,7 @@ __global__ __launch_bounds__(GR_NT) void k_gr_hubs(GrGraph gg, GrHubPool hp, con
         if (fG <= FL_WAVE) {
             fo = gr_side_reg(gg.fw, 0, fg0, (int)fG, w, -1, topk, temp);
             if (lane < fo.n) {
-                sc.oop[lane] = fo.op;
-                sc.ostart[lane] = fo.start;
-                sc.otake[lane] = fo.take;
+                sc.oopt[lane] = make_int4(fo.op, fo.start, fo.take, 0);
                 sc.omass[lane] = fo.mass;
             }
             fo.mem = 1;
@@ -514,9 +627,7 @@ __global__ __launch_bounds__(GR_NT) void k_gr_hubs(GrGraph gg, GrHubPool hp, con
         if (iG <= FL_WAVE) {
             io = gr_side_reg(gg.inv, R, ig0, (int)iG, w, -1, topk, temp);
             if (lane < io.n) {
-                sc.oop[ibase + lane] = io.op;
-                sc.ostart[ibase + lane] = io.start;
-                sc.otake[ibase + lane] = io.take;
+                sc.oopt[ibase + lane] = make_int4(io.op, io.start, io.take, 0);
                 sc.omass[ibase + lane] = io.mass;
             }
             io.mem = 1;
@@ -531,10 +642,9 @@ __global__ __launch_bounds__(GR_NT) void k_gr_hubs(GrGraph gg, GrHubPool hp, con
         if (wid > 0.0f) total = __dadd_rn(total, gr_proposal(wid, temp));
         if (lane == 0) {
             GrHubHdr hd;
-            hd.nf = fo.n;
-            hd.ni = io.n;
+            hd.off = (uint32_t)hp.hub_off[hid];
+            hd.n = (uint32_t)(fo.n + io.n) | (wid > 0.0f ? GR_HDR_ID : 0u);
             hd.total = total;
-            hd.off = ob;
             hp.hdr[combo * hp.nhub + hid] = hd;
         }
         __syncthreads();  // scratch reused by the next hub
@@ -561,11 +671,9 @@ __global__ __launch_bounds__(GR_NT) void k_gr_walk(GrGraph gg, const float *__re
     char *ws = scratch + (size_t)blockIdx.x * stride;
     GrScratch sc;
     sc.skey = (uint64_t *)ws;
-    sc.omass = (double *)(sc.skey + pmax);
+    sc.oopt = (int4 *)(sc.skey + pmax);  // pmax is even: 16-byte aligned
+    sc.omass = (double *)(sc.oopt + ocap);
     sc.sgrp = (int32_t *)(sc.omass + ocap);
-    sc.oop = sc.sgrp + pmax;
-    sc.ostart = sc.oop + ocap;
-    sc.otake = sc.ostart + ocap;
     if (LS) {  // the large-side sort runs in LDS (the option lists stay in the scratch)
         sc.skey = (uint64_t *)gr_lds;
         sc.sgrp = (int32_t *)(sc.skey + pmax);
@@ -614,16 +722,14 @@ __global__ __launch_bounds__(GR_NT) void k_gr_walk(GrGraph gg, const float *__re
                     // a hub: the options this (head, step, rank) gives it, ranked once per call
                     const int64_t combo = ((int64_t)hslot * 3 + step) * ranks + rank;
                     const GrHubHdr hd = hp.hdr[combo * hp.nhub + hid];
-                    const int64_t ob = hd.off;
-                    scs.oop = hp.op + ob;
-                    scs.ostart = hp.start + ob;
-                    scs.otake = hp.take + ob;
+                    const int64_t ob = combo * hp.nopt + hd.off;
+                    scs.oopt = hp.opt + ob;
                     scs.omass = hp.cum + ob;
-                    fo.n = hd.nf;
+                    fo.n = (int)(hd.n & ~GR_HDR_ID);  // both sides' options, one list
                     fo.mem = 1;
-                    io.n = hd.ni;
+                    io.n = 0;
                     io.mem = 1;
-                    ibase = hd.nf;
+                    ibase = fo.n;
                     total = hd.total;
                 } else {
                     const int64_t fg0 = gg.fw.ptr[node], fG = gg.fw.ptr[node + 1] - fg0;
@@ -693,6 +799,226 @@ __global__ __launch_bounds__(GR_NT) void k_gr_walk(GrGraph gg, const float *__re
 }
 
 // ---------------------------------------------------------------------------
+// Walks side by side.  With every node's lists in the pool a step needs no
+// cooperation of the lanes, but the walks of a source share one engine, so
+// where a walk's words start depends on how many the walks before it used:
+// 6 for three edges, one less for every identity step (a draw without an
+// edge pick), more only where Lemire's method rejects a word.  The lanes of
+// a wave therefore walk GL_I consecutive walks, each from GL_W assumed
+// deficits d (words saved against 6 per walk so far), a band around the mean
+// deficit of the task's recent walks; the chain of walks whose assumption is
+// the sum of what came before is then followed from walk 0, whose start is
+// known, and those walks are the reference's, word for word.  The others are
+// dropped; the next round starts behind the last walk kept.
+//   Bound by the latency of its dependent gathers (per step: header, about
+// log2(options) cumulative masses, option, target column), which a round
+// pays once for all the walks that it keeps instead of once per walk.
+constexpr int GL_W = 4;                    // deficits per walk
+constexpr int GL_I = FL_WAVE / GL_W;       // walks per round
+constexpr int GL_LOOK = 6 * GL_I + 32;     // words ahead of the round's start that are generated
+constexpr int GL_FILTER = 8192;            // bits of the positive-target filter
+constexpr int64_t GR_LANES_GRID = 1 << 20;
+static_assert(GL_LOOK < MT_N, "a round's words lie in two blocks of the engine");
+
+// The engine's next block of 312 words: from src (one block) to dst, in two
+// phases (the second reads the first's).
+__device__ __forceinline__ void gl_twist(const uint64_t *src, uint64_t *dst) {
+    const int lane = fl_lane();
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int i = lane + FL_WAVE * k;
+        if (i < MT_M) dst[i] = mt_mix(src[i], src[i + 1], src[i + MT_M]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const int i = MT_M + lane + FL_WAVE * k;
+        if (i < MT_N) dst[i] = mt_mix(src[i], i + 1 < MT_N ? src[i + 1] : dst[0], dst[i - MT_M]);
+    }
+    __syncthreads();
+}
+
+__device__ __forceinline__ uint64_t mt_temper(uint64_t z) {
+    z ^= (z >> 29) & 0x5555555555555555ull;
+    z ^= (z << 17) & 0x71D67FFFEDA60000ull;
+    z ^= (z << 37) & 0xFFF7EEE000000000ull;
+    z ^= z >> 43;
+    return z;
+}
+
+__global__ __launch_bounds__(GR_NT) void k_gr_lanes(GrGraph gg, int64_t ranks, const int64_t *__restrict__ heads,
+                                                   const int64_t *__restrict__ seeds, int64_t ntasks,
+                                                   const int32_t *__restrict__ task_head,
+                                                   const int64_t *__restrict__ task_source,
+                                                   const int64_t *__restrict__ task_index, int64_t walks,
+                                                   GrHubPool hp, uint64_t *__restrict__ out_key,
+                                                   uint8_t *__restrict__ out_pos) {
+    __shared__ uint64_t ring[2 * MT_N];  // the engine's two newest blocks
+    __shared__ uint32_t filter[GL_FILTER / 32];
+    const int lane = fl_lane();
+    const int li = lane / GL_W, lk = lane % GL_W;
+    const int32_t R = gg.R;
+    for (int64_t tb = blockIdx.x; tb < ntasks; tb += gridDim.x) {
+        // (a grid of all tasks: neighbouring tasks, of one head, on one XCD)
+        const int64_t t = gridDim.x >= ntasks ? fl_xcd_contig(tb, ntasks) : tb;
+        const int32_t hslot = task_head[t];
+        const int32_t head = (int32_t)heads[hslot];
+        const int32_t source = (int32_t)task_source[t];
+        __syncthreads();  // the previous task is done with the LDS arrays
+        mt_seed(ring + MT_N, fl_splitmix64((uint64_t)seeds[hslot] ^ ((uint64_t)task_index[t] << 32) ^
+                                           (uint64_t)(uint32_t)source));
+        gl_twist(ring + MT_N, ring);
+        int newest = 0;    // half that holds the newest block
+        int base = 0;      // ring index of the round's first word
+        int left = MT_N;   // generated words from there on
+        // positive targets: the (source, head) group of the head's side
+        const GrSide &hs = head >= R ? gg.inv : gg.fw;
+        const int32_t hrel = head >= R ? head - R : head;
+        int32_t plo = hs.ptr[source], phi = hs.ptr[source + 1];
+        const int32_t pend = phi;
+        while (plo < phi) {
+            const int32_t mid = plo + (phi - plo) / 2;
+            if ((int32_t)hs.rel[mid] < hrel) plo = mid + 1;
+            else phi = mid;
+        }
+        int32_t pstart = 0, pcount = 0;
+        if (plo < pend && (int32_t)hs.rel[plo] == hrel) {
+            pstart = hs.start[plo];
+            pcount = hs.count[plo];
+        }
+        pstart = __builtin_amdgcn_readfirstlane(pstart);
+        pcount = __builtin_amdgcn_readfirstlane(pcount);
+        const int32_t preg = lane < pcount ? hs.col[pstart + lane] : -1;
+        if (pcount > FL_WAVE) {
+            // more targets than lanes: a hashed bitmap of them rules most nodes out
+            for (int q = lane; q < GL_FILTER / 32; q += FL_WAVE) filter[q] = 0;
+            __syncthreads();
+            for (int32_t q = lane; q < pcount; q += FL_WAVE) {
+                const uint32_t x = (uint32_t)hs.col[pstart + q] % GL_FILTER;
+                atomicOr(&filter[x >> 5], 1u << (x & 31));
+            }
+            __syncthreads();
+        }
+        int m8 = 64;  // mean deficit per walk, in 1/256 of a word
+        for (int64_t j = 0; j < walks;) {
+            if (left < GL_LOOK) {
+                // the round's start lies in the newest block (left < 312): the other one is free
+                gl_twist(ring + newest * MT_N, ring + (newest ^ 1) * MT_N);
+                newest ^= 1;
+                left += MT_N;
+            }
+            const int d = max(((m8 * li + 128) >> 8) - 1, 0) + lk;
+            const int off = 6 * li - d;
+            int used = -1;  // words; -1: no such walk, or its words ran past those generated
+            uint64_t key = 0;
+            int32_t node = source;
+            if (off >= 0 && j + li < walks) {
+                const int64_t rank = (j + li) % ranks;
+                int p = off, len = 0;
+                uint64_t body = 0;
+                bool viable = true, fit = true;
+                auto word = [&]() {
+                    int q = base + p;
+                    if (q >= 2 * MT_N) q -= 2 * MT_N;
+                    ++p;
+                    return mt_temper(ring[q]);
+                };
+                for (int step = 0; step < 3; ++step) {
+                    const int64_t combo = ((int64_t)hslot * 3 + step) * ranks + rank;
+                    const GrHubHdr hd = hp.hdr[combo * hp.nhub + node];
+                    const int64_t ob = combo * hp.nopt + hd.off;
+                    if (!(hd.total > 0.0)) {
+                        viable = false;
+                        break;
+                    }
+                    if (p + 2 > left) { fit = false; break; }
+                    double u = __dmul_rn(__ull2double_rn(word()), 0x1.0p-64);
+                    u = u >= 1.0 ? 0x1.fffffffffffffp-1 : u;
+                    const double draw = __dmul_rn(u, hd.total);
+                    // first option (forward, then inverse) with draw < its
+                    // cumulative mass, which does not decrease
+                    const int n = (int)(hd.n & ~GR_HDR_ID);
+                    const double *cum = hp.cum + ob;
+                    int lo = 0, hi = n;
+                    while (lo < hi) {
+                        const int mid = (lo + hi) >> 1;
+                        if (draw < cum[mid]) hi = mid;
+                        else lo = mid + 1;
+                    }
+                    if (lo == n) {
+                        if (hd.n & GR_HDR_ID) continue;  // the identity
+                        lo = n - 1;                // none below the draw: the last option
+                    }
+                    const int4 o = hp.opt[ob + lo];
+                    const uint64_t range = (uint64_t)o.z;
+                    uint64_t x = word();
+                    uint64_t pick = __umul64hi(x, range), low = x * range;
+                    if (low < range) {
+                        const uint64_t threshold = (0ull - range) % range;
+                        while (low < threshold && p < left) {
+                            x = word();
+                            pick = __umul64hi(x, range);
+                            low = x * range;
+                        }
+                        if (low < threshold) { fit = false; break; }
+                    }
+                    node = (o.x >= R ? gg.inv.col : gg.fw.col)[o.y + (int64_t)pick];
+                    body |= ((uint64_t)o.x & ((1ull << 20) - 1)) << (40 - 20 * len);
+                    ++len;
+                }
+                if (fit) used = p - off;
+                if (viable && len > 0) key = ((uint64_t)len << 60) | body;
+            }
+            // the chain of walks that start where the one before them ended.
+            // (Walk 0 has GL_LOOK - 6 words to spare for rejections, each of
+            // probability below 2^-32: it never runs out.)
+            const int dn = d + 6 - used;
+            uint64_t kept = 0;
+            int cur = 0, i = 0, dend = 0;
+            for (;;) {
+                if (__builtin_amdgcn_readlane(used, cur) < 0) break;
+                kept |= 1ull << cur;
+                dend = __builtin_amdgcn_readlane(dn, cur);
+                ++i;
+                const int k = dend - max(((m8 * i + 128) >> 8) - 1, 0);
+                if (i == GL_I || k < 0 || k >= GL_W) break;
+                cur = i * GL_W + k;
+            }
+            if (i == 0) { kept = 1; i = 1; dend = 0; }  // (out of words, see above: the loop goes on)
+            const bool mine = (kept >> lane) & 1ull;
+            bool pos = false;
+            if (pcount <= FL_WAVE) {
+                for (int q = 0; q < pcount; ++q) pos |= node == __builtin_amdgcn_readlane(preg, q);
+                pos = pos && key != 0;
+            } else {
+                const uint32_t x = (uint32_t)node % GL_FILTER;
+                uint64_t maybe = __ballot(mine && key != 0 && ((filter[x >> 5] >> (x & 31)) & 1u));
+                while (maybe) {
+                    const int l = __ffsll((long long)maybe) - 1;
+                    maybe &= maybe - 1;
+                    const int32_t e = __builtin_amdgcn_readlane(node, l);
+                    bool hit = false;
+                    for (int32_t q = 0; q < pcount && !hit; q += FL_WAVE)
+                        hit = __ballot(q + lane < pcount && hs.col[pstart + q + lane] == e) != 0;
+                    if (lane == l) pos = hit;
+                }
+            }
+            if (mine) {
+                out_key[t * walks + j + li] = key;
+                out_pos[t * walks + j + li] = pos ? 1 : 0;
+            }
+            const int advance = 6 * i - dend;
+            j += i;
+            base += advance;
+            if (base >= 2 * MT_N) base -= 2 * MT_N;
+            left -= advance;
+            m8 = (3 * m8 + max(256 * dend / i, 0)) >> 2;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // Counting (soft_grounding.cpp:427-614).  Records of (head, fold) segment s
 // are [seg_off[s], seg_off[s+1]) x walks; after the stable sort by key the
 // runs of equal nonzero keys are the fold's bodies.
@@ -729,7 +1055,10 @@ __global__ void k_ct_flags(const uint64_t *__restrict__ key, const uint32_t *__r
 }
 
 // per run: key, segment, walk hits, positive walk hits, source hits; per
-// source run: any positive
+// source run: any positive.  The records are sorted, so a run's records in a
+// wave are neighbours: its first one there adds the wave's counts (an atomic
+// per run, wave and counter instead of one per record: 22.3M records 2.6 ms
+// before).
 __global__ void k_ct_accum(const uint64_t *__restrict__ key, const uint32_t *__restrict__ rec,
                            const uint8_t *__restrict__ pos, int64_t n, const int64_t *__restrict__ rec_off,
                            int64_t nseg, const int32_t *__restrict__ run_head, const int64_t *__restrict__ run_id,
@@ -737,24 +1066,43 @@ __global__ void k_ct_accum(const uint64_t *__restrict__ key, const uint32_t *__r
                            uint64_t *__restrict__ rkey, int32_t *__restrict__ rseg,
                            unsigned long long *__restrict__ rcnt, int32_t *__restrict__ src_run,
                            int32_t *__restrict__ src_pos) {
+    const int lane = fl_lane();
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n || key[i] == 0) return;
-    const int64_t r = run_id[i] + run_head[i] - 1;  // inclusive
-    const int64_t q = src_id[i] + src_head[i] - 1;
-    const int p = pos[rec[i]];
-    if (run_head[i]) {
-        rkey[r] = key[i];
-        rseg[r] = (int32_t)ct_segment(rec_off, nseg, i);
+    const bool live = i < n && key[i] != 0;
+    int64_t r = -1, q = -1;
+    int rh = 0, sh = 0, p = 0;
+    if (live) {
+        rh = run_head[i];
+        sh = src_head[i];
+        r = run_id[i] + rh - 1;  // inclusive
+        q = src_id[i] + sh - 1;
+        p = pos[rec[i]];
+        if (rh) {
+            rkey[r] = key[i];
+            rseg[r] = (int32_t)ct_segment(rec_off, nseg, i);
+        }
+        if (sh) src_run[q] = (int32_t)r;
     }
-    if (src_head[i]) {
-        src_run[q] = (int32_t)r;
-        atomicAdd(&rcnt[4 * r + 1], 1ull);
+    const uint64_t lives = __ballot(live), pm = __ballot(p != 0), sm = __ballot(sh != 0);
+    // lanes that open a run (a source run) in this wave: their own flag, or
+    // the wave's first lane, or a record without a run before them
+    const uint64_t before = lives << 1;
+    const bool ropen = live && (rh || !((before >> lane) & 1ull));
+    const bool sopen = live && (sh || !((before >> lane) & 1ull));
+    const uint64_t ro = __ballot(ropen), so = __ballot(sopen), gaps = ~lives;
+    const uint64_t above = lane == FL_WAVE - 1 ? 0ull : ~0ull << (lane + 1);
+    auto span = [&](uint64_t opens) {  // this lane up to the next opening or gap
+        const uint64_t stop = (opens | gaps) & above;
+        const uint64_t up = stop ? (1ull << (__ffsll((long long)stop) - 1)) - 1 : ~0ull;
+        return up & ~((1ull << lane) - 1);
+    };
+    if (ropen) {
+        const uint64_t m = span(ro);
+        atomicAdd(&rcnt[4 * r + 0], (unsigned long long)__popcll(m));
+        if (m & sm) atomicAdd(&rcnt[4 * r + 1], (unsigned long long)__popcll(m & sm));
+        if (m & pm) atomicAdd(&rcnt[4 * r + 2], (unsigned long long)__popcll(m & pm));
     }
-    atomicAdd(&rcnt[4 * r + 0], 1ull);
-    if (p) {
-        atomicAdd(&rcnt[4 * r + 2], 1ull);
-        atomicMax(&src_pos[q], 1);
-    }
+    if (sopen && (span(so) & pm)) atomicMax(&src_pos[q], 1);
 }
 
 __global__ void k_ct_srcpos(const int32_t *__restrict__ src_run, const int32_t *__restrict__ src_pos, int64_t nsrc,
@@ -1048,9 +1396,9 @@ GrGraph gr_graph(const fl_ground_graph *g) {
 }
 
 struct GrWalkLayout {
-    int64_t pmax, ocap, waves, ncombo;
+    int64_t pmax, ocap, waves, hub_waves, ncombo;
     size_t stride, bytes;
-    size_t hub_hdr, hub_cum, hub_op, hub_start, hub_take;  // byte offsets of the hub cache (ncombo > 0)
+    size_t hub_hdr, hub_cum, hub_opt, hub_list;  // byte offsets of the hub cache (ncombo > 0)
 };
 
 GrWalkLayout gr_walk_layout(const fl_ground_graph *g, int64_t ntasks, int64_t nheads, int64_t ranks) {
@@ -1060,21 +1408,26 @@ GrWalkLayout gr_walk_layout(const fl_ground_graph *g, int64_t ntasks, int64_t nh
     L.ocap = 2 * (g->max_groups > 1 ? g->max_groups : 1);
     L.waves = ntasks < 8192 ? ntasks : 8192;
     L.stride = gal(sizeof(uint64_t) * (size_t)L.pmax + sizeof(double) * (size_t)L.ocap +
-                   sizeof(int32_t) * (size_t)L.pmax + 3 * sizeof(int32_t) * (size_t)L.ocap);
-    L.bytes = L.stride * (size_t)(L.waves > 0 ? L.waves : 1);
+                   sizeof(int32_t) * (size_t)L.pmax + sizeof(int4) * (size_t)L.ocap);
+    L.hub_waves = 0;
     if (g->nhub > 0 && g->hub_options > 0 && nheads > 0 && ranks > 0) {
+        // the lists are ranked by as many waves as the chip holds, whatever
+        // the number of tasks
         L.ncombo = nheads * 3 * ranks;
+        L.hub_waves = L.ncombo * g->nhub < 8192 ? L.ncombo * g->nhub : 8192;
+    }
+    const int64_t strides = L.waves > L.hub_waves ? L.waves : L.hub_waves;
+    L.bytes = L.stride * (size_t)(strides > 0 ? strides : 1);
+    if (L.ncombo > 0) {
         const size_t slots = (size_t)L.ncombo * (size_t)g->hub_options;
         L.hub_hdr = L.bytes;
         L.bytes += gal(sizeof(GrHubHdr) * (size_t)L.ncombo * (size_t)g->nhub);
         L.hub_cum = L.bytes;
         L.bytes += gal(sizeof(double) * slots);
-        L.hub_op = L.bytes;
-        L.bytes += gal(sizeof(int32_t) * slots);
-        L.hub_start = L.bytes;
-        L.bytes += gal(sizeof(int32_t) * slots);
-        L.hub_take = L.bytes;
-        L.bytes += gal(sizeof(int32_t) * slots);
+        L.hub_list = L.bytes;
+        L.bytes += gal(sizeof(int32_t) * ((size_t)g->nhub + 2));
+        L.hub_opt = L.bytes;
+        L.bytes += gal(sizeof(int4) * slots);
     }
     return L;
 }
@@ -1190,6 +1543,8 @@ int fl_ground_walks(void *stream, const fl_ground_graph *g, const float *att, in
     if (ntasks == 0) return FL_OK;
     if (!att || !heads || !seeds || !task_head || !task_source || !task_index || !keys || !positive || !ws)
         return fl_fail(FL_ERR_ARG, "ground_walks: null argument");
+    if (g->hub_options >= ((int64_t)1 << 32))
+        return fl_fail(FL_ERR_ARG, "ground_walks: more than 2^32 option slots");
     if (g->nhub > 0 && (!g->hub_id || !g->hub_node || !g->hub_off))
         return fl_fail(FL_ERR_ARG, "ground_walks: hub cache without its arrays");
     const GrWalkLayout L = gr_walk_layout(g, ntasks, nheads, ranks);
@@ -1199,18 +1554,30 @@ int fl_ground_walks(void *stream, const fl_ground_graph *g, const float *att, in
     if (L.ncombo > 0) {
         hp.hdr = (GrHubHdr *)(wsb + L.hub_hdr);
         hp.cum = (double *)(wsb + L.hub_cum);
-        hp.op = (int32_t *)(wsb + L.hub_op);
-        hp.start = (int32_t *)(wsb + L.hub_start);
-        hp.take = (int32_t *)(wsb + L.hub_take);
+        hp.opt = (int4 *)(wsb + L.hub_opt);
         hp.hub_id = g->hub_id;
         hp.hub_node = g->hub_node;
         hp.hub_off = g->hub_off;
         hp.nhub = g->nhub;
         hp.nopt = g->hub_options;
-        const int64_t units = L.ncombo * g->nhub;
-        FL_LAUNCH("k_gr_hubs", k_gr_hubs, dim3((unsigned)(units < L.waves ? units : L.waves)), dim3(GR_NT), 0,
-                  (hipStream_t)stream, gr_graph(g), hp, att, ranks, 2 * g->num_relations + 1, L.ncombo, topk_edges,
-                  temperature, L.pmax, L.ocap, wsb, L.stride);
+        hp.nlist = (int32_t *)(wsb + L.hub_list);
+        hp.list = hp.nlist + 2;
+        hipStream_t st = (hipStream_t)stream;
+        const GrGraph gg = gr_graph(g);
+        FL_LAUNCH("k_i32_fill", k_i32_fill, dim3(1), dim3(64), 0, st, hp.nlist, (int64_t)2, 0);
+        FL_LAUNCH("k_gr_kinds", k_gr_kinds, dim3((unsigned)((g->nhub + 255) / 256)), dim3(256), 0, st, gg, hp);
+        const int64_t small_g = (L.ncombo * g->nhub + 7) / 8;
+        FL_LAUNCH("k_gr_small", k_gr_small, dim3((unsigned)(small_g < 8192 ? small_g : 8192)), dim3(256), 0, st, gg, hp,
+                  att, ranks, 2 * g->num_relations + 1, L.ncombo, topk_edges, temperature);
+        FL_LAUNCH("k_gr_hubs", k_gr_hubs, dim3((unsigned)L.hub_waves), dim3(GR_NT), 0, (hipStream_t)stream,
+                  gr_graph(g), hp, att, ranks, 2 * g->num_relations + 1, L.ncombo, topk_edges, temperature, L.pmax,
+                  L.ocap, wsb, L.stride);
+        if (g->nhub == g->nodes && !mask_query_head) {
+            // every node's lists are there: walks of a source side by side
+            FL_LAUNCH("k_gr_lanes", k_gr_lanes, dim3((unsigned)(ntasks < GR_LANES_GRID ? ntasks : GR_LANES_GRID)),
+                      dim3(GR_NT), 0, st, gg, ranks, heads, seeds, ntasks, task_head, task_source, task_index, walks, hp, keys, positive);
+            return fl_check_launch("ground_walks");
+        }
     }
     // sides of up to GR_LDS_SORT_MAX groups are sorted in LDS, larger ones in the scratch
     const int lds_sort = L.pmax <= GR_LDS_SORT_MAX ? 1 : 0;

@@ -17,8 +17,13 @@ from ... import _lib
 from ..._lib import FlGroundGraph, check, ptr
 
 RULE_STEPS = 3  # the reference's default build (FLASHLOG_RULE_STEPS)
-HUB_MIN_GROUPS = 8  # sides with more groups make a node a hub of the walk's option cache
-HUB_CACHE_MAX_BYTES = 2 << 30  # the cache is skipped above this size
+HUB_MIN_GROUPS = 8  # sides with more groups make a node a hub where not every node is in the walk's option cache
+HUB_CACHE_MAX_BYTES = 2 << 30  # the cache's largest size
+# Lists of every node are ranked where that takes less time than they save: 0.8 ns a list (C3, 2.1M lists in
+# 1.8 ms), against 28 us a walk of a source that ranks as it goes and 2 us with the lists (the sources of about
+# 5000 tasks walk at a time).
+LISTS_PER_WALK = 32000
+TASKS_AT_ONCE = 5000
 
 
 def _device():
@@ -54,24 +59,38 @@ def _graph(csr, dev, num_relations):
     g.num_relations = int(num_relations)
     widths = [int((p[1:] - p[:-1]).max()) if p.numel() > 1 else 0 for p in (t[8], t[12])]
     g.max_groups = max(widths + [1])
-    # hub cache: nodes with more than 64 groups on a side (their options are
-    # ranked once per call for every head, step and rank)
+    g.arrays = t  # alive as long as the struct that points at them
+    _set_hubs(g, 0)
+    return g, t
+
+
+def _set_hubs(g, min_groups):
+    """Gives the graph's option cache the nodes with more than min_groups
+    groups on a side (0: every node; hub i is then node i)."""
+    t = g.arrays
+    dev = t[8].device
     fw = (t[8][1:] - t[8][:-1]).long()
     iv = (t[12][1:] - t[12][:-1]).long()
-    hub = (fw > HUB_MIN_GROUPS) | (iv > HUB_MIN_GROUPS)
-    hub_node = torch.nonzero(hub).view(-1)
+    if min_groups:
+        hub_node = torch.nonzero((fw > min_groups) | (iv > min_groups)).view(-1)
+    else:
+        hub_node = torch.arange(g.nodes, device=dev)
     nhub = hub_node.numel()
     g.nhub, g.hub_options = 0, 0
-    if nhub:
-        hub_id = torch.full((g.nodes,), -1, dtype=torch.int32, device=dev)
-        hub_id[hub_node] = torch.arange(nhub, dtype=torch.int32, device=dev)
-        cap = (fw + iv)[hub_node]
-        hub_off = torch.zeros(nhub + 1, dtype=torch.int64, device=dev)
-        hub_off[1:] = torch.cumsum(cap, 0)
-        t["hub_id"], t["hub_node"], t["hub_off"] = hub_id, hub_node.to(torch.int32).contiguous(), hub_off
-        g.nhub, g.hub_options = nhub, int(hub_off[-1])
-        g.hub_id, g.hub_node, g.hub_off = ptr(hub_id).value, ptr(t["hub_node"]).value, ptr(hub_off).value
-    return g, t
+    if not nhub:
+        return
+    hub_id = torch.full((g.nodes,), -1, dtype=torch.int32, device=dev)
+    hub_id[hub_node] = torch.arange(nhub, dtype=torch.int32, device=dev)
+    hub_off = torch.zeros(nhub + 1, dtype=torch.int64, device=dev)
+    hub_off[1:] = torch.cumsum((fw + iv)[hub_node], 0)
+    t["hub_id"], t["hub_node"], t["hub_off"] = hub_id, hub_node.to(torch.int32).contiguous(), hub_off
+    g.nhub, g.hub_options = nhub, int(hub_off[-1])
+    g.hub_id, g.hub_node, g.hub_off = ptr(hub_id).value, ptr(t["hub_node"]).value, ptr(hub_off).value
+
+
+def _cache_bytes(g, ranks):
+    """The option cache of one head."""
+    return 3 * ranks * (24 * g.hub_options + 16 * g.nhub)
 
 
 def _walks(g, attentions, heads_d, seeds, task_head, task_source, task_index, walks, topk_edges, mask, temperature,
@@ -87,14 +106,28 @@ def _walks(g, attentions, heads_d, seeds, task_head, task_source, task_index, wa
     keys = torch.empty(max(ntasks * walks, 1), dtype=torch.int64, device=dev)
     positive = torch.empty(max(ntasks * walks, 1), dtype=torch.uint8, device=dev)
     nheads, ranks = attentions.shape[0], attentions.shape[2]
-    if g.nhub and 3 * nheads * ranks * (20 * g.hub_options + 16 * g.nhub) > HUB_CACHE_MAX_BYTES:
-        g.nhub = 0  # too large a cache: every step ranks its options
-    ws = torch.empty(max(lib.fl_ground_walk_bytes(ctypes.byref(g), ntasks, nheads, ranks), 1), dtype=torch.uint8,
-                     device=dev)
-    check(lib.fl_ground_walks(_stream(dev), ctypes.byref(g), ptr(att), att.shape[0], att.shape[2], ptr(heads_d),
-                              ptr(seeds_d), ntasks, ptr(th), ptr(ts), ptr(ti), walks, int(topk_edges),
-                              1 if mask else 0, temperature, ptr(ws), ws.numel(), ptr(keys), ptr(positive)),
-          "ground_walks")
+    few = 3 * nheads * ranks * g.nodes > LISTS_PER_WALK * walks * max(ntasks // TASKS_AT_ONCE, 1)
+    if g.nhub and (few or _cache_bytes(g, ranks) > HUB_CACHE_MAX_BYTES):
+        # few walks on a large graph, or not even one head's lists of every node fit: the lists of the large nodes,
+        # of all heads at once
+        _set_hubs(g, HUB_MIN_GROUPS)
+        if nheads * _cache_bytes(g, ranks) > HUB_CACHE_MAX_BYTES:
+            g.nhub = 0  # too large a cache: every step ranks its options
+        per_call = nheads
+    else:
+        per_call = max(HUB_CACHE_MAX_BYTES // max(_cache_bytes(g, ranks), 1), 1)
+    # (tasks are in head order)
+    bounds = torch.searchsorted(task_head.cpu().contiguous(), torch.arange(nheads + 1, dtype=task_head.dtype)).tolist()
+    chunks = [(h, min(h + per_call, nheads)) for h in range(0, nheads, per_call)]
+    sizes = [lib.fl_ground_walk_bytes(ctypes.byref(g), bounds[h1] - bounds[h0], h1 - h0, ranks) for h0, h1 in chunks]
+    ws = torch.empty(max(sizes + [1]), dtype=torch.uint8, device=dev)
+    for h0, h1 in chunks:
+        t0, t1 = bounds[h0], bounds[h1]
+        head_slots = th[t0:t1] - h0 if h0 else th[t0:t1]
+        check(lib.fl_ground_walks(_stream(dev), ctypes.byref(g), ptr(att[h0:h1]), h1 - h0, att.shape[2],
+                                  ptr(heads_d[h0:h1]), ptr(seeds_d[h0:h1]), t1 - t0, ptr(head_slots), ptr(ts[t0:t1]),
+                                  ptr(ti[t0:t1]), walks, int(topk_edges), 1 if mask else 0, temperature, ptr(ws),
+                                  ws.numel(), ptr(keys[t0 * walks:]), ptr(positive[t0 * walks:])), "ground_walks")
     return keys, positive
 
 
@@ -193,7 +226,7 @@ def ground_head_batch_source_folds_sampled_capped_counts(
                               ptr(heads_d), ptr(folds_d), budgets_h, ptr(cws), cws.numel(), ptr(rows), cap,
                               ptr(info)), "ground_count")
     info_h = info.cpu()
-    rows_h = rows.cpu()
+    rows_h = rows[:int(info_h[-1])].cpu()  # the rows there are, not the room for them
     elapsed = time.perf_counter() - started
     del keep
     raw = info_h[:nseg].tolist()

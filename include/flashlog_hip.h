@@ -715,9 +715,11 @@ typedef struct fl_ground_graph {
     int64_t nodes;          /* entities (ptr arrays hold nodes + 1)       */
     int64_t num_relations;  /* R: operators 0..2R-1, identity 2R          */
     int64_t max_groups;     /* most groups of one node on one side        */
-    /* optional hub cache (nhub = 0 disables it): nodes with more than 64
-       groups on a side get their transition options precomputed once per
-       call for every (head, step, rank) instead of ranked at every visit */
+    /* optional hub cache (nhub = 0 disables it): the hubs get their
+       transition options precomputed once per call for every (head, step,
+       rank) instead of ranked at every visit.  With nhub = nodes (hub_id and
+       hub_node then the identity) and no excluded operator the walks of a
+       source also run side by side */
     int64_t nhub;           /* hub nodes                                  */
     int64_t hub_options;    /* hub_off[nhub]                              */
     const int32_t *hub_id;  /* [nodes] hub index of a node, -1 for others */
