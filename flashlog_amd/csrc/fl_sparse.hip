@@ -51,8 +51,27 @@
 
 namespace fl {
 
-constexpr int SP_S = 13;               // destinations per bucket = 2^SP_S
-constexpr int SP_W = 1 << SP_S;
+// Destination buckets.  A row's items are partitioned into buckets of 2^S
+// consecutive entities, S between SP_S_MIN and SP_S_MAX by the hop's size
+// (sp_shift): buckets of 64 entities have no more destinations than a wave
+// has lanes, so that no bucket needs a sort; wider ones keep the number of
+// buckets a row, and with it the partition, at two digits of the radix sort
+// (SP_NB_MAX), and a hop of few items from spreading them over empty buckets.
+//   Fixed 2^13 buckets before: of 41,000 entities every bucket held over a
+// thousand destinations and was sorted 2048 items at a time.
+constexpr int SP_S_MIN = 6, SP_S_MAX = 13;
+constexpr int SP_W = 1 << SP_S_MAX;     // the widest bucket
+constexpr int64_t SP_NB_MAX = 1022;     // buckets a row (with the holes' key: 10 bits)
+constexpr int64_t SP_SLOT_ITEMS = 16;   // items per (row, bucket) below which buckets are made wider
+
+__host__ __device__ inline int64_t sp_buckets_of(int64_t E, int S) { return E <= 0 ? 1 : (E + ((int64_t)1 << S) - 1) >> S; }
+
+__host__ __device__ inline int sp_shift(int64_t E, int64_t R, int64_t items) {
+    int s = SP_S_MIN;
+    while (s < SP_S_MAX && sp_buckets_of(E, s) > SP_NB_MAX) ++s;
+    while (s < SP_S_MAX && sp_buckets_of(E, s) > 1 && R * sp_buckets_of(E, s) * SP_SLOT_ITEMS > items) ++s;
+    return s;
+}
 constexpr int SP_NT = 256;
 constexpr int NM_NT0 = 256;  // row-reduction workgroup size
 constexpr int SP_IPT = 16;
@@ -756,6 +775,7 @@ struct SpRows {
     const int64_t *row_item0;  // [R+1]
     const int64_t *tile_base;  // [R+1]
     int64_t NB;                // buckets per row
+    int S;                     // a bucket's entities: 2^S
 };
 
 // Mask of position p on a side: its bit when the side has a bitmap (every
@@ -1145,11 +1165,11 @@ __global__ __launch_bounds__(SP_NT) void k_sp_hist(int64_t R, SpRows rows, const
         for (int j = 0; j < Q; ++j) dd[j] = fl_ld32(tdst, (uint32_t)(j * SP_NT) + threadIdx.x);
 #pragma unroll
         for (int j = 0; j < Q; ++j)
-            if (dd[j] >= 0) atomicAdd(&hb[dd[j] >> SP_S], 1);
+            if (dd[j] >= 0) atomicAdd(&hb[dd[j] >> rows.S], 1);
     } else {
         for (uint32_t idx = threadIdx.x; idx < (uint32_t)c; idx += SP_NT) {
             const int32_t d = fl_ld32(tdst, idx);
-            if (d >= 0) atomicAdd(&hb[d >> SP_S], 1);
+            if (d >= 0) atomicAdd(&hb[d >> rows.S], 1);
         }
     }
     __syncthreads();
@@ -1326,7 +1346,7 @@ __global__ __launch_bounds__(SP_PT_NT) void k_sp_partition(int64_t R, SpRows row
     for (int j = 0; j < SP_PT_IPT; ++j) {
         const int idx = j * SP_PT_NT + t;
         uint32_t key = 0xFFFFF000u | (uint32_t)idx;  // padding and holes sort last
-        if (idx < c && dk[j] >= 0) key = ((uint32_t)(dk[j] >> SP_S) << 12) | (uint32_t)idx;
+        if (idx < c && dk[j] >= 0) key = ((uint32_t)(dk[j] >> rows.S) << 12) | (uint32_t)idx;
         kb[0][idx] = key;
     }
     __syncthreads();
@@ -1473,7 +1493,7 @@ __device__ __forceinline__ void sp_bucket_range(const SpRows &rows, const int64_
 // Loads items [c0, c0 + SP_NT*IPT) of the bucket (blocked) as sort keys and
 // LDS values, sorts them, and returns the sorted keys.
 template <int IPT>
-__device__ __forceinline__ const uint32_t *sp_load_sort(const int32_t *__restrict__ dst_arr,
+__device__ __forceinline__ const uint32_t *sp_load_sort(int wmask, const int32_t *__restrict__ dst_arr,
                                                         const float *__restrict__ val_arr, int64_t start, int64_t c0,
                                                         int64_t n, uint32_t (*kb)[SP_CHUNK], float *val,
                                                         uint16_t *cnt, int *scan_lds) {
@@ -1485,7 +1505,7 @@ __device__ __forceinline__ const uint32_t *sp_load_sort(const int32_t *__restric
         if (c0 + k < n) {
             const int32_t d = dst_arr[start + c0 + k];
             if (d >= 0) {
-                dl = (uint32_t)d & (SP_W - 1);
+                dl = (uint32_t)d & (uint32_t)wmask;
                 val[k] = val_arr[start + c0 + k];
             }
         }
@@ -1515,7 +1535,7 @@ __device__ __forceinline__ void sp_chunk_regs(const int32_t *__restrict__ dst_ar
 }
 
 template <int IPT>
-__device__ __forceinline__ void sp_regs_to_lds(const int32_t *pd, const float *pv, uint32_t (*kb)[SP_CHUNK],
+__device__ __forceinline__ void sp_regs_to_lds(int wmask, const int32_t *pd, const float *pv, uint32_t (*kb)[SP_CHUNK],
                                                float *val) {
     const int t = threadIdx.x;
 #pragma unroll
@@ -1523,7 +1543,7 @@ __device__ __forceinline__ void sp_regs_to_lds(const int32_t *pd, const float *p
         const int k = t * IPT + j;
         uint32_t dl = SP_W;  // no item / hole: sorts last
         if (pd[j] >= 0) {
-            dl = (uint32_t)pd[j] & (SP_W - 1);
+            dl = (uint32_t)pd[j] & (uint32_t)wmask;
             val[k] = pv[j];
         }
         kb[0][k] = (dl << 11) | (uint32_t)k;
@@ -1620,12 +1640,12 @@ __device__ __forceinline__ void sp_raw_ranks(const uint32_t *key, int p0, int ra
 }
 
 template <int IPT>
-__device__ __forceinline__ void sp_accum_one(int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
+__device__ __forceinline__ void sp_accum_one(int wmask, int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
                              float *__restrict__ val_arr, int32_t *__restrict__ raw_local, int32_t *out_count, uint32_t (*kb)[SP_CHUNK],
                              float *val, uint16_t *cnt, int *scan_lds) {
     constexpr int SIZE = SP_NT * IPT;
     const int t = threadIdx.x;
-    const uint32_t *key = sp_load_sort<IPT>(dst_arr, val_arr, start, 0, n, kb, val, cnt, scan_lds);
+    const uint32_t *key = sp_load_sort<IPT>(wmask, dst_arr, val_arr, start, 0, n, kb, val, cnt, scan_lds);
     const float *sv = sp_sorted_values<IPT>(key, kb, val);
     int heads = 0;
 #pragma unroll
@@ -1655,40 +1675,25 @@ constexpr int SP_WB = FL_WAVE * SP_WIPT;  // 512 items
 constexpr int SP_SMALL_WAVES = SP_NT / FL_WAVE;
 constexpr int SP_MID_GRID = 2048;  // workgroups of the persistent mid-size kernel
 
-// A bucket of at most 64 * IPT items with at most SP_WFEW distinct
-// destinations, by one wave without a sort: the destinations are marked in
-// a bitmap, destination j (in destination order) is slot j and the bucket's
-// output j; each item's slot is ranked among the equal slots of its round
-// (64 items in raw order) with SP_WFEW_RB ballots, the values are scattered
-// slot-major in raw order within each slot, and lane j adds slot j's run to
-// 0 in order.  Holes are skipped.  Returns false, having written nothing,
-// when the bucket has more destinations.  LDS: bits (SP_W / 32 words), wpre
-// (their prefix counts), tab ((SP_WFEW) x (IPT + 1) counts), dl (slot
-// destinations), sv (64 * IPT values, 16-byte aligned).
+// Slots of a wave's items by destination: the destinations (d >= 0, modulo
+// the bucket's width) are marked in a bitmap (bits, SP_W / 32 words, wpre
+// their prefix counts); destination j in destination order is slot j
+// (dl_of[j]).  Returns the number of destinations; with more than SP_WFEW
+// the slots are not made.
 constexpr int SP_WFEW = 64;
 constexpr int SP_WFEW_RB = 6;
 template <int IPT>
-__device__ __forceinline__ bool sp_wave_few(int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
-                                            float *__restrict__ val_arr, int32_t *__restrict__ raw_local,
-                                            int32_t *out_count, uint32_t *bits, uint16_t *wpre, uint16_t *tab,
-                                            int16_t *dl_of, float *sv) {
+__device__ __forceinline__ int sp_wave_marks(const int32_t *d, int wmask, uint32_t *bits, uint16_t *wpre,
+                                             int16_t *dl_of) {
     constexpr int WPL = SP_W / 32 / FL_WAVE;  // bitmap words per lane
     const int lane = fl_lane();
-    int32_t d[IPT];
-    float v[IPT];
-#pragma unroll
-    for (int j = 0; j < IPT; ++j) {  // striped: round j, lane t holds item j*64 + t
-        const int64_t k = (int64_t)j * FL_WAVE + lane;
-        d[j] = k < n ? dst_arr[start + k] : -1;
-        v[j] = k < n ? val_arr[start + k] : 0.0f;
-    }
 #pragma unroll
     for (int q = 0; q < WPL; ++q) bits[lane * WPL + q] = 0;
     fl_wave_sync();
 #pragma unroll
     for (int j = 0; j < IPT; ++j) {
         if (d[j] < 0) continue;
-        const int x = d[j] & (SP_W - 1);
+        const int x = d[j] & wmask;
         const uint32_t b = 1u << (x & 31);
         if (!(bits[x >> 5] & b)) atomicOr(&bits[x >> 5], b);
     }
@@ -1702,7 +1707,7 @@ __device__ __forceinline__ bool sp_wave_few(int64_t start, int64_t n, int32_t db
     }
     const int incl = fl_wave_incl_scan_i32(c);
     const int total = __builtin_amdgcn_readlane(incl, FL_WAVE - 1);
-    if (total > SP_WFEW) return false;
+    if (total > SP_WFEW) return total;
     int pre = incl - c;
 #pragma unroll
     for (int q = 0; q < WPL; ++q) {
@@ -1714,6 +1719,38 @@ __device__ __forceinline__ bool sp_wave_few(int64_t start, int64_t n, int32_t db
         }
         pre += __popc(wd[q]);
     }
+    return total;
+}
+
+__device__ __forceinline__ int sp_wave_slot(int32_t d, int wmask, const uint32_t *bits, const uint16_t *wpre) {
+    const int x = d & wmask;
+    return wpre[x >> 5] + __popc(bits[x >> 5] & ((1u << (x & 31)) - 1u));
+}
+
+// A bucket of at most 64 * IPT items with at most SP_WFEW distinct
+// destinations, by one wave without a sort: slots by destination (above),
+// destination j the bucket's output j; each item's slot is ranked among the
+// equal slots of its round (64 items in raw order) with SP_WFEW_RB ballots,
+// the values are scattered slot-major in raw order within each slot, and
+// lane j adds slot j's run to 0 in order.  Holes are skipped.  Returns false,
+// having written nothing, when the bucket has more destinations.  LDS: tab
+// ((SP_WFEW) x (IPT + 1) counts), sv (64 * IPT values, 16-byte aligned).
+template <int IPT>
+__device__ __forceinline__ bool sp_wave_few(int wmask, int64_t start, int64_t n, int32_t dbase,
+                                            int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
+                                            int32_t *__restrict__ raw_local, int32_t *out_count, uint32_t *bits,
+                                            uint16_t *wpre, uint16_t *tab, int16_t *dl_of, float *sv) {
+    const int lane = fl_lane();
+    int32_t d[IPT];
+    float v[IPT];
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {  // striped: round j, lane t holds item j*64 + t
+        const int64_t k = (int64_t)j * FL_WAVE + lane;
+        d[j] = k < n ? dst_arr[start + k] : -1;
+        v[j] = k < n ? val_arr[start + k] : 0.0f;
+    }
+    const int total = sp_wave_marks<IPT>(d, wmask, bits, wpre, dl_of);
+    if (total > SP_WFEW) return false;
 #pragma unroll
     for (int j = 0; j < IPT; ++j) tab[lane * (IPT + 1) + j] = 0;
     fl_wave_sync();
@@ -1722,10 +1759,7 @@ __device__ __forceinline__ bool sp_wave_few(int64_t start, int64_t n, int32_t db
     for (int j = 0; j < IPT; ++j) {
         const bool valid = d[j] >= 0;
         int sj = 0;
-        if (valid) {
-            const int x = d[j] & (SP_W - 1);
-            sj = wpre[x >> 5] + __popc(bits[x >> 5] & ((1u << (x & 31)) - 1u));
-        }
+        if (valid) sj = sp_wave_slot(d[j], wmask, bits, wpre);
         uint32_t mlo, mhi;
         sp_peers<SP_WFEW_RB>((uint32_t)sj, __builtin_amdgcn_ballot_w64(valid), mlo, mhi);
         const uint32_t below = __builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u));
@@ -1804,22 +1838,23 @@ __global__ __launch_bounds__(SP_NT) void k_sp_accum_small(SpRows rows, const int
         if (lane == 0) *oc = 0;
         return;
     }
-    const int32_t dbase = (int32_t)(bk << SP_S);
+    const int32_t dbase = (int32_t)(bk << rows.S);
     // buckets of few destinations without a sort; the others go to the
     // workgroup sort of k_sp_accum_mid
     uint32_t *fbits = fw[w];
     uint16_t *fwpre = reinterpret_cast<uint16_t *>(fw[w] + FB_WORDS);
     int16_t *fdl = reinterpret_cast<int16_t *>(fw[w] + FB_WORDS + FP_WORDS);
     uint16_t *ftab = reinterpret_cast<uint16_t *>(fw[w] + FB_WORDS + FP_WORDS + FD_WORDS);
+    const int wmask = (1 << rows.S) - 1;
     bool done;
     if (n <= FL_WAVE)
-        done = sp_wave_few<1>(start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
+        done = sp_wave_few<1>(wmask, start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
     else if (n <= 2 * FL_WAVE)
-        done = sp_wave_few<2>(start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
+        done = sp_wave_few<2>(wmask, start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
     else if (n <= 4 * FL_WAVE)
-        done = sp_wave_few<4>(start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
+        done = sp_wave_few<4>(wmask, start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
     else
-        done = sp_wave_few<8>(start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
+        done = sp_wave_few<8>(wmask, start, n, dbase, dst_arr, val_arr, raw_local, oc, fbits, fwpre, ftab, fdl, val[w]);
     if (!done && lane == 0) mid_fb[atomicAdd(&lists[6], 1)] = (int32_t)slot;
 }
 
@@ -1850,12 +1885,13 @@ __global__ __launch_bounds__(SP_NT) void k_sp_accum_mid(SpRows rows, const int64
         int64_t start, end;
         sp_bucket_range(rows, base, r, bk, &start, &end);
         const int64_t n = end - start;
-        const int32_t dbase = (int32_t)(bk << SP_S);
+        const int32_t dbase = (int32_t)(bk << rows.S);
         int32_t *oc = &out_count[slot];
+        const int wmask = (1 << rows.S) - 1;
         if (n <= SP_NT * 4)
-            sp_accum_one<4>(start, n, dbase, dst_arr, val_arr, raw_local, oc, kb, val, cnt, scan_lds);
+            sp_accum_one<4>(wmask, start, n, dbase, dst_arr, val_arr, raw_local, oc, kb, val, cnt, scan_lds);
         else
-            sp_accum_one<8>(start, n, dbase, dst_arr, val_arr, raw_local, oc, kb, val, cnt, scan_lds);
+            sp_accum_one<8>(wmask, start, n, dbase, dst_arr, val_arr, raw_local, oc, kb, val, cnt, scan_lds);
     }
 }
 
@@ -1880,7 +1916,7 @@ constexpr int SP_FEW_TAB = SP_FEW * (SP_FEW_SPAN + 1);     // one count table, p
 constexpr int SP_FEW_PER = SP_FEW * SP_FEW_SPAN / SP_NT;   // scanned entries per thread
 static_assert(SP_FEW == (1 << SP_FEW_RB) && SP_FEW <= SP_NT, "one slot per thread");
 
-__device__ __forceinline__ void sp_few_one(int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
+__device__ __forceinline__ void sp_few_one(int wmask, int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
                                            float *__restrict__ val_arr, int32_t *__restrict__ raw_local,
                                            int32_t *out_count, int total, const uint32_t *bits, const int *wpre,
                                            const int32_t *slot_dl, uint16_t (*tab)[SP_FEW_TAB], float *sv,
@@ -1915,7 +1951,7 @@ __device__ __forceinline__ void sp_few_one(int64_t start, int64_t n, int32_t dba
             okm |= valid ? 1u << j : 0u;
             int sj = 0;
             if (valid) {
-                const int dl = pd[j] & (SP_W - 1);
+                const int dl = pd[j] & wmask;
                 sj = wpre[dl >> 5] + __popc(bits[dl >> 5] & ((1u << (dl & 31)) - 1u));
             }
             uint32_t mlo, mhi;
@@ -1996,6 +2032,7 @@ __global__ __launch_bounds__(SP_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) v
     __shared__ int claim;
     static_assert(SP_W / 32 == SP_NT, "one bitmap word per thread");
     const int t = threadIdx.x;
+    const int wmask = (1 << rows.S) - 1;
     const int nhot = ctr[0], nmid = ctr[2];
     // workgroups past the listed buckets take none: the others claim every
     // one (a participant stops only after a claim past the lists); the whole
@@ -2032,7 +2069,7 @@ __global__ __launch_bounds__(SP_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) v
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 if (dv[u] < 0) continue;
-                const int dl = dv[u] & (SP_W - 1);
+                const int dl = dv[u] & wmask;
                 const uint32_t b = 1u << (dl & 31);
                 if (!(bits[dl >> 5] & b)) atomicOr(&bits[dl >> 5], b);
             }
@@ -2056,7 +2093,7 @@ __global__ __launch_bounds__(SP_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) v
             slot_dl[q] = t * 32 + bit;
         }
         __syncthreads();
-        sp_few_one(start, n, (int32_t)(bk << SP_S), dst_arr, val_arr, raw_local, &out_count[slot], total, bits, wpre,
+        sp_few_one(wmask, start, n, (int32_t)(bk << rows.S), dst_arr, val_arr, raw_local, &out_count[slot], total, bits, wpre,
                    slot_dl, tab, sv, scan_lds);
     }
 }
@@ -2106,6 +2143,7 @@ __device__ __forceinline__ void sp_accum_hot_one(SpRows rows, const int64_t *__r
     sp_bucket_range(rows, base, r, bk, &start, &end);
     const int64_t n = end - start;
     const int t = threadIdx.x;
+    const int wmask = (1 << rows.S) - 1;
     for (int q = t; q < SP_W / 32; q += SP_NT) bits[q] = 0;
     // the next chunk's items are requested while this chunk is sorted and folded
     int32_t pd[SP_CHUNK_IPT];
@@ -2113,7 +2151,7 @@ __device__ __forceinline__ void sp_accum_hot_one(SpRows rows, const int64_t *__r
     sp_chunk_regs<SP_CHUNK_IPT>(dst_arr, val_arr, start, 0, n, pd, pv);
     for (int64_t c0 = 0; c0 < n; c0 += SP_CHUNK) {
         __syncthreads();  // previous chunk's folds done with kb / val
-        sp_regs_to_lds<SP_CHUNK_IPT>(pd, pv, kb, val);
+        sp_regs_to_lds<SP_CHUNK_IPT>(wmask, pd, pv, kb, val);
         if (c0 + SP_CHUNK < n) sp_chunk_regs<SP_CHUNK_IPT>(dst_arr, val_arr, start, c0 + SP_CHUNK, n, pd, pv);
         __syncthreads();
         const uint32_t *key = sp_block_sort<SP_CHUNK_IPT>(kb[0], kb[1], 11, 14, cnt, scan_lds);
@@ -2139,13 +2177,13 @@ __device__ __forceinline__ void sp_accum_hot_one(SpRows rows, const int64_t *__r
         for (int64_t k = t; k < n; k += SP_NT) {
             const int32_t d = dst_arr[start + k];
             if (d < 0) continue;  // hole
-            const int dl = d & (SP_W - 1);
+            const int dl = d & wmask;
             raw_local[start + k] =
                 wpre[dl >> 5] + __popc(bits[dl >> 5] & ((1u << (dl & 31)) - 1u));
         }
         __syncthreads();
     }
-    const int32_t dbase = (int32_t)(bk << SP_S);
+    const int32_t dbase = (int32_t)(bk << rows.S);
     uint32_t wd = word;
     int64_t o = start + pre;
     while (wd) {
@@ -2165,11 +2203,16 @@ __device__ __forceinline__ void sp_accum_hot_one(SpRows rows, const int64_t *__r
 // the earliest raw item; outputs are compacted in destination order as for
 // the sum, with the winning value (+0 for a zero), and raw_local[the item's
 // position] = the output index of winners, -1 for the other items.
-//   k_sp_max      buckets of at most SP_CHUNK items: stable LDS sort by
-//                 destination, the first thread of every run scans it;
-//   k_sp_max_hot  larger buckets: dense LDS arrays over the bucket's 8192
-//                 destinations, a max of the value keys, then a min of
-//                 (tie key, position) among the items holding the max.
+//   k_sp_max_small  wave per bucket of at most 512 items and 64
+//                 destinations: a largest value key and a smallest (tie key,
+//                 position) per slot, in LDS;
+//   k_sp_max_hot  larger buckets: the same over dense LDS arrays of the
+//                 bucket's destinations (12 bytes each: one workgroup a CU
+//                 at 8192 destinations, all that fit at 128);
+//   k_sp_max      what neither takes: buckets of at most SP_CHUNK items
+//                 where the dense arrays are wide, and those that hold a NaN:
+//                 stable LDS sort by destination, the first thread of every
+//                 run scans it.
 __device__ __forceinline__ float sp_canon(float v) { return v == 0.0f ? 0.0f : v; }
 
 __device__ __forceinline__ float fl_order_key_inv(uint32_t k) {
@@ -2177,7 +2220,7 @@ __device__ __forceinline__ float fl_order_key_inv(uint32_t k) {
 }
 
 template <int IPT>
-__device__ __forceinline__ void sp_max_one(int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
+__device__ __forceinline__ void sp_max_one(int wmask, int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
                            float *__restrict__ val_arr, const uint32_t *__restrict__ tie_arr,
                            int32_t *__restrict__ raw_local, int32_t *out_count,
                            uint32_t (*kb)[SP_CHUNK], float *val, uint32_t *tie, uint16_t *cnt,
@@ -2189,7 +2232,7 @@ __device__ __forceinline__ void sp_max_one(int64_t start, int64_t n, int32_t dba
         const int k = t * IPT + j;
         if (k < n) tie[k] = tie_arr[start + k];
     }
-    const uint32_t *key = sp_load_sort<IPT>(dst_arr, val_arr, start, 0, n, kb, val, cnt, scan_lds);
+    const uint32_t *key = sp_load_sort<IPT>(wmask, dst_arr, val_arr, start, 0, n, kb, val, cnt, scan_lds);
     int heads = 0;
 #pragma unroll
     for (int j = 0; j < IPT; ++j) heads += sp_is_head(key, t * IPT + j) ? 1 : 0;
@@ -2221,97 +2264,237 @@ __device__ __forceinline__ void sp_max_one(int64_t start, int64_t n, int32_t dba
     if (t == 0) *out_count = total;
 }
 
+// A bucket of at most 64 * IPT items, at most SP_WFEW destinations and no NaN
+// by one wave: slots by destination as for the sum, then per slot the largest
+// value key and, of the items that hold it, the smallest (tie key, position).
+// A slot's key is read before it is raised: of the many items of a popular
+// destination few are above all earlier ones.
+template <int IPT>
+__device__ __forceinline__ bool sp_wave_max(int wmask, int64_t start, int64_t n, int32_t dbase,
+                                            int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
+                                            const uint32_t *__restrict__ tie_arr, int32_t *__restrict__ raw_local,
+                                            int32_t *out_count, uint32_t *bits, uint16_t *wpre, int16_t *dl_of,
+                                            uint32_t *vbest, unsigned long long *tbest) {
+    const int lane = fl_lane();
+    int32_t d[IPT];
+    uint32_t key[IPT], tie[IPT];
+    bool nan = false;
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        const int64_t k = (int64_t)j * FL_WAVE + lane;
+        d[j] = k < n ? dst_arr[start + k] : -1;
+        const float v = k < n ? val_arr[start + k] : 0.0f;
+        tie[j] = k < n ? tie_arr[start + k] : 0u;
+        key[j] = fl_order_key(sp_canon(v));
+        nan |= d[j] >= 0 && v != v;
+    }
+    if (__ballot(nan) != 0) return false;
+    vbest[lane] = 0u;  // below the key of every value
+    tbest[lane] = ~0ull;
+    const int total = sp_wave_marks<IPT>(d, wmask, bits, wpre, dl_of);
+    if (total > SP_WFEW) return false;
+    fl_wave_sync();
+    int sl[IPT];
+#pragma unroll
+    for (int j = 0; j < IPT; ++j) {
+        sl[j] = d[j] >= 0 ? sp_wave_slot(d[j], wmask, bits, wpre) : 0;
+        if (d[j] >= 0 && key[j] > vbest[sl[j]]) atomicMax(&vbest[sl[j]], key[j]);
+    }
+    fl_wave_sync();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+        if (d[j] >= 0 && key[j] == vbest[sl[j]])
+            atomicMin(&tbest[sl[j]], ((unsigned long long)tie[j] << 32) | (unsigned)(j * FL_WAVE + lane));
+    fl_wave_sync();
+#pragma unroll
+    for (int j = 0; j < IPT; ++j)
+        if (raw_local && d[j] >= 0)
+            raw_local[start + (int64_t)j * FL_WAVE + lane] =
+                (uint32_t)tbest[sl[j]] == (uint32_t)(j * FL_WAVE + lane) ? sl[j] : -1;
+    // every item was read before: outputs may overwrite them
+    if (lane < total) {
+        dst_arr[start + lane] = dbase + dl_of[lane];
+        val_arr[start + lane] = fl_order_key_inv(vbest[lane]);
+    }
+    if (lane == 0) *out_count = total;
+    return true;
+}
+
+// One wave per (row, bucket) slot; larger buckets listed (lists[0] hot,
+// lists[2] the others; lists[1], lists[3] their claim counters).
+__global__ __launch_bounds__(SP_NT) void k_sp_max_small(SpRows rows, const int64_t *__restrict__ base,
+                                                       int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
+                                                       const uint32_t *__restrict__ tie_arr,
+                                                       int32_t *__restrict__ raw_local,
+                                                       int32_t *__restrict__ out_count, int64_t nslots,
+                                                       int32_t *__restrict__ hot_list,
+                                                       int32_t *__restrict__ mid_list, int32_t *__restrict__ lists) {
+    __shared__ uint32_t bits[SP_SMALL_WAVES][SP_W / 32];
+    __shared__ uint16_t wpre[SP_SMALL_WAVES][SP_W / 32];
+    __shared__ int16_t dl[SP_SMALL_WAVES][SP_WFEW];
+    __shared__ uint32_t vbest[SP_SMALL_WAVES][SP_WFEW];
+    __shared__ unsigned long long tbest[SP_SMALL_WAVES][SP_WFEW];
+    const int w = fl_wave_id();
+    const int64_t slot = fl_xcd_contig(blockIdx.x, gridDim.x) * SP_SMALL_WAVES + w;
+    if (slot >= nslots) return;  // no block barrier follows
+    const int64_t r = slot / rows.NB, bk = slot - r * rows.NB;
+    int64_t start, end;
+    sp_bucket_range(rows, base, r, bk, &start, &end);
+    const int64_t n = end - start;
+    const int lane = fl_lane();
+    int32_t *oc = &out_count[slot];
+    if (n == 0) {
+        if (lane == 0) *oc = 0;
+        return;
+    }
+    const int32_t dbase = (int32_t)(bk << rows.S);
+    const int wmask = (1 << rows.S) - 1;
+    bool done = false;
+    if (n <= FL_WAVE)
+        done = sp_wave_max<1>(wmask, start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, bits[w], wpre[w],
+                              dl[w], vbest[w], tbest[w]);
+    else if (n <= 2 * FL_WAVE)
+        done = sp_wave_max<2>(wmask, start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, bits[w], wpre[w],
+                              dl[w], vbest[w], tbest[w]);
+    else if (n <= 4 * FL_WAVE)
+        done = sp_wave_max<4>(wmask, start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, bits[w], wpre[w],
+                              dl[w], vbest[w], tbest[w]);
+    else if (n <= SP_WB)
+        done = sp_wave_max<8>(wmask, start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, bits[w], wpre[w],
+                              dl[w], vbest[w], tbest[w]);
+    if (!done && lane == 0) {
+        if (n > SP_CHUNK) hot_list[atomicAdd(&lists[0], 1)] = (int32_t)slot;
+        else mid_list[atomicAdd(&lists[2], 1)] = (int32_t)slot;
+    }
+}
+
+// Persistent grid over a list of buckets of at most SP_CHUNK items; ctr[0] =
+// listed buckets, ctr[1] = next one to claim.
 __global__ __launch_bounds__(SP_NT) void k_sp_max(SpRows rows, const int64_t *__restrict__ base,
                                                  int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
                                                  const uint32_t *__restrict__ tie_arr,
                                                  int32_t *__restrict__ raw_local, int32_t *__restrict__ out_count,
-                                                 int32_t *__restrict__ hot_list, int32_t *__restrict__ hot_count) {
+                                                 const int32_t *__restrict__ list, int32_t *__restrict__ ctr) {
     __shared__ __align__(16) uint32_t kb[2][SP_CHUNK];
     __shared__ float val[SP_CHUNK];
     __shared__ uint32_t tie[SP_CHUNK];
     __shared__ uint16_t cnt[SP_SORT_TAB];
     __shared__ int scan_lds[SP_NT / FL_WAVE + 1];
-    const int64_t r = blockIdx.x / rows.NB, bk = blockIdx.x - (blockIdx.x / rows.NB) * rows.NB;
-    int64_t start, end;
-    sp_bucket_range(rows, base, r, bk, &start, &end);
-    const int64_t n = end - start;
-    if (n > SP_CHUNK) {  // for k_sp_max_hot
-        if (threadIdx.x == 0) hot_list[atomicAdd(hot_count, 1)] = (int32_t)blockIdx.x;
-        return;
+    __shared__ int claim;
+    const int nlist = ctr[0];
+    if ((int)blockIdx.x >= nlist) return;  // no bucket left for this workgroup (see k_sp_accum_few)
+    for (;;) {
+        __syncthreads();  // the previous bucket is done with the LDS arrays
+        if (threadIdx.x == 0) claim = atomicAdd(&ctr[1], 1);
+        __syncthreads();
+        const int ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
+        if (ci >= nlist) break;
+        const int64_t slot = list[ci];
+        const int64_t r = slot / rows.NB, bk = slot - r * rows.NB;
+        int64_t start, end;
+        sp_bucket_range(rows, base, r, bk, &start, &end);
+        const int64_t n = end - start;
+        int32_t *oc = &out_count[slot];
+        const int32_t dbase = (int32_t)(bk << rows.S);
+        const int wmask = (1 << rows.S) - 1;
+        if (n <= SP_NT * 2)
+            sp_max_one<2>(wmask, start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, kb, val, tie, cnt,
+                          scan_lds);
+        else if (n <= SP_NT * 4)
+            sp_max_one<4>(wmask, start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, kb, val, tie, cnt,
+                          scan_lds);
+        else
+            sp_max_one<8>(wmask, start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, kb, val, tie, cnt,
+                          scan_lds);
     }
-    int32_t *oc = &out_count[r * rows.NB + bk];
-    if (n == 0) {
-        if (threadIdx.x == 0) *oc = 0;
-        return;
-    }
-    const int32_t dbase = (int32_t)(bk << SP_S);
-    if (n <= SP_NT * 2)
-        sp_max_one<2>(start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, kb, val, tie, cnt, scan_lds);
-    else if (n <= SP_NT * 4)
-        sp_max_one<4>(start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, kb, val, tie, cnt, scan_lds);
-    else
-        sp_max_one<8>(start, n, dbase, dst_arr, val_arr, tie_arr, raw_local, oc, kb, val, tie, cnt, scan_lds);
 }
 
-__device__ __forceinline__ void sp_max_hot_one(SpRows rows, const int64_t *__restrict__ base, int64_t r, int64_t bk,
-                               int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
-                               const uint32_t *__restrict__ tie_arr, int32_t *__restrict__ raw_local, int32_t *__restrict__ out_count, uint32_t *vbest,
-                               unsigned long long *tbest, uint32_t *bits, int *wpre, int *scan_lds);
+// Persistent grid over the listed buckets: the hot ones (ctr[0] listed,
+// ctr[1] claim) and, when mid_too, the others (ctr[2], ctr[3]), of which
+// those that hold a NaN go on to fb (ctr[6]).
+constexpr int SP_DENSE_MID_MAX = 1024;  // bucket widths whose dense arrays also serve the mid-size buckets
 
-// Persistent grid over the list of hot buckets collected by k_sp_max.
+__device__ __forceinline__ void sp_max_hot_one(SpRows rows, int64_t start, int64_t n, int64_t slot, int32_t dbase,
+                                               int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
+                                               const uint32_t *__restrict__ tie_arr, int32_t *__restrict__ raw_local,
+                                               int32_t *__restrict__ out_count, uint32_t *vbest,
+                                               unsigned long long *tbest, uint32_t *bits, int *wpre, int *scan_lds,
+                                               int *nan_seen, int32_t *fb, int32_t *fb_ctr);
+
 __global__ __launch_bounds__(SP_NT) void k_sp_max_hot(SpRows rows, const int64_t *__restrict__ base,
                                                      int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
                                                      const uint32_t *__restrict__ tie_arr,
                                                      int32_t *__restrict__ raw_local,
                                                      int32_t *__restrict__ out_count,
                                                      const int32_t *__restrict__ hot_list,
-                                                     int32_t *__restrict__ hot_count) {
-    __shared__ uint32_t vbest[SP_W];
-    __shared__ unsigned long long tbest[SP_W];
+                                                     const int32_t *__restrict__ mid_list, int mid_too,
+                                                     int32_t *__restrict__ fb, int32_t *__restrict__ ctr) {
+    extern __shared__ __align__(8) unsigned char max_lds[];  // per destination: (tie, position), then the value key
     __shared__ uint32_t bits[SP_W / 32];
     __shared__ int wpre[SP_W / 32];
     __shared__ int scan_lds[SP_NT / FL_WAVE + 1];
-    __shared__ int claim;
-    const int nhot = hot_count[0];
-    if ((int)blockIdx.x >= nhot) return;  // no bucket left for this workgroup (see k_sp_accum_few)
+    __shared__ int claim, nan_seen;
+    unsigned long long *tbest = reinterpret_cast<unsigned long long *>(max_lds);
+    uint32_t *vbest = reinterpret_cast<uint32_t *>(max_lds + ((size_t)8 << rows.S));
+    const int nhot = ctr[0], nmid = mid_too ? ctr[2] : 0;
+    if ((int)blockIdx.x >= nhot + nmid) return;  // no bucket left for this workgroup (see k_sp_accum_few)
     for (;;) {
         __syncthreads();  // the previous bucket is done with the LDS arrays
-        if (threadIdx.x == 0) claim = atomicAdd(&hot_count[1], 1);
+        if (threadIdx.x == 0) {
+            int c = atomicAdd(&ctr[1], 1);
+            if (c >= nhot && nmid > 0) c = nhot + atomicAdd(&ctr[3], 1);
+            claim = c;
+            nan_seen = 0;
+        }
         __syncthreads();
-        const int hi = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
-        if (hi >= nhot) break;
-        const int64_t slot = hot_list[hi];
-        sp_max_hot_one(rows, base, slot / rows.NB, slot % rows.NB, dst_arr, val_arr, tie_arr, raw_local,
-                       out_count, vbest, tbest, bits, wpre, scan_lds);
+        const int ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
+        if (ci >= nhot + nmid) break;
+        const int64_t slot = ci < nhot ? hot_list[ci] : mid_list[ci - nhot];
+        const int64_t r = slot / rows.NB, bk = slot - r * rows.NB;
+        int64_t start, end;
+        sp_bucket_range(rows, base, r, bk, &start, &end);
+        sp_max_hot_one(rows, start, end - start, slot, (int32_t)(bk << rows.S), dst_arr, val_arr, tie_arr, raw_local,
+                       out_count, vbest, tbest, bits, wpre, scan_lds, &nan_seen, ci < nhot ? nullptr : fb, ctr + 6);
     }
 }
 
-__device__ __forceinline__ void sp_max_hot_one(SpRows rows, const int64_t *__restrict__ base, int64_t r, int64_t bk,
-                               int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
-                               const uint32_t *__restrict__ tie_arr, int32_t *__restrict__ raw_local, int32_t *__restrict__ out_count, uint32_t *vbest,
-                               unsigned long long *tbest, uint32_t *bits, int *wpre, int *scan_lds) {
-    int64_t start, end;
-    sp_bucket_range(rows, base, r, bk, &start, &end);
-    const int64_t n = end - start;
+__device__ __forceinline__ void sp_max_hot_one(SpRows rows, int64_t start, int64_t n, int64_t slot, int32_t dbase,
+                                               int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
+                                               const uint32_t *__restrict__ tie_arr, int32_t *__restrict__ raw_local,
+                                               int32_t *__restrict__ out_count, uint32_t *vbest,
+                                               unsigned long long *tbest, uint32_t *bits, int *wpre, int *scan_lds,
+                                               int *nan_seen, int32_t *fb, int32_t *fb_ctr) {
     const int t = threadIdx.x;
-    for (int q = t; q < SP_W; q += SP_NT) {
+    const int W = 1 << rows.S, wmask = W - 1;
+    for (int q = t; q < W; q += SP_NT) {
         vbest[q] = 0u;  // below the key of every non-NaN value
         tbest[q] = ~0ull;
     }
     for (int q = t; q < SP_W / 32; q += SP_NT) bits[q] = 0;
     __syncthreads();
+#pragma unroll 4
     for (int64_t k = t; k < n; k += SP_NT) {
         const int32_t d = dst_arr[start + k];
         if (d < 0) continue;
-        const int dl = d & (SP_W - 1);
-        atomicMax(&vbest[dl], fl_order_key(sp_canon(val_arr[start + k])));
-        atomicOr(&bits[dl >> 5], 1u << (dl & 31));
+        const int dl = d & wmask;
+        const float v = val_arr[start + k];
+        const uint32_t key = fl_order_key(sp_canon(v));
+        // read first: few items of a popular destination raise its key
+        if (key > vbest[dl]) atomicMax(&vbest[dl], key);
+        const uint32_t b = 1u << (dl & 31);
+        if (!(bits[dl >> 5] & b)) atomicOr(&bits[dl >> 5], b);
+        if (fb && v != v) *nan_seen = 1;
     }
     __syncthreads();
+    if (fb && *nan_seen) {  // uniform: a NaN among the items of a mid-size bucket
+        if (t == 0) fb[atomicAdd(fb_ctr, 1)] = (int32_t)slot;
+        return;
+    }
+#pragma unroll 4
     for (int64_t k = t; k < n; k += SP_NT) {
         const int32_t d = dst_arr[start + k];
         if (d < 0) continue;
-        const int dl = d & (SP_W - 1);
+        const int dl = d & wmask;
         if (fl_order_key(sp_canon(val_arr[start + k])) == vbest[dl])
             atomicMin(&tbest[dl], ((unsigned long long)tie_arr[start + k] << 32) | (unsigned long long)k);
     }
@@ -2326,13 +2509,12 @@ __device__ __forceinline__ void sp_max_hot_one(SpRows rows, const int64_t *__res
         for (int64_t k = t; k < n; k += SP_NT) {
             const int32_t d = dst_arr[start + k];
             if (d < 0) continue;
-            const int dl = d & (SP_W - 1);
+            const int dl = d & wmask;
             const int o = wpre[dl >> 5] + __popc(bits[dl >> 5] & ((1u << (dl & 31)) - 1u));
             raw_local[start + k] = (uint32_t)tbest[dl] == (uint32_t)k ? o : -1;
         }
         __syncthreads();
     }
-    const int32_t dbase = (int32_t)(bk << SP_S);
     uint32_t wd = word;
     int64_t o = start + pre;
     while (wd) {
@@ -2343,7 +2525,7 @@ __device__ __forceinline__ void sp_max_hot_one(SpRows rows, const int64_t *__res
         val_arr[o] = fl_order_key_inv(vbest[dl]);
         ++o;
     }
-    if (t == 0) out_count[r * rows.NB + bk] = total;
+    if (t == 0) out_count[slot] = total;
 }
 
 // Wave per (row, bucket), four per workgroup: staged outputs -> COO at
@@ -2469,7 +2651,7 @@ __global__ __launch_bounds__(SP_NT) void k_sp_local_to_out(int64_t R, SpRows row
 #pragma unroll
         for (int j = 0; j < Q; ++j) {
             const uint32_t idx = (uint32_t)(j * SP_NT) + threadIdx.x;
-            fl_st32(tloc, idx, qq[j] >= 0 ? obase[dd[j] >> SP_S] + qq[j] : -1);
+            fl_st32(tloc, idx, qq[j] >= 0 ? obase[dd[j] >> rows.S] + qq[j] : -1);
         }
         return;
     }
@@ -2482,7 +2664,7 @@ __global__ __launch_bounds__(SP_NT) void k_sp_local_to_out(int64_t R, SpRows row
             int32_t o = -1;
             if (d >= 0) {
                 const int32_t loc = part_local[fl_ld32(tinv, idx)];
-                if (loc >= 0) o = (int32_t)((lds ? (int64_t)obase[d >> SP_S] : orow[d >> SP_S]) + loc);
+                if (loc >= 0) o = (int32_t)((lds ? (int64_t)obase[d >> rows.S] : orow[d >> rows.S]) + loc);
             }
             fl_st32(tloc, idx, o);
         } else {
@@ -2851,11 +3033,11 @@ __global__ void k_sp_finite(const float *__restrict__ w, int64_t count, unsigned
     if (__ballot(bad) != 0 && fl_lane() == 0) atomicOr(flag, 1ull);
 }
 
-__global__ void k_sp_plan_out(const int64_t *__restrict__ items, const int64_t *__restrict__ tiles, int64_t NB,
-                              const int64_t *__restrict__ chunks, int64_t *__restrict__ plan) {
+__global__ void k_sp_plan_out(const int64_t *__restrict__ items, const int64_t *__restrict__ tiles, int64_t E,
+                              int64_t R, const int64_t *__restrict__ chunks, int64_t *__restrict__ plan) {
     plan[0] = *items;
     plan[1] = *tiles;
-    plan[3] = NB;
+    plan[3] = sp_buckets_of(E, sp_shift(E, R, *items));
     plan[4] = chunks ? *chunks : 0;
 }
 
@@ -3241,7 +3423,8 @@ namespace {
 
 size_t al(size_t x) { return (x + 255) & ~(size_t)255; }
 
-int64_t sp_buckets(int64_t E) { return E <= 0 ? 1 : (E + SP_W - 1) / SP_W; }
+// buckets per row of a hop with that many items
+int64_t sp_buckets(int64_t E, int64_t R, int64_t items) { return sp_buckets_of(E, sp_shift(E, R, items)); }
 
 int sp_bucket_bits(int64_t NB) {
     int b = 0;
@@ -3496,7 +3679,7 @@ __global__ void k_cs_weighted_add(const int64_t *__restrict__ sb, const int64_t 
 
 extern "C" {
 
-int64_t fl_sparse_buckets(int64_t E) { return sp_buckets(E); }
+int64_t fl_sparse_buckets(int64_t E) { return sp_buckets(E, 0, 0); }
 
 size_t fl_sparse_plan_bytes(int64_t nnz, int64_t R, int64_t r_size) {
     if (nnz < 0 || R < 0 || r_size < 0) return 0;
@@ -3514,7 +3697,7 @@ static bool sp_quotas(const fl_sparse_hop *h) { return h->sampling_seed >= 0 && 
 // when every mask is a bitmap) with no edge factors.
 static bool sp_pos_optional(const fl_side *ori, const fl_side *inv, const fl_sparse_hop *h) {
     const auto side_ok = [](const fl_side *s) { return (!s->mask || s->mask_bits) && !s->dscore; };
-    return h->mode == SP_TOPK && h->aggregate == SP_SUM && sp_buckets(h->E) > 1 && side_ok(ori) && side_ok(inv);
+    return h->mode == SP_TOPK && h->aggregate == SP_SUM && sp_buckets(h->E, h->B * h->L, h->items) > 1 && side_ok(ori) && side_ok(inv);
 }
 
 int fl_sparse_plan(void *stream, const fl_side *ori, const fl_side *inv, const fl_sparse_hop *h, int64_t *plan) {
@@ -3580,14 +3763,14 @@ int fl_sparse_plan(void *stream, const fl_side *ori, const fl_side *inv, const f
               p.item_off, R, p.row_item0, p.ntiles);
     if ((rc = exclusive_scan(st, p.ntiles, p.tile_base, R, p.tmp)) != FL_OK) return rc;
     FL_LAUNCH("k_sp_plan_out", k_sp_plan_out, dim3(1), dim3(1), 0, st, p.item_off + nnz, p.tile_base + R,
-              sp_buckets(h->E), fixed ? (const int64_t *)nullptr : p.chunk_off + nnz, plan);
+              h->E, R, fixed ? (const int64_t *)nullptr : p.chunk_off + nnz, plan);
     return fl_check_launch("sparse_plan");
 }
 
 size_t fl_sparse_expand_bytes(int64_t items, int64_t tiles, int64_t chunks, int64_t R, int64_t E, int backward,
                               int aggregate) {
     if (items < 0 || tiles < 0 || chunks < 0 || R < 0) return 0;
-    return sp_exp_layout(items, tiles, chunks, R, sp_buckets(E), backward, aggregate, nullptr).bytes;
+    return sp_exp_layout(items, tiles, chunks, R, sp_buckets(E, R, items), backward, aggregate, nullptr).bytes;
 }
 
 // c2 budget of the plan and walk kernels: K > 0 selects, 0 keeps every
@@ -3601,7 +3784,9 @@ int fl_sparse_expand(void *stream, const fl_side *ori, const fl_side *inv, const
                      int64_t *out_base, int32_t *raw_local) {
     int rc;
     if ((rc = sp_check(ori, inv, h, "sparse_expand")) != FL_OK) return rc;
-    const int64_t R = h->B * h->L, NB = sp_buckets(h->E);
+    const int64_t R = h->B * h->L;
+    const int S = sp_shift(h->E, R, h->items);
+    const int64_t NB = sp_buckets_of(h->E, S);
     if (!h->ws1 || !h->ws2 || !out_base) return fl_fail(FL_ERR_ARG, "sparse_expand: null workspace or out_base");
     if (h->items < 0 || h->tiles < 0 || h->chunks < 0)
         return fl_fail(FL_ERR_ARG, "sparse_expand: negative plan sizes");
@@ -3622,7 +3807,7 @@ int fl_sparse_expand(void *stream, const fl_side *ori, const fl_side *inv, const
     const bool mx = h->aggregate == SP_MAX;
     hipStream_t st = (hipStream_t)stream;
     const int64_t nnz = h->nnz;
-    SpRows rows{p.row_item0, p.tile_base, NB};
+    SpRows rows{p.row_item0, p.tile_base, NB, S};
     if (nnz > 0 && h->mode == SP_FIXED)
         FL_LAUNCH("k_fx_fill", k_fx_fill, dim3((unsigned)((nnz + SEL_NT / FL_WAVE - 1) / (SEL_NT / FL_WAVE))),
                   dim3(SEL_NT), 0, st, *ori, *inv, h->sp_e, h->sp_v, nnz, p.cut, p.item_off, x.raw_dst, x.raw_val);
@@ -3706,10 +3891,18 @@ int fl_sparse_expand(void *stream, const fl_side *ori, const fl_side *inv, const
     if (R * NB > 0)
         FL_LAUNCH("k_fill_i32", k_fill_i32, dim3(1), dim3(64), 0, st, x.hot_count, (int64_t)8, 0);
     if (R * NB > 0 && mx) {
-        FL_LAUNCH("k_sp_max", k_sp_max, dim3((unsigned)(R * NB)), dim3(SP_NT), 0, st, rows, x.base, dst_arr,
-                  val_arr, tie_arr, acc_local, x.out_count, x.hot_list, x.hot_count);
-        FL_LAUNCH("k_sp_max_hot", k_sp_max_hot, dim3(hot_grid), dim3(SP_NT), 0, st, rows, x.base, dst_arr, val_arr,
-                  tie_arr, acc_local, x.out_count, x.hot_list, x.hot_count);
+        const int64_t nslot = R * NB;
+        const bool dense = ((int64_t)1 << S) <= SP_DENSE_MID_MAX;
+        FL_LAUNCH("k_sp_max_small", k_sp_max_small, dim3((unsigned)((nslot + SP_SMALL_WAVES - 1) / SP_SMALL_WAVES)),
+                  dim3(SP_NT), 0, st, rows, x.base, dst_arr, val_arr, tie_arr, acc_local, x.out_count, nslot,
+                  x.hot_list, x.mid_list, x.hot_count);
+        // (a bucket of any size may have more than SP_WFEW destinations)
+        const int64_t any_g = R * NB < SP_MID_GRID ? R * NB : SP_MID_GRID;
+        FL_LAUNCH("k_sp_max_hot", k_sp_max_hot, dim3(dense ? (unsigned)any_g : hot_grid), dim3(SP_NT),
+                  (size_t)12 << S, st, rows, x.base, dst_arr, val_arr, tie_arr, acc_local, x.out_count, x.hot_list,
+                  x.mid_list, dense ? 1 : 0, x.mid_fb, x.hot_count);
+        FL_LAUNCH("k_sp_max", k_sp_max, dim3((unsigned)any_g), dim3(SP_NT), 0, st, rows, x.base, dst_arr, val_arr,
+                  tie_arr, acc_local, x.out_count, dense ? x.mid_fb : x.mid_list, x.hot_count + (dense ? 6 : 2));
     } else if (R * NB > 0) {
         const int64_t nslot = R * NB;
         FL_LAUNCH("k_sp_accum_small", k_sp_accum_small,
@@ -3738,11 +3931,13 @@ int fl_sparse_expand(void *stream, const fl_side *ori, const fl_side *inv, const
 int fl_sparse_emit(void *stream, const fl_sparse_hop *h, const int64_t *out_base, int64_t *out_b, int64_t *out_l,
                    int64_t *out_e, float *out_v) {
     if (!h || !out_base) return fl_fail(FL_ERR_ARG, "sparse_emit: null argument");
-    const int64_t R = h->B * h->L, NB = sp_buckets(h->E);
+    const int64_t R = h->B * h->L;
+    const int S = sp_shift(h->E, R, h->items);
+    const int64_t NB = sp_buckets_of(h->E, S);
     if (R * NB == 0) return FL_OK;
     SpPlan p = sp_plan_layout(h->nnz, R, sp_rsize(h), (char *)h->ws1);
     SpExp x = sp_exp_layout(h->items, h->tiles, h->chunks, R, NB, 0, h->aggregate, (char *)h->ws2);
-    SpRows rows{p.row_item0, p.tile_base, NB};
+    SpRows rows{p.row_item0, p.tile_base, NB, S};
     FL_LAUNCH("k_sp_emit", k_sp_emit, dim3((unsigned)((R * NB + SP_EMIT_SLOTS - 1) / SP_EMIT_SLOTS)),
               dim3(SP_EMIT_WAVES * FL_WAVE), 0, (hipStream_t)stream, rows, h->L, R * NB, x.base,
               NB > 1 ? x.part_dst : x.raw_dst, NB > 1 ? x.part_val : x.raw_val, out_base, out_b, out_l, out_e,

@@ -341,8 +341,9 @@ typedef struct fl_sparse_hop {
                                           error 1                            */
 } fl_sparse_hop;
 
-/* Destination buckets per row (8192 entities each).  The sparse hop
- * supports E <= 2^27 entities. */
+/* The most destination buckets a row can have (64 to 8192 entities each, by
+ * the hop's size: fl_sparse_plan reports the hop's own number).  The sparse
+ * hop supports E <= 2^27 entities. */
 int64_t fl_sparse_buckets(int64_t E);
 
 /* Plan workspace bytes for nnz entries, R = B*L rows and r_size relations
