@@ -183,6 +183,18 @@ _SIGS = {
     "fl_rule_accumulate_bytes": (ctypes.c_size_t, [ctypes.c_int64] * 3),
     "fl_rule_accumulate": (ctypes.c_int, [ctypes.c_void_p] * 5 + [ctypes.c_int64, ctypes.c_void_p] +
                            [ctypes.c_int64] * 4 + [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t]),
+    "fl_rule_ground_max_entities": (ctypes.c_int64, []),
+    "fl_rule_ground_bytes": (ctypes.c_size_t, [ctypes.c_int64] * 3),
+    "fl_rule_ground": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(FlSide), ctypes.POINTER(FlSide),
+                                      ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p, ctypes.c_void_p] +
+                       [ctypes.c_int64] * 3 + [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64, ctypes.c_int,
+                                               ctypes.c_int, ctypes.c_void_p, ctypes.c_int64, ctypes.c_void_p,
+                                               ctypes.c_size_t, ctypes.c_void_p]),
+    "fl_rule_collect_bytes": (ctypes.c_size_t, [ctypes.c_int64] * 2),
+    "fl_rule_collect_plan": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_int64, ctypes.c_int64,
+                                            ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]),
+    "fl_rule_collect_fill": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_int64] * 3 +
+                             [ctypes.c_void_p] * 4),
     "fl_rule_finalize": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_int64] * 3 +
                          [ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p]),
     "fl_filtered_ranks_workspace_bytes": (ctypes.c_size_t, [ctypes.c_int64, ctypes.c_int]),

@@ -30,6 +30,7 @@ and sparse accumulators change only how the exact integer path counts are
 produced or the order of floating-point additions of the normalizers, not
 the values of the channel sums.
 """
+import ctypes
 import types
 import weakref
 
@@ -131,6 +132,71 @@ def _finalize(dense, nb, E, final_max):
     return keys, total[keys]
 
 
+# Room for the final states of a chunk in the one-launch grounding (8 bytes an entry).
+_POOL_ENTRIES = 1 << 25
+
+
+def _grounds_in_one_launch(ev, csr, entities, device):
+    """True when the chunks can be grounded by fl_rule_ground: this package's own grounding hooks, CSR arrays on
+    the GPU and entities that fit its accumulators."""
+    return (device.type == "cuda" and ev is _default_ev() and len(csr) >= 16 and 0 < entities
+            and ev.vectorized_operation_sparse3d_fixed_relation is fk.vectorized_operation_sparse3d_fixed_relation
+            and ev.initial_rule_state.__module__ == ev.__name__
+            and entities <= _lib.lib().fl_rule_ground_max_entities())
+
+
+def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, relations, E, block, is_max, boolean_paths,
+                         final_max, stats):
+    """(rows, columns, scores) of the blocks of sources with every chunk of rules grounded by one launch
+    (fl_rule_ground) and the scored entities collected with one host read per block, or None when a state outgrew
+    what those kernels hold (the caller grounds step by step)."""
+    lib = _lib.lib()
+    device = sources.device
+    sides = fk._fixed_sides(csr)
+    ranks = weights.shape[1]
+    lengths_d = torch.tensor(lengths, dtype=torch.int32).to(device)
+    st = fk._stream(sources)
+    parts = []
+    for s0 in range(0, sources.numel(), block):
+        src = sources[s0:s0 + block]
+        nb = src.numel()
+        dense = torch.zeros((ranks, nb * E), dtype=torch.float32, device=device)
+        status = torch.zeros(1, dtype=torch.int64, device=device)
+        widest = max(hi - lo for lo, hi in chunks)
+        pool = min(nb * widest * E, _POOL_ENTRIES)
+        collect_bytes = lib.fl_rule_collect_bytes(nb, E)
+        ws_bytes = max(lib.fl_rule_ground_bytes(nb, widest, pool), collect_bytes)
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+        for lo, hi in chunks:
+            check(lib.fl_rule_ground(st, ctypes.byref(sides.ori), ctypes.byref(sides.inv), ptr(src), nb,
+                                     ptr(operators[lo:hi]), ptr(lengths_d[lo:hi]), hi - lo, operators.shape[1],
+                                     int(relations), ptr(weights[lo:hi]), ranks, E, 1 if boolean_paths else 0,
+                                     1 if is_max else 0, ptr(dense), pool, ptr(ws), ws_bytes, ptr(status)),
+                  "rule_ground")
+        rowsum = torch.empty(ranks * nb, dtype=torch.float32, device=device)
+        total = torch.empty(nb * E, dtype=torch.float32, device=device)
+        check(lib.fl_rule_finalize(st, ptr(dense), ranks, nb, E, 1 if final_max else 0, ptr(rowsum), ptr(total)),
+              "rule_finalize")
+        info = torch.empty(2, dtype=torch.int64, device=device)
+        check(lib.fl_rule_collect_plan(st, ptr(total), nb, E, ptr(status), ptr(ws), ws_bytes, ptr(info)),
+              "rule_collect")
+        count, bad = info.tolist()
+        if bad == 1:
+            raise ValueError("sparse state index out of range for shape (%d, %d, %d)" % (nb, widest, E))
+        if bad:
+            return None
+        idx = torch.empty((2, count), dtype=torch.int64, device=device)
+        vals = torch.empty(count, dtype=torch.float32, device=device)
+        check(lib.fl_rule_collect_fill(st, ptr(total), nb, E, s0, ptr(ws), ptr(idx[0]), ptr(idx[1]), ptr(vals)),
+              "rule_collect")
+        parts.append((idx, vals))
+    stats["chunks"] += len(chunks) * len(parts)
+    stats["ground_calls"] += len(parts) * sum(max(lengths[lo:hi]) for lo, hi in chunks)
+    if len(parts) == 1:
+        return parts[0]
+    return torch.cat([i for i, _ in parts], 1), torch.cat([v for _, v in parts])
+
+
 @torch.inference_mode()
 def score(ev, sources, rules, csr, relations, entities, chunk_size,
           final_max=False, reduction="sum", boolean_paths=False, dense_budget_bytes=None,
@@ -210,6 +276,16 @@ def score(ev, sources, rules, csr, relations, entities, chunk_size,
     stats["dense_accumulation"] = True
     stats["prefix_enabled"] = False
     is_max = reduction == "max"
+    if _grounds_in_one_launch(ev, csr, E, device):
+        chunks = [(lo, min(lo + chunk_size, len(rules))) for lo in range(0, len(rules), chunk_size)]
+        try:
+            found = _score_in_one_launch(sources.contiguous(), chunks, operators, lengths, weights, csr, relations, E,
+                                         block, is_max, boolean_paths, final_max, stats)
+        except torch.cuda.OutOfMemoryError:
+            found = None  # step by step, with chunks halved as far as needed
+            torch.cuda.empty_cache()
+        if found is not None:
+            return torch.sparse_coo_tensor(*found, shape, is_coalesced=True)
 
     def advance(state, ops, nb):
         stats["ground_calls"] += 1

@@ -587,6 +587,38 @@ int fl_rule_accumulate(void *stream, const int64_t *sb, const int64_t *sl,
 int fl_rule_finalize(void *stream, const float *dense, int64_t K, int64_t B,
                      int64_t E, int final_max, float *rowsum, float *total);
 
+/* Grounds a chunk of C rules from nb sources and adds it to dense, as the
+ * fixed-relation steps of every operator followed by fl_rule_accumulate do
+ * (the same terms in the same order), without a host read.  operators
+ * [C, steps] (ids as the fixed-relation step takes them), lengths [C] a
+ * rule's operators; boolean_paths: every state 0 or 1.  pool: room for that
+ * many final state entries, at most nb * C * E are needed.  At most
+ * fl_rule_ground_max_entities() entities.  status (device, zeroed by the
+ * caller before the first of the calls that share it) receives 1 when a
+ * source is outside [0, E), 2 when a path count reached 2^24, a row passed
+ * 2^20 edges in a step or the pool was too small: dense is then not what it
+ * should be and the caller takes the steps one by one. */
+int64_t fl_rule_ground_max_entities(void);
+size_t fl_rule_ground_bytes(int64_t nb, int64_t C, int64_t pool);
+int fl_rule_ground(void *stream, const fl_side *ori, const fl_side *inv,
+                   const int64_t *sources, int64_t nb,
+                   const int64_t *operators, const int32_t *lengths,
+                   int64_t C, int64_t steps, int64_t r_size, const float *W,
+                   int64_t K, int64_t E, int boolean_paths, int is_max,
+                   float *dense, int64_t pool, void *ws, size_t ws_bytes,
+                   int64_t *status);
+
+/* The nonzero cells of total [B, E] in order: plan writes info (device
+ * int64[2]) = {their number, *status or 0}; the host reads it, allocates and
+ * fill writes (row0 + b, e, value) with the same workspace. */
+size_t fl_rule_collect_bytes(int64_t B, int64_t E);
+int fl_rule_collect_plan(void *stream, const float *total, int64_t B,
+                         int64_t E, const int64_t *status, void *ws,
+                         size_t ws_bytes, int64_t *info);
+int fl_rule_collect_fill(void *stream, const float *total, int64_t B,
+                         int64_t E, int64_t row0, void *ws, int64_t *out_b,
+                         int64_t *out_e, float *out_v);
+
 /* ---- evaluation --------------------------------------------------------- */
 
 /* Replaces the rank computation of calculate_hits_full_with_filter_indices

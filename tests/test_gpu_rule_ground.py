@@ -1,0 +1,120 @@
+"""Rule scoring with every chunk grounded by one launch, bit for bit against
+the same call grounded operator by operator (a hook object with this
+package's own steps), and against the float64 oracle: states at the edge of
+the hash table, states that outgrow it, path counts and rows beyond the
+kernels' limits, a pool that is too small, and entity counts around the
+largest the accumulators hold."""
+import types
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+from tests.helpers import to_torch_csr
+
+pytestmark = pytest.mark.gpu
+
+
+def _score(ev, *a, **k):
+    from flashlog_amd.rules import shared_inference as si
+    return si.score(ev, *a, **k)
+
+
+def _stepwise():
+    from flashlog_amd.rules import evaluate as ev
+    return types.SimpleNamespace(
+        initial_rule_state=ev.initial_rule_state,
+        vectorized_operation_sparse3d_fixed_relation=ev.vectorized_operation_sparse3d_fixed_relation,
+        advance_single_rule_state_memory_bounded=ev.advance_single_rule_state_memory_bounded)
+
+
+def _graph(E, fans, pairs=()):
+    """Relation i: node i to fans[i] distinct nodes; relation len(fans): node
+    j to j + 1; then the edges (h, relation, t) of pairs."""
+    rng = np.random.default_rng(5)
+    h, r, t = [np.arange(E - 1)], [np.full(E - 1, len(fans))], [np.arange(1, E)]
+    for i, n in enumerate(fans):
+        h.append(np.full(n, i))
+        r.append(np.full(n, i))
+        t.append(rng.choice(E, n, replace=False))
+    for a, b, c in pairs:
+        h.append(np.asarray(a))
+        r.append(np.full(len(a), b))
+        t.append(np.asarray(c))
+    return tuple(np.concatenate(x).astype(np.int64) for x in (h, r, t))
+
+
+def _both(E, R, trip, sources, bodies, one_launch=True, monkeypatch=None, oracle=True, **kw):
+    from flashlog_amd.rules import shared_inference as si
+    h, r, t = trip
+    tc = to_torch_csr(O.build_csr_structure(h, t, r, E), torch.device("cuda"))
+    W = np.random.default_rng(9).random((len(bodies), 2)).astype(np.float32)
+    rules = [{"body": b, "rank_weights": [float(x) for x in w]} for b, w in zip(bodies, W)]
+    src = torch.tensor(sources).cuda()
+    used = []
+    real = si._score_in_one_launch
+    if monkeypatch is not None:
+        monkeypatch.setattr(si, "_score_in_one_launch", lambda *a: used.append(real(*a)) or used[-1])
+    got = _score(None, src, rules, tc, R, E, 5, **kw)
+    assert not one_launch or used == [] or used[0] is not None
+    want = _score(_stepwise(), src, rules, tc, R, E, 5, **kw)
+    assert torch.equal(got.indices(), want.indices()) and torch.equal(got.values(), want.values())
+    if oracle:
+        ref = O.rule_scores(h, r, t, E, R, sources, bodies, W.astype(np.float64), kw.get("reduction", "sum"),
+                            kw.get("boolean_paths", False), kw.get("final_max", False))
+        # two float32 divisions and at most len(bodies) + 2 additions and products per score
+        np.testing.assert_allclose(got.to_dense().cpu().numpy(), ref, rtol=(len(bodies) + 6) * 2.0 ** -24, atol=1e-30)
+    return used
+
+
+@pytest.mark.parametrize("kw", [{}, {"boolean_paths": True}, {"reduction": "max"},
+                                {"reduction": "max", "final_max": True}])
+@pytest.mark.parametrize("E", [1700, 16384, 16385])
+def test_state_sizes(monkeypatch, E, kw):
+    """Endpoints just below, at and above the hash table's 1536, and repeated
+    paths to one endpoint."""
+    fans = [0, 1, 63, 64, 128, 129, 1535, 1536, 1537, 1600]
+    R = len(fans) + 3
+    back = np.arange(200)
+    trip = _graph(E, fans, [(back, R - 2, np.full(200, 3)), (np.full(200, 3), R - 1, back)])
+    bodies = [[i] for i in range(len(fans))] + [[i, len(fans)] for i in range(len(fans))]
+    bodies += [[2 * R], [], [R - 1, R - 2, R - 1], [R + 3, 4, 2 * R], [R - 1, 2 * R, R - 2], [R + R - 2, R - 2],
+               [9, len(fans), R + len(fans)]]
+    used = _both(E, R, trip, [0, 1, 2, 3, 6, 7, 8, 9, 9, E - 1], bodies, monkeypatch=monkeypatch, **kw)
+    assert (used != []) == (E <= 16384)
+
+
+@pytest.mark.parametrize("case", ["paths", "edges", "pool"])
+def test_beyond_the_limits(monkeypatch, case):
+    from flashlog_amd.rules import shared_inference as si
+    if case == "pool":
+        E, R = 1700, 3
+        monkeypatch.setattr(si, "_POOL_ENTRIES", 100)
+        trip = _graph(E, [700])
+        bodies = [[0], [0, 1]]
+    elif case == "paths":
+        # 300 parallel edges there, back and there again: 300^3 paths above 2^24
+        E, R = 500, 3
+        trip = _graph(E, [2], [(np.full(300, 7), 2, np.full(300, 8))])
+        bodies = [[2], [2, R + 2], [2, R + 2, 2]]
+    else:
+        # one row of 2^20 + 1 edges in a step
+        E, R = 3000, 3
+        n = (1 << 20) + 1
+        trip = _graph(E, [2], [(np.full(n, 7), 2, np.arange(n) % E)])
+        bodies = [[2], [1, 2]]
+    used = _both(E, R, trip, [0, 7, 8], bodies, one_launch=False, monkeypatch=monkeypatch, oracle=case != "edges")
+    assert used == [None]
+
+
+def test_source_outside():
+    E, R = 400, 3
+    h, r, t = _graph(E, [2])
+    tc = to_torch_csr(O.build_csr_structure(h, t, r, E), torch.device("cuda"))
+    from flashlog_amd.rules import shared_inference as si
+    ops = torch.tensor([[0]]).cuda()
+    W = torch.ones(1, 1).cuda()
+    with pytest.raises(ValueError, match="out of range"):
+        si._score_in_one_launch(torch.tensor([1, E]).cuda(), [(0, 1)], ops, [1], W, tc, R, E, 2, False, False, False,
+                                {"chunks": 0, "ground_calls": 0})
