@@ -2979,14 +2979,24 @@ __global__ void k_sp_order_check(const int32_t *__restrict__ seen, int64_t nnz, 
     if (i < nnz && seen[i] != 1) atomicMax((unsigned long long *)err, 1ull);
 }
 
-// Entry visiting order by source entity, in blocks of SP_ORD_BLK entity ids
-// (a counting sort over the blocks; the entries of one block in any order):
+// Entry visiting order by source entity, in blocks of 2^shift entity ids (a
+// counting sort over the blocks; the entries of one block in any order):
 // rank[i] = the entry's slot among its block's entries, then
 // order[start of block + rank] = i.  Entity ids outside [0, E) share the
 // last bin (the plan reports them).
-constexpr int SP_ORD_SHIFT = 6;  // 64 entity ids per block
+//   Blocks of 64 ids, fewer where that leaves less than SP_ORD_BINS counters:
+// an entry's rank is an atomic on its block's counter, and 60,000 entries on
+// the 47 counters of 3,000 entities took 210 us (one counter an entity: 6).
+constexpr int SP_ORD_SHIFT = 6;
+constexpr int64_t SP_ORD_BINS = 1 << 16;
+__host__ __device__ __forceinline__ int sp_ord_shift(int64_t E) {
+    int s = 0;
+    while (s < SP_ORD_SHIFT && (E >> s) > SP_ORD_BINS) ++s;
+    return s;
+}
 __device__ __forceinline__ int64_t sp_ord_bin(int64_t e, int64_t E) {
-    return (e >= 0 && e < E) ? (e >> SP_ORD_SHIFT) : (E >> SP_ORD_SHIFT) + 1;
+    const int s = sp_ord_shift(E);
+    return (e >= 0 && e < E) ? (e >> s) : (E >> s) + 1;
 }
 
 __global__ void k_sp_ord_count(const int64_t *__restrict__ se, int64_t nnz, int64_t E, int32_t *__restrict__ cnt,
@@ -4219,9 +4229,9 @@ int fl_sparse_race_select_compact(void *stream, const int64_t *sp_b, const int64
     return fl_check_launch("sparse_race_select");
 }
 
-// the count bins of the entry order: (E >> SP_ORD_SHIFT) + 1 blocks and one
+// the count bins of the entry order: (E >> shift) + 1 blocks and one
 // for out-of-range ids
-static int64_t sp_ord_bins(int64_t E) { return (E >> SP_ORD_SHIFT) + 2; }
+static int64_t sp_ord_bins(int64_t E) { return (E >> sp_ord_shift(E)) + 2; }
 
 static size_t sp_order_layout(int64_t nnz, int64_t E, char *base, int32_t **cnt, int32_t **rank, int64_t **start,
                               int64_t **tmp) {

@@ -977,22 +977,27 @@ def dense_filtered_ranks_cuda(state, targets, filter_indices=None, use_eql=False
     targets = targets.long().contiguous()
     if targets.numel() != B:
         raise ValueError("dense_filtered_ranks_cuda: one target per query")
-    if B and (int(targets.min()) < 0 or int(targets.max()) >= E):
-        raise ValueError("dense_filtered_ranks_cuda: target out of range")
-    keys = None
-    if filter_indices is not None:
-        fb, fe = filter_indices
-        batch_idx = torch.arange(B, device=state.device, dtype=torch.long)
-        fb = torch.cat([fb.to(state.device).long(), batch_idx])
-        fe = torch.cat([fe.to(state.device).long(), targets])
-        if fb.numel() and (int(fb.min()) < 0 or int(fb.max()) >= B or int(fe.min()) < 0 or int(fe.max()) >= E):
-            raise ValueError("dense_filtered_ranks_cuda: filter index out of range")
-        keys = torch.unique(fb * E + fe)
     ranks = torch.empty(B, dtype=torch.float32, device=state.device)
-    check(_lib.lib().fl_dense_filtered_ranks(_stream(state), ptr(state), ptr(targets),
-                                             ptr(keys) if keys is not None else None,
-                                             keys.numel() if keys is not None else 0, B, E,
-                                             1 if use_eql else 0, ptr(ranks)), "dense_filtered_ranks_cuda")
+    if B == 0:
+        return ranks
+    fb = fe = None
+    if filter_indices is not None:
+        fb, fe = (x.to(state.device).long().contiguous() for x in filter_indices)
+        if fb.dim() != 1 or fb.shape != fe.shape:
+            raise ValueError("dense_filtered_ranks_cuda: filter indices must be equal 1D tensors")
+    n = fb.numel() if fb is not None else 0
+    lib = _lib.lib()
+    ws_bytes = lib.fl_dense_filtered_ranks_pairs_bytes(n, B)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=state.device)
+    err = torch.empty(1, dtype=torch.int64, device=state.device)
+    check(lib.fl_dense_filtered_ranks_pairs(_stream(state), ptr(state), ptr(targets), ptr(fb), ptr(fe), n,
+                                            1 if filter_indices is not None else 0, B, E, 1 if use_eql else 0,
+                                            ptr(ranks), ptr(ws), ws_bytes, ptr(err)), "dense_filtered_ranks_cuda")
+    bad = int(err)
+    if bad & 1:
+        raise ValueError("dense_filtered_ranks_cuda: target out of range")
+    if bad & 2:
+        raise ValueError("dense_filtered_ranks_cuda: filter index out of range")
     return ranks
 
 

@@ -633,6 +633,19 @@ int fl_dense_filtered_ranks(void *stream, const float *state, const int64_t *tar
                             const int64_t *filter_keys, int64_t n_filter, int64_t B,
                             int64_t E, int use_eql, float *ranks);
 
+/* The same from the filter's pairs as they come (unsorted, duplicates
+ * counted once, the targets joined by the call; filtered = 0: no filtering,
+ * n_pairs = 0): err (device) receives 1 when a target is outside [0, E), 2
+ * when a pair is outside [B, E], 3 for both; ranks are then unspecified. */
+size_t fl_dense_filtered_ranks_pairs_bytes(int64_t n_pairs, int64_t B);
+int fl_dense_filtered_ranks_pairs(void *stream, const float *state,
+                                  const int64_t *targets,
+                                  const int64_t *filter_b,
+                                  const int64_t *filter_e, int64_t n_pairs,
+                                  int filtered, int64_t B, int64_t E,
+                                  int use_eql, float *ranks, void *ws,
+                                  size_t ws_bytes, int64_t *err);
+
 /* Replaces the known-answer expansion of the filtered evaluation
  * (src/main.py:212-276, _expand_filter_side): per query q with key
  * keys[q] = source * R + relation, the columns (in CSR order) of that

@@ -1,0 +1,40 @@
+"""Dense filtered ranks from pairs as they come: duplicates, any order, the
+targets among them, rows of every alignment, no pairs, and indices out of
+range, against the oracle (whole counts: equal)."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,E,n", [(1, 1, 0), (1, 5, 7), (3, 257, 1), (7, 1022, 5000), (64, 3001, 63), (5, 40001, 31)])
+@pytest.mark.parametrize("use_eql", [False, True])
+@pytest.mark.parametrize("filtered", [False, True])
+def test_ranks_from_pairs(B, E, n, use_eql, filtered):
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    rng = np.random.default_rng(B * 1000 + n)
+    state = np.round(rng.random((B, E)) * 5).astype(np.float32)
+    state[rng.random((B, E)) < 0.3] = 0
+    if E > 3:
+        state[0, 1], state[B - 1, 2], state[0, 3] = np.nan, np.inf, -np.inf
+    targets = rng.integers(0, E, B)
+    fb, fe = rng.integers(0, B, n), rng.integers(0, min(E, 50), n)
+    got = fk.dense_filtered_ranks_cuda(torch.from_numpy(state).cuda(), torch.from_numpy(targets).cuda(),
+                                       (torch.from_numpy(fb).cuda(), torch.from_numpy(fe).int().cuda()) if filtered
+                                       else None, use_eql)
+    want = O.dense_filtered_ranks(state, targets, fb if filtered else None, fe if filtered else None, use_eql)
+    np.testing.assert_array_equal(got.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("target,pair,message", [(10, (0, 0), "target"), (-1, (0, 0), "target"),
+                                                 (3, (2, 0), "filter"), (3, (0, 10), "filter"), (3, (-1, 4), "filter"),
+                                                 (3, (1, -1), "filter"), (10, (9, 9), "target")])
+def test_out_of_range(target, pair, message):
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    state = torch.rand(2, 10, device="cuda")
+    with pytest.raises(ValueError, match=message + ".* out of range"):
+        fk.dense_filtered_ranks_cuda(state, torch.tensor([1, target]).cuda(),
+                                     (torch.tensor([pair[0]]).cuda(), torch.tensor([pair[1]]).cuda()))
