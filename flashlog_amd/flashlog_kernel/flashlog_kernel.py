@@ -1375,7 +1375,7 @@ def _same_index_rows(gi, rows):
 
 def _grad_at_outputs(grad, out_indices, L, E):
     """The upstream gradient's values at the hop's output coordinates
-    [3, n] (the role of flashlog_kernel.py:360-376): a dense gradient is
+    [3, n] or [2, n] (the role of flashlog_kernel.py:360-376): a dense gradient is
     indexed; a sparse one with the very index rows of the output is taken
     as is; any other sparse one is coalesced and looked up by fl_sparse_gather
     (0 where it holds no entry)."""
@@ -1389,9 +1389,12 @@ def _grad_at_outputs(grad, out_indices, L, E):
     gv = g.values().float().contiguous()
     q = out_indices.long()
     out = torch.empty(q.shape[1], dtype=torch.float32, device=q.device)
-    check(_lib.lib().fl_sparse_gather(_stream(q), ptr(gi[0].contiguous()), ptr(gi[1].contiguous()),
+    if out_indices.shape[0] == 2:  # [B, E]: one channel
+        gi = (gi[0], torch.zeros_like(gi[0]), gi[1])
+        q = (q[0], torch.zeros_like(q[0]), q[1])
+    check(_lib.lib().fl_sparse_gather(_stream(gv), ptr(gi[0].contiguous()), ptr(gi[1].contiguous()),
                                       ptr(gi[2].contiguous()), ptr(gv), gv.numel(), ptr(q[0].contiguous()),
-                                      ptr(q[1].contiguous()), ptr(q[2].contiguous()), q.shape[1], int(L), int(E),
+                                      ptr(q[1].contiguous()), ptr(q[2].contiguous()), out.numel(), int(L), int(E),
                                       ptr(out)), "sparse_gather")
     return out.to(grad.dtype)
 
@@ -1882,32 +1885,46 @@ def _channel_reduce(sp_batch, sp_level, sp_entity, sp_value, B, L, E, op):
     check(lib.fl_sparse_channel_sum_emit(st, ptr(sb), ptr(se), ptr(v), nnz, B, L, op, ptr(ws), nout,
                                          ptr(idx[0]), ptr(idx[1]), ptr(out), ptr(slot)),
           "sparse_channel_sum_emit")
-    return idx, out, slot.long(), v
+    return idx, out, slot, v
+
+
+def _channel_grad(grad, idx, E):
+    """The gradient at the channel reduction's outputs.  One that itself
+    carries a graph (a second derivative is asked for) is taken through
+    torch's differentiable mask."""
+    if grad.requires_grad and torch.is_grad_enabled():
+        if not grad.is_sparse:
+            return grad[tuple(idx)].float()
+        pattern = torch.sparse_coo_tensor(idx, torch.ones(idx.shape[1], device=idx.device), grad.shape,
+                                          is_coalesced=True)
+        return grad.sparse_mask(pattern).values().float()
+    return _grad_at_outputs(grad, idx, 1, E).float()
 
 
 class Sparse3DChannelSumFunction(autograd.Function):
-    """Values of the channel sum of a coalesced [B, L, E] state: per (b, e)
-    the entries of every channel added from 0 in channel order, as torch's
-    coalesce of the (b, e) re-index adds them (src/model_DRUM_kernel_sp.py:
-    22-28); the gradient of an entry is its output's."""
+    """The channel sum of a coalesced [B, L, E] state, a coalesced [B, E] COO
+    tensor: per (b, e) the entries of every channel added from 0 in channel
+    order, as torch's coalesce of the (b, e) re-index adds them
+    (src/model_DRUM_kernel_sp.py:22-28); the gradient of an entry is its
+    output's.  (The function returns the sparse tensor itself, as the hops do:
+    a tensor built around its values would look every gradient entry up
+    again.)"""
 
     @staticmethod
     def forward(ctx, sp_batch, sp_level, sp_entity, sp_value, B, L, E):
-        idx, out, slot, _ = _channel_reduce(sp_batch, sp_level, sp_entity, sp_value, B, L, E, 0)
-        ctx.slot = slot
-        ctx.mark_non_differentiable(idx)
-        return idx, out
+        idx, out, ctx.slot, _ = _channel_reduce(sp_batch, sp_level, sp_entity, sp_value, B, L, E, 0)
+        ctx.idx, ctx.E = idx, int(E)
+        return torch.sparse_coo_tensor(idx, out, [B, E], is_coalesced=True)
 
     @staticmethod
-    def backward(ctx, grad_idx, grad_out):
-        if grad_out is None:
-            return (None,) * 7
-        return None, None, None, grad_out.contiguous().float()[ctx.slot], None, None, None
+    def backward(ctx, grad_out):
+        g = _channel_grad(grad_out, ctx.idx, ctx.E)
+        return None, None, None, g.index_select(0, ctx.slot), None, None, None
 
 
 class Sparse3DChannelMaxFunction(autograd.Function):
-    """Values of the channel maximum of a coalesced [B, L, E] state
-    (src/model_mmDRUM_kernel_sp.py:17-32, scatter_reduce amax with
+    """The channel maximum of a coalesced [B, L, E] state, a coalesced [B, E]
+    COO tensor (src/model_mmDRUM_kernel_sp.py:17-32, scatter_reduce amax with
     include_self=False).  Backward as torch's for amax: an output's gradient
     is divided evenly among the entries equal to it and, where the maximum
     is 0, the zero the reference reduces into (torch counts that initial
@@ -1917,27 +1934,23 @@ class Sparse3DChannelMaxFunction(autograd.Function):
     def forward(ctx, sp_batch, sp_level, sp_entity, sp_value, B, L, E):
         idx, out, slot, v = _channel_reduce(sp_batch, sp_level, sp_entity, sp_value, B, L, E, 1)
         ctx.save_for_backward(v, out, slot)
-        ctx.mark_non_differentiable(idx)
-        return idx, out
+        ctx.idx, ctx.E = idx, int(E)
+        return torch.sparse_coo_tensor(idx, out, [B, E], is_coalesced=True)
 
     @staticmethod
-    def backward(ctx, grad_idx, grad_out):
-        if grad_out is None:
-            return (None,) * 7
+    def backward(ctx, grad_out):
         v, out, slot = ctx.saved_tensors
-        value = out[slot]
-        is_max = (v == value).to(v.dtype)
-        count = (out == 0).to(out.dtype).scatter_add_(0, slot, is_max)
-        share = grad_out.contiguous().float() / count
-        return None, None, None, is_max * share[slot], None, None, None
+        is_max = (v == out.index_select(0, slot)).to(v.dtype)
+        count = (out == 0).to(out.dtype).scatter_add_(0, slot.long(), is_max)
+        share = _channel_grad(grad_out, ctx.idx, ctx.E) / count
+        return None, None, None, is_max * share.index_select(0, slot), None, None, None
 
 
 def _channel_state(s, fn):
     s = s if s.is_coalesced() else s.coalesce()
     B, L, E = s.shape
     idx = s.indices()
-    out_idx, out_val = fn.apply(idx[0], idx[1], idx[2], s.values(), B, L, E)
-    return torch.sparse_coo_tensor(out_idx, out_val, [B, E], is_coalesced=True)
+    return fn.apply(idx[0], idx[1], idx[2], s.values(), B, L, E)
 
 
 def sum_sp_3d(s):
