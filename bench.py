@@ -769,7 +769,7 @@ def main_grounding(args):
         cands, raw, _ = call()
     torch.cuda.synchronize()
     el = (time.perf_counter() - t0) / reps
-    kn = ["k_gr_hubs", "k_gr_walk", "k_ct_flags", "k_ct_accum", "k_ct_capkey", "k_ct_keep", "k_ct_gather", "k_ct_emit"]
+    kn = ["k_gr_kinds", "k_gr_small", "k_gr_hubs", "k_gr_lanes", "k_gr_walk", "k_ct_flags", "k_ct_accum", "k_ct_capkey", "k_ct_keep", "k_ct_gather", "k_ct_emit"]
     prof = {k: _lib.prof_read(k) for k in kn}
     _lib.prof_enable(False)
     per_call = {k: v[0] / reps for k, v in prof.items()}
@@ -872,15 +872,21 @@ def main_rules(args):
         run()
     torch.cuda.synchronize()
     el = (time.perf_counter() - t0) / reps
-    # kernel times (HIP events around each launch) and the steps' sizes, one more pass
+    # kernel times (HIP events around each launch), one more pass
     _lib.prof_enable(True)
+    run()
+    torch.cuda.synchronize()
+    prof = {k: _lib.prof_read(k) for k in RULE_STEP_KERNELS + RULE_ACC_KERNELS}
+    _lib.prof_enable(False)
+    # the steps' sizes, from a pass that grounds step by step
+    whole = si._grounds_in_one_launch
+    si._grounds_in_one_launch = lambda *a: False
     fk.plan_log = []
     run()
     torch.cuda.synchronize()
     plans = fk.plan_log
     fk.plan_log = None
-    prof = {k: _lib.prof_read(k) for k in RULE_STEP_KERNELS + RULE_ACC_KERNELS}
-    _lib.prof_enable(False)
+    si._grounds_in_one_launch = whole
     per_pass = {k: v[0] for k, v in prof.items()}
     step_ms = sum(per_pass[k] for k in RULE_STEP_KERNELS)
     step_bytes = float(sum(rule_step_bytes(p) for p in plans))
@@ -913,7 +919,7 @@ def main_rules(args):
                                "queries, %d heads, chunks of %d rules" % (NR, RANKS, NQ, len(groups), CHUNK)},
         "kernel_ms_per_pass": per_pass,
         "kernel_ms_total": sum(per_pass.values()),
-        "roofline": {"kernel": "fixed-relation rule steps (their kernels, per pass)", "bound": "hbm",
+        "roofline": {"kernel": "rule grounding (k_rg_rows and k_rg_dense, per pass)", "bound": "hbm",
                      "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "algorithmic_bytes_per_launch": step_bytes, "ms_per_launch": step_ms, "traffic": None,
                      "steps_per_pass": len(plans)},
@@ -923,14 +929,11 @@ def main_rules(args):
     print(json.dumps(result), flush=True)
 
 
-# The fixed-relation rule step's kernels (the sparse pipeline's mode 2) and the
-# rule bank's accumulation kernels.
-RULE_STEP_KERNELS = ["k_fx_count", "k_fx_fill", "k_sp_rowptr", "k_sp_rowinfo", "k_sp_hist", "k_sp_vscan",
-                     "k_sp_partition", "k_sp_accum_small", "k_sp_accum_few", "k_sp_accum_mid", "k_sp_accum_hot",
-                     "k_sp_emit", "k_scan_tiles", "k_scan_totals", "k_scan_apply", "k_scan_one", "k_fill_i32",
-                     "k_fill_i64", "k_sp_plan_out"]
-RULE_ACC_KERNELS = ["k_ra_rows", "k_ra_sum", "k_cs_rank", "k_cs_weighted_add", "k_rule_accum_max", "k_rule_rowsum",
-                    "k_rule_combine"]
+# The kernels that ground a chunk of rules, and those that accumulate the rules'
+# masses and collect the scored entities.
+RULE_STEP_KERNELS = ["k_rg_zero", "k_rg_rows", "k_rg_dense"]
+RULE_ACC_KERNELS = ["k_rg_sum", "k_rg_status", "k_rule_combine", "k_rule_count", "k_rule_info", "k_rule_fill",
+                    "k_scan_tiles", "k_scan_totals", "k_scan_apply", "k_scan_one"]
 
 
 def rule_step_bytes(plan):
@@ -946,21 +949,21 @@ def rule_step_bytes(plan):
     return 28 * nnz + 8 * rows + nnz * (16 + 2 * lg) + 4 * items + 28 * nout
 
 
-SPARSE_KERNELS = ["k_sp_topc", "k_race_flags", "k_race_keys", "k_race_rows", "k_race_select", "k_fill_from",
-                  "k_sp_rowptr", "k_sp_relorder", "k_sp_select", "k_sp_rowinfo", "k_sp_runs", "k_sp_items",
+SPARSE_KERNELS = ["k_sp_topc", "k_race_flags", "k_race_keys", "k_race_rows", "k_race_select", "k_race_info",
+                  "k_sp_plan_zero", "k_sp_prep", "k_sp_plan_one", "k_sp_rowptr", "k_sp_relorder", "k_sp_select", "k_sp_rowinfo", "k_sp_runs", "k_sp_items",
                   "k_sp_expand_fused",
                   "k_sp_hist",
                   "k_sp_partition", "k_sp_accum_small", "k_sp_accum_few", "k_sp_accum_mid", "k_sp_accum_hot", "k_sp_emit", "k_sp_local_to_out",
                   "k_norm_fwd", "k_norm_bwd", "k_sp_bwd", "k_fill_f32", "k_scan_tiles", "k_scan_totals",
                   "k_scan_apply", "k_scan_one", "k_sp_vscan", "k_fill_i32", "k_fill_i64", "k_sp_plan_out", "k_apply_mask",
-                  "k_sp_ord_count", "k_sp_ord_place", "k_sp_rowptr_search", "k_sp_order_count", "k_sp_order_check", "k_sp_gather_nch",
-                  "k_sp_finite", "k_sp_bw_chunks", "k_sp_gw_fin",
+                  "k_sp_ord_count", "k_sp_ord_place", "k_sp_order_count", "k_sp_order_check", "k_sp_gather_nch",
+                  "k_sp_bw_chunks", "k_sp_gw_fin",
                   "k_cs_rank", "k_cs_emit", "k_pack_bool_bits", "k_order_bits"]
 
 
 # The sparse hop's own kernels (forward and backward), without the c1 entity
 # selection, the normalizer and the channel sums that surround it in a step.
-HOP_EXCLUDE = ("k_sp_topc", "k_race_flags", "k_race_keys", "k_race_rows", "k_race_select", "k_fill_from",
+HOP_EXCLUDE = ("k_sp_topc", "k_race_flags", "k_race_keys", "k_race_rows", "k_race_select", "k_race_info",
                "k_norm_fwd", "k_norm_bwd", "k_cs_rank", "k_cs_emit")
 HOP_KERNELS = [k for k in SPARSE_KERNELS if k not in HOP_EXCLUDE]
 

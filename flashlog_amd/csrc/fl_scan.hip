@@ -1,6 +1,7 @@
 // Device-wide exclusive prefix sum (int32 or int64 input, int64 output) in
-// three launches: per-tile totals, a scan of the tile totals by one
-// workgroup, and the per-tile scan with its offset.  Used for the count ->
+// two launches, per-tile totals and the per-tile scan, whose workgroups add
+// the totals before their own tile themselves; beyond SC_SELF_TILES tiles a
+// scan of the totals by one workgroup goes between them.  Used for the count ->
 // offset steps of the sparse hop (entry item offsets, bucket bases, output
 // offsets).  out may alias in for int64 input.
 #include "fl_common.h"
@@ -60,10 +61,22 @@ __global__ __launch_bounds__(SC_NT) void k_scan_totals(int64_t *__restrict__ til
     if (threadIdx.x == 0) tile_sum[ntiles] = carry;
 }
 
-template <typename T>
+// SELF: tile_sum holds the tiles' totals, not their scan.  (96,000 counts: 14
+// us by three launches, the one in the middle of a single workgroup; 12 by two.)
+constexpr int64_t SC_SELF_TILES = 4096;
+
+template <typename T, bool SELF>
 __global__ __launch_bounds__(SC_NT) void k_scan_apply(const T *in, int64_t n, const int64_t *__restrict__ tile_sum,
                                                      int64_t *out) {
     __shared__ long long wsum[SC_NT / FL_WAVE];
+    __shared__ long long wbefore[SC_NT / FL_WAVE];
+    long long before = 0;
+    if (SELF) {
+        long long x = 0;
+        for (int64_t k = threadIdx.x; k < (int64_t)blockIdx.x; k += SC_NT) x += tile_sum[k];
+        x = fl_wave_sum_i64(x);
+        if (fl_lane() == 0) wbefore[threadIdx.x / FL_WAVE] = x;
+    }
     const int64_t base = (int64_t)blockIdx.x * SC_TILE;
     // blocked: thread t owns elements [base + t*IPT, +IPT)
     long long v[SC_IPT];
@@ -77,7 +90,10 @@ __global__ __launch_bounds__(SC_NT) void k_scan_apply(const T *in, int64_t n, co
     const long long incl = fl_wave_incl_scan_i64(s);
     if (fl_lane() == FL_WAVE - 1) wsum[threadIdx.x / FL_WAVE] = incl;
     __syncthreads();
-    long long run = tile_sum[blockIdx.x];
+    if (SELF)
+        for (int k = 0; k < SC_NT / FL_WAVE; ++k) before += wbefore[k];
+    else before = tile_sum[blockIdx.x];
+    long long run = before;
     for (int k = 0; k < (int)(threadIdx.x / FL_WAVE); ++k) run += wsum[k];
     run += incl - s;
 #pragma unroll
@@ -86,7 +102,8 @@ __global__ __launch_bounds__(SC_NT) void k_scan_apply(const T *in, int64_t n, co
         if (i < n) out[i] = run;
         run += v[j];
     }
-    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = tile_sum[gridDim.x];
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0)
+        out[n] = SELF ? before + tile_sum[blockIdx.x] : tile_sum[gridDim.x];
 }
 
 // One workgroup for at most one tile (n <= SC_TILE): every element read
@@ -137,8 +154,12 @@ static int scan_impl(hipStream_t st, const T *in, int64_t *out, int64_t n, int64
     }
     const int64_t nt = (n + SC_TILE - 1) / SC_TILE;
     FL_LAUNCH("k_scan_tiles", k_scan_tiles<T>, dim3((unsigned)nt), dim3(SC_NT), 0, st, in, n, tmp);
+    if (nt <= SC_SELF_TILES) {
+        FL_LAUNCH("k_scan_apply", (k_scan_apply<T, true>), dim3((unsigned)nt), dim3(SC_NT), 0, st, in, n, tmp, out);
+        return fl_check_launch("exclusive_scan");
+    }
     FL_LAUNCH("k_scan_totals", k_scan_totals, dim3(1), dim3(SC_NT), 0, st, tmp, nt);
-    FL_LAUNCH("k_scan_apply", k_scan_apply<T>, dim3((unsigned)nt), dim3(SC_NT), 0, st, in, n, tmp, out);
+    FL_LAUNCH("k_scan_apply", (k_scan_apply<T, false>), dim3((unsigned)nt), dim3(SC_NT), 0, st, in, n, tmp, out);
     return fl_check_launch("exclusive_scan");
 }
 

@@ -11,11 +11,12 @@
 // then to the smaller original edge id, then to the earlier raw item.
 //
 // Pipeline (rows r = b*L + l; entries must be sorted by row):
-//   plan    k_sp_rowptr   entry range of every row, input validation
+//   plan    k_sp_prep     entry range of every row, input validation
 //           k_sp_select   per (entry, side): c2 threshold and cut (training:
 //                         quota parameters), item counts and 64-item chunks
 //           scan          item and chunk offsets of every entry (raw order)
 //           k_sp_rowinfo  item range and tile count of every row; scan
+//                         (k_sp_plan_one: all of these for a small state)
 //   expand  k_sp_runs     wave per entry: one descriptor per run (the kept
 //                         edges of one group) and the entry's chunk records
 //           k_sp_items    wave per 64 raw items: destination and value of
@@ -86,6 +87,60 @@ constexpr uint32_t SP_TIE_IDENTITY = 0xFFFFFFFFu;
 
 // ---------------------------------------------------------------------------
 // plan
+
+// First entry of row r (or a later row) for r in [0, R], by binary search
+// over the row keys b*L + l of entries sorted by row, without checking the
+// order: every value stays in [0, nnz], so kernels bounded by it stay in
+// range on any input.  The first row starts at entry 0 and the last ends at
+// nnz whatever the keys hold: the search result is monotone in r even over
+// unsorted keys, so every entry lies in exactly one row's range (keys outside
+// [0, R) or out of order give unspecified ranges, never gaps).
+__device__ __forceinline__ int64_t sp_row_start(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl,
+                                                int64_t nnz, int64_t L, int64_t R, int64_t r) {
+    if (r == 0) return 0;
+    if (r >= R) return nnz;
+    int64_t lo = 0, hi = nnz;
+    while (lo < hi) {
+        const int64_t mid = (lo + hi) >> 1;
+        if (sb[mid] * L + sl[mid] < r) lo = mid + 1;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// The plan's first pass (its words and scratch counters cleared by
+// k_sp_plan_zero): row starts by search, every entry's range and row order
+// checked (err: 1 an index out of range, 2 rows not sorted), and whether an
+// attention weight is not finite.  Thread i takes row i, entry i and, with
+// the grid's stride, weights.
+__global__ __launch_bounds__(256) void k_sp_prep(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl,
+                                                const int64_t *__restrict__ se, int64_t nnz, int64_t B, int64_t L,
+                                                int64_t E, const float *__restrict__ w, int64_t wcount,
+                                                int64_t *__restrict__ row_ptr, int64_t *__restrict__ plan) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t R = B * L;
+    if (i <= R) row_ptr[i] = sp_row_start(sb, sl, nnz, L, R, i);
+    if (i < nnz) {
+        const int64_t b = sb[i], l = sl[i], e = se[i];
+        if (b < 0 || b >= B || l < 0 || l >= L || e < 0 || e >= E) {
+            atomicMax((unsigned long long *)(plan + 2), 1ull);
+        } else if (i > 0) {
+            const int64_t pb = sb[i - 1], pl = sl[i - 1];
+            if (pb >= 0 && pb < B && pl >= 0 && pl < L && pb * L + pl > b * L + l)
+                atomicMax((unsigned long long *)(plan + 2), 2ull);
+        }
+    }
+    bool bad = false;
+    for (int64_t q = i; q < wcount; q += (int64_t)gridDim.x * blockDim.x) bad |= !isfinite(w[q]);
+    if (__ballot(bad) != 0 && fl_lane() == 0) atomicOr((unsigned long long *)(plan + 5), 1ull);
+}
+
+// The plan's words and the order check's counters cleared by one launch.
+__global__ void k_sp_plan_zero(int64_t *__restrict__ plan, int32_t *__restrict__ seen, int64_t nseen) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < 6) plan[i] = 0;
+    if (i < nseen) seen[i] = 0;
+}
 
 // row_ptr[r] = first entry of row r (entries sorted by row); err[0] gets a
 // nonzero code for a malformed input (1: index out of range, 2: rows not
@@ -614,7 +669,7 @@ __global__ __launch_bounds__(SEL_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) 
             th[2 * i] = th[2 * i + 1] = 0.0f;
             cut[2 * i] = cut[2 * i + 1] = 0;
         }
-        return;  // reported by k_sp_rowptr; the plan is not used
+        return;  // reported by k_sp_prep; the plan is not used
     }
     const float *wrow = w + (sb[i] * L + sl[i]) * n;
     int total = wot_i ? 0 : 1;
@@ -3029,18 +3084,95 @@ __global__ void k_fill_i32(int32_t *__restrict__ p, int64_t n, int32_t v) {
     if (i < n) p[i] = v;
 }
 
-__global__ void k_fill_i64(int64_t *__restrict__ p, int64_t n, int64_t v) {
+// p[0, n) = v, and a second range q[0, m) = v where a caller has one
+__global__ void k_fill_i64(int64_t *__restrict__ p, int64_t n, int64_t v, int64_t *__restrict__ q, int64_t m) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < n) p[i] = v;
+    else if (i - n < m) q[i - n] = v;
 }
 
-// plan[5] = 1 when an attention weight is not finite (any lane of a wave
-// that sees one sets it).
-__global__ void k_sp_finite(const float *__restrict__ w, int64_t count, unsigned long long *__restrict__ flag) {
-    bool bad = false;
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count; i += (int64_t)gridDim.x * blockDim.x)
-        bad |= !isfinite(w[i]);
-    if (__ballot(bad) != 0 && fl_lane() == 0) atomicOr(flag, 1ull);
+// What follows the item counts of a plan, for hops of at most SP_ONE_MAX
+// entries and rows by one workgroup instead of nine launches: the items' and
+// chunks' offsets, the rows' first items and tiles, the plan's words.  nch may
+// be null (the fixed-relation step); chunk counts are taken in visiting order.
+constexpr int SP_ONE_NT = 1024;  // (also k_sp_bw_chunks_one: the rows' chunk counts and their offsets)
+constexpr int SP_ONE_PER = 4;
+constexpr int64_t SP_ONE_MAX = SP_ONE_NT * SP_ONE_PER;
+
+template <typename Get, typename Put>
+__device__ __forceinline__ int64_t sp_one_scan(int64_t n, long long *w64, Get get, Put put) {
+    // exclusive prefix sums of get(i), i < n (their total fits 32 bits or the
+    // hop does not take this path)
+    const int t = threadIdx.x;
+    int64_t x[SP_ONE_PER], sum = 0;
+#pragma unroll
+    for (int j = 0; j < SP_ONE_PER; ++j) {
+        const int64_t i = (int64_t)t * SP_ONE_PER + j;
+        x[j] = i < n ? get(i) : 0;
+        sum += x[j];
+    }
+    const long long incl = fl_wave_incl_scan_i64(sum);
+    __syncthreads();
+    if (fl_lane() == FL_WAVE - 1) w64[t / FL_WAVE] = incl;
+    __syncthreads();
+    long long run = incl - sum, total = 0;
+    for (int k = 0; k < SP_ONE_NT / FL_WAVE; ++k) {
+        if (k < t / FL_WAVE) run += w64[k];
+        total += w64[k];
+    }
+#pragma unroll
+    for (int j = 0; j < SP_ONE_PER; ++j) {
+        const int64_t i = (int64_t)t * SP_ONE_PER + j;
+        if (i < n) put(i, run);
+        run += x[j];
+    }
+    if (t == 0) put(n, total);
+    __syncthreads();  // (also: the offsets are visible to the workgroup)
+    return total;
+}
+
+__global__ __launch_bounds__(SP_ONE_NT) void k_sp_bw_chunks_one(const int64_t *__restrict__ row_ptr, int64_t R,
+                                                               int64_t *__restrict__ chunk_ptr) {
+    __shared__ long long lds[SP_ONE_NT / FL_WAVE];
+    sp_one_scan(R, lds, [&](int64_t r) { return (row_ptr[r + 1] - row_ptr[r] + BW_CH - 1) / BW_CH; },
+                [&](int64_t r, int64_t x) { chunk_ptr[r] = x; });
+}
+
+__global__ __launch_bounds__(SP_ONE_NT) void k_sp_plan_one(const int32_t *__restrict__ cnt,
+                                                          const int32_t *__restrict__ nch,
+                                                          const int32_t *__restrict__ order, int64_t nnz, int64_t E,
+                                                          int64_t R, const int64_t *__restrict__ row_ptr,
+                                                          int64_t *item_off, int64_t *chunk_off, int64_t *row_item0,
+                                                          int32_t *ntiles, int64_t *tile_base,
+                                                          int64_t *__restrict__ plan) {
+    __shared__ long long lds[SP_ONE_NT / FL_WAVE];
+    const int64_t items = sp_one_scan(nnz, lds, [&](int64_t i) { return (int64_t)cnt[i]; },
+                                      [&](int64_t i, int64_t x) { item_off[i] = x; });
+    int64_t chunks = 0;
+    if (nch)
+        chunks = sp_one_scan(nnz, lds,
+                             [&](int64_t i) {
+                                 const int32_t o = order ? order[i] : (int32_t)i;
+                                 return (int64_t)((o >= 0 && o < nnz) ? nch[o] : 0);
+                             },
+                             [&](int64_t i, int64_t x) { chunk_off[i] = x; });
+    const volatile int64_t *off = item_off;  // written above by other threads of the workgroup
+    const int64_t tiles = sp_one_scan(R, lds,
+                                      [&](int64_t r) {
+                                          const int64_t a = off[row_ptr[r]], b = off[row_ptr[r + 1]];
+                                          row_item0[r] = a;
+                                          const int64_t k = (b - a + SP_TILE - 1) / SP_TILE;
+                                          ntiles[r] = (int32_t)k;
+                                          return k;
+                                      },
+                                      [&](int64_t r, int64_t x) { tile_base[r] = x; });
+    if (threadIdx.x == 0) {
+        row_item0[R] = off[row_ptr[R]];
+        plan[0] = items;
+        plan[1] = tiles;
+        plan[3] = sp_buckets_of(E, sp_shift(E, R, items));
+        plan[4] = chunks;
+    }
 }
 
 __global__ void k_sp_plan_out(const int64_t *__restrict__ items, const int64_t *__restrict__ tiles, int64_t E,
@@ -3051,7 +3183,11 @@ __global__ void k_sp_plan_out(const int64_t *__restrict__ items, const int64_t *
     plan[4] = chunks ? *chunks : 0;
 }
 
-__global__ void k_fill_from(const int64_t *__restrict__ src, int64_t *__restrict__ dst) { *dst = *src; }
+__global__ void k_race_info(const int64_t *__restrict__ cand, const int64_t *__restrict__ kept,
+                            int64_t *__restrict__ info) {
+    info[0] = *cand;
+    info[2] = kept ? *kept : 0;
+}
 
 __global__ void k_fill_f32(float *__restrict__ p, int64_t n, float v) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -3319,52 +3455,87 @@ __device__ __forceinline__ float block_tree_sum(float v, float *red) {
     return s;
 }
 
-// row_ptr[r] for r in [0, R] by binary search over the row keys b*L + l of
-// entries sorted by row (the first entry of row r or later), without
-// checking the order: every value stays in [0, nnz], so kernels bounded by
-// it stay in range on any input.
-__global__ void k_sp_rowptr_search(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl, int64_t nnz,
-                                   int64_t L, int64_t R, int64_t *__restrict__ row_ptr) {
-    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r > R) return;
-    int64_t lo = 0, hi = nnz;
-    while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (sb[mid] * L + sl[mid] < r) lo = mid + 1;
-        else hi = mid;
-    }
-    // The first row starts at entry 0 and the last ends at nnz whatever the
-    // keys hold: the search result is monotone in r even over unsorted keys,
-    // so every entry then lies in exactly one row's range and every output
-    // is written (keys outside [0, R) or out of order give unspecified
-    // values, never unwritten ones).
-    row_ptr[r] = r == 0 ? 0 : (r == R ? nnz : lo);
-}
-
 // Per row (workgroup): the denominator is a left fold from 0 over the row's
 // values in entry (= output key) order, as the CPU path adds them
-// (flashlog.cpp:1561-1565); the workgroup stages chunks of the row in LDS
-// (double-buffered) while its first thread folds the previous chunk.  The
-// clamp is the GPU path's (flashlog.cu:2540): d >= eps ? d : eps, so a NaN
-// sum divides by eps.
+// (flashlog.cpp:1561-1565).  The clamp is the GPU path's (flashlog.cu:2540):
+// d >= eps ? d : eps, so a NaN sum divides by eps.
+//   The chain of dependent adds bounds it.  The first wave does nothing else:
+// its first thread adds chunk c from LDS, the next 32 values on their way
+// while 32 are added, and the other waves bring in chunk c + 1 meanwhile.
+// The row's range is searched by the workgroup itself (row_ptr is kept for
+// the backward), so that the normalizer is one launch.
+//   Rows of 14,000 values: 87 us; with the chunk loaded by all
+// waves and each LDS round trip waited for 98 us.  Composing the adds of a
+// binade as maps of the mantissa's parity, in parallel, took as long (95 us).
 constexpr int NF_CHUNK = 2048;
 
-__global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ row_ptr,
-                                                   const float *__restrict__ v, float eps, float *__restrict__ out,
-                                                   float *__restrict__ denom) {
+// sv[0 .. n) added to a, left to right; sv is 16-byte aligned.
+__device__ __forceinline__ float nf_fold(float a, const float *sv, int n) {
+    constexpr int U = 8;  // float4s on their way
+    const float4 *v4 = reinterpret_cast<const float4 *>(sv);
+    const int groups = n / (4 * U);
+    float4 x[U], y[U];
+    auto get = [&](float4 *d, int g) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) d[u] = v4[g * U + u];
+    };
+    auto add = [&](const float4 *d) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            a = fl_add(a, d[u].x);
+            a = fl_add(a, d[u].y);
+            a = fl_add(a, d[u].z);
+            a = fl_add(a, d[u].w);
+        }
+    };
+    int g = 0;
+    if (groups > 0) get(x, 0);
+    for (; g + 2 <= groups; g += 2) {
+        get(y, g + 1);
+        add(x);
+        get(x, min(g + 2, groups - 1));
+        add(y);
+    }
+    if (g < groups) add(x);
+    return sp_fold(a, sv, groups * 4 * U, n);
+}
+
+__global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl,
+                                                   int64_t nnz, int64_t L, int64_t R, const float *__restrict__ v,
+                                                   float eps, float *__restrict__ out, float *__restrict__ denom,
+                                                   int64_t *__restrict__ row_ptr, int64_t *__restrict__ err) {
     __shared__ float4 buf[2][NF_CHUNK / 4];
     __shared__ float dsh;
+    __shared__ int64_t range[2];
     const int64_t r = blockIdx.x;
-    const int64_t a = row_ptr[r], b = row_ptr[r + 1];
     const int t = threadIdx.x;
+    if (t < 2) {
+        const int64_t p = sp_row_start(sb, sl, nnz, L, R, r + t);
+        range[t] = p;
+        if (t == 0 || r == R - 1) row_ptr[r + t] = p;
+    }
+    if (r == 0 && t == 0) *err = 0;
+    __syncthreads();
+    const int64_t a = range[0], b = range[1];
+    {
+        const int len = (int)((b - a) < NF_CHUNK ? (b - a) : NF_CHUNK);
+        float *cb = (float *)buf[0];
+        for (int i = t; i < len; i += NM_NT) cb[i] = v[a + i];
+    }
+    __syncthreads();
     float acc = 0.0f;
     int c = 0;
     for (int64_t base = a; base < b; base += NF_CHUNK, ++c) {
-        const int len = (int)((b - base) < NF_CHUNK ? (b - base) : NF_CHUNK);
-        float *cb = (float *)buf[c & 1];
-        for (int i = t; i < len; i += NM_NT) cb[i] = v[base + i];
+        if (t >= FL_WAVE) {
+            const int64_t left = b - base - NF_CHUNK;
+            const int len = (int)(left < NF_CHUNK ? left : NF_CHUNK);  // (<= 0 behind the last chunk)
+            float *cb = (float *)buf[(c + 1) & 1];
+#pragma unroll 4
+            for (int i = t - FL_WAVE; i < len; i += NM_NT - FL_WAVE) cb[i] = v[base + NF_CHUNK + i];
+        } else if (t == 0) {
+            acc = nf_fold(acc, (const float *)buf[c & 1], (int)((b - base) < NF_CHUNK ? (b - base) : NF_CHUNK));
+        }
         __syncthreads();
-        if (t == 0) acc = sp_fold(acc, cb, 0, len);  // 32 values per LDS round trip
     }
     if (t == 0) {
         dsh = acc;
@@ -3373,6 +3544,7 @@ __global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ 
     __syncthreads();
     const float d = dsh;
     const float dc = d >= eps ? d : eps;
+#pragma unroll 4
     for (int64_t k = a + t; k < b; k += NM_NT) out[k] = __fdiv_rn(v[k], dc);
 }
 
@@ -3497,11 +3669,12 @@ SpExp sp_exp_layout(int64_t T, int64_t tiles, int64_t chunks, int64_t R, int64_t
     auto take = [&](size_t b) { char *q = base ? base + off : nullptr; off += al(b); return q; };
     const int64_t T1 = T > 0 ? T : 1;
     const int64_t U1 = chunks > 0 ? chunks : 1;
-    // run table (at most one run per item) and chunk table
-    x.runs.first = (int32_t *)take(sizeof(int32_t) * (size_t)T1);
-    x.runs.p = (int32_t *)take(sizeof(int32_t) * (size_t)T1);
-    x.runs.aw = (float *)take(sizeof(float) * (size_t)T1);
-    x.runs.meta = (uint32_t *)take(sizeof(uint32_t) * (size_t)T1);
+    // run table (at most one run per item) and chunk table, where the hop has chunks
+    const int64_t TR = chunks > 0 ? T1 : 1;
+    x.runs.first = (int32_t *)take(sizeof(int32_t) * (size_t)TR);
+    x.runs.p = (int32_t *)take(sizeof(int32_t) * (size_t)TR);
+    x.runs.aw = (float *)take(sizeof(float) * (size_t)TR);
+    x.runs.meta = (uint32_t *)take(sizeof(uint32_t) * (size_t)TR);
     x.runs.c_base = (int64_t *)take(sizeof(int64_t) * (size_t)U1);
     x.runs.c_run = (int64_t *)take(sizeof(int64_t) * (size_t)U1);
     x.runs.c_rlim = (int64_t *)take(sizeof(int64_t) * (size_t)U1);
@@ -3697,6 +3870,10 @@ size_t fl_sparse_plan_bytes(int64_t nnz, int64_t R, int64_t r_size) {
 }
 
 static int64_t sp_budget(const fl_sparse_hop *h);
+// Hops whose runs stay in LDS (k_sp_expand_fused): no run table, no chunks.
+static bool sp_fused(const fl_sparse_hop *h) {
+    return h->mode != SP_FIXED && sp_budget(h) > 0 && sp_budget(h) <= SP_FUSE_KMAX && h->n <= (int64_t)SP_LR_COL + 1;
+}
 // relations per side of the hop's attention (0 for the fixed-relation step)
 static int64_t sp_rsize(const fl_sparse_hop *h) { return h->mode == SP_FIXED ? 0 : h->r_size; }
 // Training quotas can apply (sampling seed, top-k mode, a positive budget).
@@ -3723,21 +3900,15 @@ int fl_sparse_plan(void *stream, const fl_side *ori, const fl_side *inv, const f
     const int64_t K = sp_budget(h);
     // plan[0] items, plan[1] tiles, plan[2] error, plan[3] buckets per row, plan[4] item chunks,
     // plan[5] non-finite attention
-    FL_LAUNCH("k_fill_i32", k_fill_i32, dim3(1), dim3(64), 0, st, (int32_t *)plan, (int64_t)12, 0);
-    if (h->mode != SP_FIXED && h->w && R * h->n > 0) {
-        const int64_t cnt = R * h->n;
-        const int64_t blocks = (cnt + 255) / 256 < 1024 ? (cnt + 255) / 256 : 1024;
-        FL_LAUNCH("k_sp_finite", k_sp_finite, dim3((unsigned)blocks), dim3(256), 0, st, h->w, cnt,
-                  (unsigned long long *)(plan + 5));
-    }
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3((unsigned)((R + 1 + 255) / 256)), dim3(256), 0, st, p.row_ptr, R + 1,
-              (int64_t)0);
+    const bool ordered = h->entry_order && nnz > 0 && h->mode != SP_FIXED;
+    const int64_t nseen = ordered ? nnz : 0;
+    FL_LAUNCH("k_sp_plan_zero", k_sp_plan_zero, dim3((unsigned)(nseen / 256 + 1)), dim3(256), 0, st, plan, p.nch_ord,
+              nseen);
     const int64_t g1 = (nnz > R + 1 ? nnz : R + 1);
-    FL_LAUNCH("k_sp_rowptr", k_sp_rowptr, dim3((unsigned)((g1 + 255) / 256)), dim3(256), 0, st, h->sp_b, h->sp_l,
-              h->sp_e, nnz, h->B, h->L, h->E, p.row_ptr, plan + 2);
-    if (h->entry_order && nnz > 0 && h->mode != SP_FIXED) {
+    FL_LAUNCH("k_sp_prep", k_sp_prep, dim3((unsigned)((g1 + 255) / 256)), dim3(256), 0, st, h->sp_b, h->sp_l, h->sp_e,
+              nnz, h->B, h->L, h->E, h->w, h->mode != SP_FIXED && h->w ? R * h->n : (int64_t)0, p.row_ptr, plan);
+    if (ordered) {
         // the order must visit every entry once (nch_ord is the count scratch here)
-        FL_LAUNCH("k_fill_i32", k_fill_i32, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, st, p.nch_ord, nnz, 0);
         FL_LAUNCH("k_sp_order_count", k_sp_order_count, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, st,
                   h->entry_order, nnz, p.nch_ord, plan + 2);
         FL_LAUNCH("k_sp_order_check", k_sp_order_check, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, st,
@@ -3760,20 +3931,26 @@ int fl_sparse_plan(void *stream, const fl_side *ori, const fl_side *inv, const f
                   lookup ? p.rel_order : (const int16_t *)nullptr, lookup ? p.rel_nelig : (const int32_t *)nullptr,
                   use_map, p.quota, p.nch, h->entry_order);
     }
+    const bool chunked = h->mode != SP_FIXED && !sp_fused(h);
+    if (nnz <= SP_ONE_MAX && R <= SP_ONE_MAX) {
+        FL_LAUNCH("k_sp_plan_one", k_sp_plan_one, dim3(1), dim3(SP_ONE_NT), 0, st, p.cnt,
+                  chunked ? p.nch : (const int32_t *)nullptr, ordered ? h->entry_order : (const int32_t *)nullptr, nnz,
+                  h->E, R, p.row_ptr, p.item_off, p.chunk_off, p.row_item0, p.ntiles, p.tile_base, plan);
+        return fl_check_launch("sparse_plan");
+    }
     if ((rc = exclusive_scan(st, p.cnt, p.item_off, nnz, p.tmp)) != FL_OK) return rc;
-    const bool fixed = h->mode == SP_FIXED;
-    if (!fixed && h->entry_order && nnz > 0) {
+    if (chunked && h->entry_order && nnz > 0) {
         FL_LAUNCH("k_sp_gather_nch", k_sp_gather_nch, dim3((unsigned)((nnz + 255) / 256)), dim3(256), 0, st, p.nch,
                   h->entry_order, nnz, p.nch_ord);
         if ((rc = exclusive_scan(st, p.nch_ord, p.chunk_off, nnz, p.tmp)) != FL_OK) return rc;
-    } else if (!fixed && (rc = exclusive_scan(st, p.nch, p.chunk_off, nnz, p.tmp)) != FL_OK) {
+    } else if (chunked && (rc = exclusive_scan(st, p.nch, p.chunk_off, nnz, p.tmp)) != FL_OK) {
         return rc;
     }
     FL_LAUNCH("k_sp_rowinfo", k_sp_rowinfo, dim3((unsigned)((R + 1 + 255) / 256)), dim3(256), 0, st, p.row_ptr,
               p.item_off, R, p.row_item0, p.ntiles);
     if ((rc = exclusive_scan(st, p.ntiles, p.tile_base, R, p.tmp)) != FL_OK) return rc;
     FL_LAUNCH("k_sp_plan_out", k_sp_plan_out, dim3(1), dim3(1), 0, st, p.item_off + nnz, p.tile_base + R,
-              h->E, R, fixed ? (const int64_t *)nullptr : p.chunk_off + nnz, plan);
+              h->E, R, chunked ? p.chunk_off + nnz : (const int64_t *)nullptr, plan);
     return fl_check_launch("sparse_plan");
 }
 
@@ -3821,8 +3998,7 @@ int fl_sparse_expand(void *stream, const fl_side *ori, const fl_side *inv, const
     if (nnz > 0 && h->mode == SP_FIXED)
         FL_LAUNCH("k_fx_fill", k_fx_fill, dim3((unsigned)((nnz + SEL_NT / FL_WAVE - 1) / (SEL_NT / FL_WAVE))),
                   dim3(SEL_NT), 0, st, *ori, *inv, h->sp_e, h->sp_v, nnz, p.cut, p.item_off, x.raw_dst, x.raw_val);
-    else if (nnz > 0 && h->items > 0 && sp_budget(h) > 0 && sp_budget(h) <= SP_FUSE_KMAX &&
-             h->n <= (int64_t)SP_LR_COL + 1) {
+    else if (nnz > 0 && h->items > 0 && sp_fused(h)) {
         // budgeted hop: at most 2K+1 items (and runs) per entry, kept in LDS
         const int holes = h->mode == SP_TOPK && h->aggregate == SP_SUM;
         const int rcap = (int)(2 * sp_budget(h) + 2);
@@ -3920,14 +4096,21 @@ int fl_sparse_expand(void *stream, const fl_side *ori, const fl_side *inv, const
                   dst_arr, val_arr, acc_local, x.out_count, nslot, x.hot_list, x.mid_list, x.mid_fb, x.hot_count);
         // buckets of more than SP_WB items: few destinations here, the rest
         // on the fallback lists
-        FL_LAUNCH("k_sp_accum_few", k_sp_accum_few, dim3((unsigned)mid_g),
-                  dim3(SP_NT), 0, st, rows, x.base, dst_arr, val_arr, acc_local, x.out_count, x.hot_list,
-                  x.mid_list, x.hot_fb, x.mid_fb, x.hot_count);
-        FL_LAUNCH("k_sp_accum_mid", k_sp_accum_mid, dim3((unsigned)mid_g),
-                  dim3(SP_NT), 0, st, rows, x.base, dst_arr, val_arr, acc_local, x.out_count, x.mid_fb,
-                  x.hot_count + 6);
-        FL_LAUNCH("k_sp_accum_hot", k_sp_accum_hot, dim3(hot_grid), dim3(SP_NT), 0, st, rows, x.base, dst_arr,
-                  val_arr, acc_local, x.out_count, x.hot_fb, x.hot_count + 4);
+        // (each only where a bucket can reach it: a hop of at most SP_WB
+        // items fills no larger bucket, and one of at most SP_FEW entities
+        // has no more destinations than the paths before it take)
+        const bool wide = ((int64_t)1 << S) > SP_FEW;
+        if (h->items > SP_WB)
+            FL_LAUNCH("k_sp_accum_few", k_sp_accum_few, dim3((unsigned)mid_g),
+                      dim3(SP_NT), 0, st, rows, x.base, dst_arr, val_arr, acc_local, x.out_count, x.hot_list,
+                      x.mid_list, x.hot_fb, x.mid_fb, x.hot_count);
+        if (wide)
+            FL_LAUNCH("k_sp_accum_mid", k_sp_accum_mid, dim3((unsigned)mid_g),
+                      dim3(SP_NT), 0, st, rows, x.base, dst_arr, val_arr, acc_local, x.out_count, x.mid_fb,
+                      x.hot_count + 6);
+        if (wide && h->items > SP_CHUNK)
+            FL_LAUNCH("k_sp_accum_hot", k_sp_accum_hot, dim3(hot_grid), dim3(SP_NT), 0, st, rows, x.base, dst_arr,
+                      val_arr, acc_local, x.out_count, x.hot_fb, x.hot_count + 4);
     }
     if ((rc = exclusive_scan(st, x.out_count, out_base, R * NB, x.tmp)) != FL_OK) return rc;
     // the backward's map: each raw item's output index
@@ -4054,13 +4237,20 @@ int fl_sparse_backward(void *stream, const fl_side *ori, const fl_side *inv, con
     SpBwd x = sp_bwd_layout(h->nnz, R, h->n, (char *)workspace);
     SpEdge eg = sp_edge_layout(h->items, ori->edges, inv->edges, edge_grads ? (char *)workspace + own : nullptr);
     hipStream_t st = (hipStream_t)stream;
-    if (R * h->n > 0)
-        FL_LAUNCH("k_fill_f32", k_fill_f32, dim3((unsigned)((R * h->n + 255) / 256)), dim3(256), 0, st, grad_w,
-                  R * h->n, 0.0f);
-    if (h->nnz == 0 || R == 0) return fl_check_launch("sparse_backward");
-    FL_LAUNCH("k_sp_bw_chunks", k_sp_bw_chunks, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, p.row_ptr, R,
-              x.chunk_ptr);
-    if ((rc = exclusive_scan(st, x.chunk_ptr, x.chunk_ptr, R, x.tmp)) != FL_OK) return rc;
+    if (h->nnz == 0 || R == 0) {
+        if (R * h->n > 0)
+            FL_LAUNCH("k_fill_f32", k_fill_f32, dim3((unsigned)((R * h->n + 255) / 256)), dim3(256), 0, st, grad_w,
+                      R * h->n, 0.0f);
+        return fl_check_launch("sparse_backward");
+    }
+    // (k_sp_gw_fin writes every element of grad_w)
+    if (R <= SP_ONE_MAX) {
+        FL_LAUNCH("k_sp_bw_chunks", k_sp_bw_chunks_one, dim3(1), dim3(SP_ONE_NT), 0, st, p.row_ptr, R, x.chunk_ptr);
+    } else {
+        FL_LAUNCH("k_sp_bw_chunks", k_sp_bw_chunks, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, st, p.row_ptr, R,
+                  x.chunk_ptr);
+        if ((rc = exclusive_scan(st, x.chunk_ptr, x.chunk_ptr, R, x.tmp)) != FL_OK) return rc;
+    }
     const int holes = (h->mode == SP_TOPK && h->aggregate == SP_SUM) ? 1 : 0;
     if (h->n <= BW_LDS_MAX_N)
         FL_LAUNCH("k_sp_bwd", k_sp_bwd<true>, dim3((unsigned)x.blocks), dim3(SEL_NT),
@@ -4120,9 +4310,8 @@ int fl_sparse_topc(void *stream, const int64_t *sp_b, const int64_t *sp_l, const
         return fl_fail(FL_ERR_ARG, "sparse_topc: null argument");
     const int64_t R = B * L;
     hipStream_t st = (hipStream_t)stream;
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3((unsigned)((R + 1 + 255) / 256)), dim3(256), 0, st, row_ptr, R + 1,
-              (int64_t)0);
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3(1), dim3(64), 0, st, err, (int64_t)1, (int64_t)0);
+    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3((unsigned)((R + 2 + 255) / 256)), dim3(256), 0, st, row_ptr, R + 1,
+              (int64_t)0, err, (int64_t)1);
     const int64_t g1 = (nnz > R + 1 ? nnz : R + 1);
     FL_LAUNCH("k_sp_rowptr", k_sp_rowptr, dim3((unsigned)((g1 + 255) / 256)), dim3(256), 0, st, sp_b, sp_l, sp_b,
               nnz, B, L, INT64_MAX, row_ptr, err);
@@ -4171,9 +4360,8 @@ int fl_sparse_race_plan(void *stream, const int64_t *sp_b, const int64_t *sp_l, 
     if (ws_bytes < fl_sparse_race_bytes(nnz, R)) return fl_fail(FL_ERR_ARG, "sparse_race: workspace too small");
     SpRace x = sp_race_layout(nnz, R, (char *)ws);
     hipStream_t st = (hipStream_t)stream;
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3(1), dim3(64), 0, st, info, (int64_t)3, (int64_t)0);
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3((unsigned)((R + 1 + 255) / 256)), dim3(256), 0, st, x.row_ptr, R + 1,
-              (int64_t)0);
+    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3((unsigned)((R + 4 + 255) / 256)), dim3(256), 0, st, x.row_ptr, R + 1,
+              (int64_t)0, info, (int64_t)3);
     const int64_t g1 = (nnz > R + 1 ? nnz : R + 1);
     FL_LAUNCH("k_sp_rowptr", k_sp_rowptr, dim3((unsigned)((g1 + 255) / 256)), dim3(256), 0, st, sp_b, sp_l, sp_b, nnz,
               B, L, INT64_MAX, x.row_ptr, info + 1);
@@ -4185,11 +4373,9 @@ int fl_sparse_race_plan(void *stream, const int64_t *sp_b, const int64_t *sp_l, 
                   nnz, L, x.over, x.cand, info + 1);
     int rc;
     if ((rc = exclusive_scan(st, x.cand, x.cand_off, nnz, x.tmp)) != FL_OK) return rc;
-    FL_LAUNCH("k_fill_from", k_fill_from, dim3(1), dim3(1), 0, st, x.cand_off + nnz, info);
-    if (R > 0) {
-        if ((rc = exclusive_scan(st, x.kept, x.kept_off, R, x.tmp)) != FL_OK) return rc;
-        FL_LAUNCH("k_fill_from", k_fill_from, dim3(1), dim3(1), 0, st, x.kept_off + R, info + 2);
-    }
+    if (R > 0 && (rc = exclusive_scan(st, x.kept, x.kept_off, R, x.tmp)) != FL_OK) return rc;
+    FL_LAUNCH("k_race_info", k_race_info, dim3(1), dim3(1), 0, st, x.cand_off + nnz,
+              R > 0 ? x.kept_off + R : (const int64_t *)nullptr, info);
     return fl_check_launch("sparse_race_plan");
 }
 
@@ -4285,11 +4471,12 @@ int fl_sparse_normalize_forward(void *stream, const int64_t *sp_b, const int64_t
     hipStream_t st = (hipStream_t)stream;
     // the reference's GPU path checks no order either (flashlog.cu:2594-2649):
     // row starts by binary search, err cleared
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3(1), dim3(64), 0, st, err, (int64_t)1, (int64_t)0);
-    FL_LAUNCH("k_sp_rowptr_search", k_sp_rowptr_search, dim3((unsigned)((R + 1 + 255) / 256)), dim3(256), 0, st,
-              sp_b, sp_l, nnz, L, R, row_ptr);
     if (R > 0)
-        FL_LAUNCH("k_norm_fwd", k_norm_fwd, dim3((unsigned)R), dim3(NM_NT), 0, st, row_ptr, v, eps, out, denom);
+        FL_LAUNCH("k_norm_fwd", k_norm_fwd, dim3((unsigned)R), dim3(NM_NT), 0, st, sp_b, sp_l, nnz, L, R, v, eps, out,
+                  denom, row_ptr, err);
+    else
+        FL_LAUNCH("k_fill_i64", k_fill_i64, dim3(1), dim3(64), 0, st, row_ptr, (int64_t)1, (int64_t)0, err,
+                  (int64_t)1);
     return fl_check_launch("sparse_normalize");
 }
 
@@ -4352,9 +4539,8 @@ int fl_sparse_channel_sum_plan(void *stream, const int64_t *sp_b, const int64_t 
         return fl_fail(FL_ERR_ARG, "sparse_channel_sum: workspace too small");
     CsLayout x = cs_layout(nnz, R, (char *)ws);
     hipStream_t st = (hipStream_t)stream;
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3((unsigned)((R + 1 + 255) / 256)), dim3(256), 0, st, x.row_ptr, R + 1,
-              (int64_t)0);
-    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3(1), dim3(64), 0, st, x.err, (int64_t)2, (int64_t)0);
+    FL_LAUNCH("k_fill_i64", k_fill_i64, dim3((unsigned)((R + 3 + 255) / 256)), dim3(256), 0, st, x.row_ptr, R + 1,
+              (int64_t)0, x.err, (int64_t)2);
     const int64_t g1 = (nnz > R + 1 ? nnz : R + 1);
     FL_LAUNCH("k_sp_rowptr", k_sp_rowptr, dim3((unsigned)((g1 + 255) / 256)), dim3(256), 0, st, sp_b, sp_l, sp_e,
               nnz, B, L, E, x.row_ptr, x.err);
