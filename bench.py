@@ -879,14 +879,14 @@ def main_rules(args):
     prof = {k: _lib.prof_read(k) for k in RULE_STEP_KERNELS + RULE_ACC_KERNELS}
     _lib.prof_enable(False)
     # the steps' sizes, from a pass that grounds step by step
-    whole = si._grounds_in_one_launch
-    si._grounds_in_one_launch = lambda *a: False
+    whole = shared_inference._grounds_in_one_launch
+    shared_inference._grounds_in_one_launch = lambda *a: False
     fk.plan_log = []
     run()
     torch.cuda.synchronize()
     plans = fk.plan_log
     fk.plan_log = None
-    si._grounds_in_one_launch = whole
+    shared_inference._grounds_in_one_launch = whole
     per_pass = {k: v[0] for k, v in prof.items()}
     step_ms = sum(per_pass[k] for k in RULE_STEP_KERNELS)
     step_bytes = float(sum(rule_step_bytes(p) for p in plans))
