@@ -1955,54 +1955,71 @@ __global__ __launch_bounds__(SP_NT) void k_sp_accum_mid(SpRows rows, const int64
 // list).  One pass over the bucket marks its destinations; with more than
 // SP_FEW the bucket goes to a fallback list (k_sp_accum_mid / k_sp_accum_hot).
 // Otherwise destination j (in destination order) is slot j, the bucket's
-// output j, and thread j owns its sum in a register.  Chunks of SP_FEW_CHUNK
-// items in raw order: each item's slot is ranked among the equal slots of its
-// wave and round with ballots (as sp_block_sort does, one 6-bit pass), the
-// values are scattered slot-major into LDS in raw order within each slot, and
-// thread j adds its slot's run to its sum, in order.  raw_local (partition
-// order) gets each item's slot, written in place.  Holes (destination -1:
-// with one bucket per row the bucket is the row's raw items) are skipped.
+// output j, and lane j of the first wave owns its sum in a register.  The
+// other waves each take a segment of SP_FEW_SEG items of a chunk, in raw
+// order: an item's slot is ranked among the equal slots of its round with
+// ballots (as sp_block_sort does, one 6-bit pass) and the values are
+// scattered slot-major into LDS in raw order within each slot; the first
+// wave adds the segments' runs in order, a chunk behind the ranking.
+// raw_local (partition order) gets each item's slot, written in place.
+// Holes (destination -1: with one bucket per row the bucket is the row's raw
+// items) are skipped.
+//   A hub takes most items of its bucket, so that a bucket's time is that
+// of one chain of adds; ranking and adding by turns, with all four waves
+// ranking, left the chain standing still while the next items were ranked:
+// web graph, 598 -> 540 us; buckets of 41,000 entities, 44 -> 26.
+//   A wave for each bucket, which needs no barrier, took 931 us with claims of
+// every bucket and longer than this with fewer of them; all four waves
+// ranking 512 items each spilled registers (554 us).
 constexpr int SP_FEW = 64;
 constexpr int SP_FEW_RB = 6;
-constexpr int SP_FEW_CHUNK = 1024;  // items per ranked chunk
-constexpr int SP_FEW_IPT = SP_FEW_CHUNK / SP_NT;
-constexpr int SP_FEW_SPAN = SP_FEW_IPT * SP_NWV;           // (round, wave) entries of one slot
-constexpr int SP_FEW_TAB = SP_FEW * (SP_FEW_SPAN + 1);     // one count table, padded per slot
-constexpr int SP_FEW_PER = SP_FEW * SP_FEW_SPAN / SP_NT;   // scanned entries per thread
-static_assert(SP_FEW == (1 << SP_FEW_RB) && SP_FEW <= SP_NT, "one slot per thread");
+constexpr int SP_FEW_IPT = 4;
+constexpr int SP_FEW_RW = SP_NWV - 1;                   // ranking waves
+constexpr int SP_FEW_SEG = SP_FEW_IPT * FL_WAVE;        // items a wave ranks
+constexpr int SP_FEW_CHUNK = SP_FEW_RW * SP_FEW_SEG;    // items per chunk
+constexpr int SP_FEW_TAB = SP_FEW * (SP_FEW_IPT + 1);   // one wave's count table, padded per slot
+static_assert(SP_FEW == (1 << SP_FEW_RB) && SP_FEW == FL_WAVE, "one slot per lane");
+
+struct SpFewLds {
+    __align__(16) float sv[2][SP_FEW_RW][SP_FEW_SEG];  // values in slot order, by chunk parity and wave
+    uint16_t off[2][SP_FEW_RW][SP_FEW + 1];            // the slots' first values
+    uint16_t tab[SP_FEW_RW][SP_FEW_TAB];
+};
 
 __device__ __forceinline__ void sp_few_one(int wmask, int64_t start, int64_t n, int32_t dbase, int32_t *__restrict__ dst_arr,
                                            float *__restrict__ val_arr, int32_t *__restrict__ raw_local,
                                            int32_t *out_count, int total, const uint32_t *bits, const int *wpre,
-                                           const int32_t *slot_dl, uint16_t (*tab)[SP_FEW_TAB], float *sv,
-                                           int *scan_lds) {
-    const int t = threadIdx.x;
+                                           const int32_t *slot_dl, SpFewLds &lds) {
+    constexpr int IPT = SP_FEW_IPT;
+    const int lane = fl_lane();
     const int w = fl_wave_id();
-    for (int q = t; q < SP_FEW_TAB; q += SP_NT) tab[0][q] = 0;
-    float acc = 0.0f;  // thread t < total: the sum of slot t
+    const int rw = w - 1;
     // the bucket's items from wave-uniform bases, 32-bit offsets (a bucket
     // holds fewer than 2^31 items)
     const int32_t *__restrict__ bd = dst_arr + start;
     const float *__restrict__ bv = val_arr + start;
     const uint32_t un = (uint32_t)n;
-    int32_t pd[SP_FEW_IPT];
-    float pv[SP_FEW_IPT];
+    int32_t pd[IPT];
+    float pv[IPT];
+    auto request = [&](uint32_t c0) {  // the wave's segment of the chunk at c0
 #pragma unroll
-    for (int j = 0; j < SP_FEW_IPT; ++j) {  // striped: round j, thread t holds item j*SP_NT + t
-        const uint32_t k = (uint32_t)(j * SP_NT + t);
-        pd[j] = k < un ? fl_ld32(bd, k) : 0;
-        pv[j] = k < un ? fl_ld32(bv, k) : 0.0f;
-    }
-    __syncthreads();  // table cleared
-    int cur = 0;
-    for (uint32_t c0 = 0; c0 < un; c0 += SP_FEW_CHUNK) {
-        uint8_t sl[SP_FEW_IPT], rk[SP_FEW_IPT];
-        float vv[SP_FEW_IPT];
+        for (int j = 0; j < IPT; ++j) {  // striped: round j, lane l holds item j*64 + l
+            const uint32_t k = c0 + (uint32_t)(rw * SP_FEW_SEG + j * FL_WAVE + lane);
+            pd[j] = k < un ? fl_ld32(bd, k) : -1;
+            pv[j] = k < un ? fl_ld32(bv, k) : 0.0f;
+        }
+    };
+    auto rank = [&](uint32_t c0, int cur) {
+        uint16_t *tab = lds.tab[rw];
+#pragma unroll
+        for (int j = 0; j < IPT; ++j) tab[lane * (IPT + 1) + j] = 0;
+        fl_wave_sync();
+        uint8_t sl[IPT], rk[IPT];
+        float vv[IPT];
         uint32_t okm = 0;  // bit j: item j exists and is no hole
 #pragma unroll
-        for (int j = 0; j < SP_FEW_IPT; ++j) {
-            const uint32_t k = c0 + (uint32_t)(j * SP_NT + t);
-            const bool valid = k < un && pd[j] >= 0;
+        for (int j = 0; j < IPT; ++j) {
+            const bool valid = pd[j] >= 0;
             okm |= valid ? 1u << j : 0u;
             int sj = 0;
             if (valid) {
@@ -2012,64 +2029,61 @@ __device__ __forceinline__ void sp_few_one(int wmask, int64_t start, int64_t n, 
             uint32_t mlo, mhi;
             sp_peers<SP_FEW_RB>((uint32_t)sj, __builtin_amdgcn_ballot_w64(valid), mlo, mhi);
             const uint32_t below = __builtin_amdgcn_mbcnt_hi(mhi, __builtin_amdgcn_mbcnt_lo(mlo, 0u));
-            if (valid && below == 0)
-                tab[cur][sj * (SP_FEW_SPAN + 1) + j * SP_NWV + w] = (uint16_t)(__popc(mlo) + __popc(mhi));
-            if (valid && raw_local) fl_st32(raw_local + start, k, (int32_t)sj);
+            if (valid && below == 0) tab[sj * (IPT + 1) + j] = (uint16_t)(__popc(mlo) + __popc(mhi));
+            if (valid && raw_local)
+                fl_st32(raw_local + start, c0 + (uint32_t)(rw * SP_FEW_SEG + j * FL_WAVE + lane), (int32_t)sj);
             sl[j] = (uint8_t)sj;
             rk[j] = (uint8_t)below;
             vv[j] = pv[j];
         }
-        // the next chunk's items are requested while this one is scanned and added
-        if (c0 + SP_FEW_CHUNK < un) {
+        // the next chunk's items are requested while this one is scattered and added
+        if (c0 + SP_FEW_CHUNK < un) request(c0 + SP_FEW_CHUNK);
+        fl_wave_sync();
+        // lane s: slot s's rounds in order; the slots' runs are consecutive
+        int cs = 0;
 #pragma unroll
-            for (int j = 0; j < SP_FEW_IPT; ++j) {
-                const uint32_t k = c0 + SP_FEW_CHUNK + (uint32_t)(j * SP_NT + t);
-                pd[j] = k < un ? fl_ld32(bd, k) : 0;
-                pv[j] = k < un ? fl_ld32(bv, k) : 0.0f;
-            }
-        }
-        __syncthreads();  // counts written; every thread is past its previous sum
-        // exclusive scan in (slot, round, wave) order; the other table is cleared
-        int v[SP_FEW_PER];
-        int sum = 0;
+        for (int j = 0; j < IPT; ++j) cs += tab[lane * (IPT + 1) + j];
+        const int incl = fl_wave_incl_scan_i32(cs);
+        int run = incl - cs;
+        lds.off[cur][rw][lane] = (uint16_t)run;
+        if (lane == FL_WAVE - 1) lds.off[cur][rw][FL_WAVE] = (uint16_t)incl;
 #pragma unroll
-        for (int q = 0; q < SP_FEW_PER; ++q) {
-            const int f = t * SP_FEW_PER + q;
-            v[q] = tab[cur][f + f / SP_FEW_SPAN];
-            sum += v[q];
+        for (int j = 0; j < IPT; ++j) {
+            const int x = tab[lane * (IPT + 1) + j];
+            tab[lane * (IPT + 1) + j] = (uint16_t)run;
+            run += x;
         }
-        int tot;
-        int run = fl_block_excl_scan<SP_NT>(sum, scan_lds, &tot);
+        fl_wave_sync();
 #pragma unroll
-        for (int q = 0; q < SP_FEW_PER; ++q) {
-            const int f = t * SP_FEW_PER + q;
-            tab[cur][f + f / SP_FEW_SPAN] = (uint16_t)run;
-            run += v[q];
+        for (int j = 0; j < IPT; ++j)
+            if (okm & (1u << j)) lds.sv[cur][rw][tab[sl[j] * (IPT + 1) + j] + rk[j]] = vv[j];
+    };
+    float acc = 0.0f;  // first wave, lane < total: the sum of slot lane
+    if (w > 0) request(0);
+    int cur = 0;
+    for (uint32_t c0 = 0;; c0 += SP_FEW_CHUNK, cur ^= 1) {  // uniform: one chunk more than the bucket has
+        if (w > 0) {
+            if (c0 < un) rank(c0, cur);
+        } else if (c0 > 0) {
+            for (int k = 0; k < SP_FEW_RW; ++k)
+                acc = sp_fold(acc, lds.sv[cur ^ 1][k], lds.off[cur ^ 1][k][lane], lds.off[cur ^ 1][k][lane + 1]);
         }
-        for (int q = t; q < SP_FEW_TAB; q += SP_NT) tab[cur ^ 1][q] = 0;
         __syncthreads();
-#pragma unroll
-        for (int j = 0; j < SP_FEW_IPT; ++j) {
-            if (okm & (1u << j)) sv[tab[cur][sl[j] * (SP_FEW_SPAN + 1) + j * SP_NWV + w] + rk[j]] = vv[j];
-        }
-        __syncthreads();
-        if (t < total) {
-            const int lo = tab[cur][t * (SP_FEW_SPAN + 1)];
-            const int hi = t + 1 < SP_FEW ? tab[cur][(t + 1) * (SP_FEW_SPAN + 1)] : tot;
-            acc = sp_fold(acc, sv, lo, hi);
-        }
-        cur ^= 1;
+        if (c0 >= un) break;
     }
-    __syncthreads();  // every item was read: outputs may overwrite them
-    if (t < total) {
-        dst_arr[start + t] = dbase + slot_dl[t];
-        val_arr[start + t] = acc;
+    // every item was read: outputs may overwrite them
+    if (w == 0 && lane < total) {
+        dst_arr[start + lane] = dbase + slot_dl[lane];
+        val_arr[start + lane] = acc;
     }
-    if (t == 0) *out_count = total;
+    if (w == 0 && lane == 0) *out_count = total;
 }
 
-// lists: hot_list (ctr[0] listed, ctr[1] claim), then mid_list (ctr[2],
-// ctr[3]); fallbacks to hot_fb (ctr[4]) and mid_fb (ctr[6]).
+// Lists: hot_list (ctr[0] listed), then mid_list (ctr[2]); fallbacks to
+// hot_fb (ctr[4]) and mid_fb (ctr[6]).  Workgroup b takes bucket b of the two
+// lists first and then claims from ctr[1].  (A claim on each list for every
+// bucket, two additions to addresses that every XCD's workgroups share, took
+// longer than the sums: web graph, 823 -> 598 us by one claim.)
 __global__ __launch_bounds__(SP_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) void k_sp_accum_few(SpRows rows, const int64_t *__restrict__ base,
                                                        int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
                                                        int32_t *__restrict__ raw_local,
@@ -2081,28 +2095,17 @@ __global__ __launch_bounds__(SP_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) v
     __shared__ uint32_t bits[SP_W / 32];
     __shared__ int wpre[SP_W / 32];
     __shared__ int32_t slot_dl[SP_FEW];
-    __shared__ __align__(16) float sv[SP_FEW_CHUNK];
-    __shared__ uint16_t tab[2][SP_FEW_TAB];
+    __shared__ SpFewLds lds;
     __shared__ int scan_lds[SP_NT / FL_WAVE + 1];
     __shared__ int claim;
     static_assert(SP_W / 32 == SP_NT, "one bitmap word per thread");
     const int t = threadIdx.x;
     const int wmask = (1 << rows.S) - 1;
     const int nhot = ctr[0], nmid = ctr[2];
-    // workgroups past the listed buckets take none: the others claim every
-    // one (a participant stops only after a claim past the lists); the whole
-    // workgroup leaves at once, before any barrier
+    // workgroups past the listed buckets take none; the whole workgroup
+    // leaves at once, before any barrier
     if ((int)blockIdx.x >= nhot + nmid) return;
-    for (;;) {
-        __syncthreads();  // the previous bucket is done with the LDS arrays
-        if (t == 0) {
-            int c = atomicAdd(&ctr[1], 1);
-            if (c >= nhot) c = nhot + atomicAdd(&ctr[3], 1);
-            claim = c;
-        }
-        __syncthreads();
-        const int ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
-        if (ci >= nhot + nmid) break;
+    for (int ci = (int)blockIdx.x;;) {
         const bool hot = ci < nhot;
         const int64_t slot = hot ? hot_list[ci] : mid_list[ci - nhot];
         const int64_t r = slot / rows.NB, bk = slot - r * rows.NB;
@@ -2138,18 +2141,22 @@ __global__ __launch_bounds__(SP_NT) __attribute__((amdgpu_waves_per_eu(8, 8))) v
                 if (hot) hot_fb[atomicAdd(&ctr[4], 1)] = (int32_t)slot;
                 else mid_fb[atomicAdd(&ctr[6], 1)] = (int32_t)slot;
             }
-            continue;
+        } else {
+            wpre[t] = pre;
+            uint32_t wd = word;
+            for (int q = pre; wd; ++q) {
+                const int bit = __ffs(wd) - 1;
+                wd &= wd - 1;
+                slot_dl[q] = t * 32 + bit;
+            }
+            __syncthreads();
+            sp_few_one(wmask, start, n, (int32_t)(bk << rows.S), dst_arr, val_arr, raw_local, &out_count[slot], total,
+                       bits, wpre, slot_dl, lds);
         }
-        wpre[t] = pre;
-        uint32_t wd = word;
-        for (int q = pre; wd; ++q) {
-            const int bit = __ffs(wd) - 1;
-            wd &= wd - 1;
-            slot_dl[q] = t * 32 + bit;
-        }
-        __syncthreads();
-        sp_few_one(wmask, start, n, (int32_t)(bk << rows.S), dst_arr, val_arr, raw_local, &out_count[slot], total, bits, wpre,
-                   slot_dl, tab, sv, scan_lds);
+        if (t == 0) claim = (int)gridDim.x + atomicAdd(&ctr[1], 1);
+        __syncthreads();  // (and the bucket is done with the LDS arrays)
+        ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
+        if (ci >= nhot + nmid) break;
     }
 }
 
@@ -2464,8 +2471,8 @@ __global__ __launch_bounds__(SP_NT) void k_sp_max(SpRows rows, const int64_t *__
     }
 }
 
-// Persistent grid over the listed buckets: the hot ones (ctr[0] listed,
-// ctr[1] claim) and, when mid_too, the others (ctr[2], ctr[3]), of which
+// Persistent grid over the listed buckets: the hot ones (ctr[0] listed) and,
+// when mid_too, the others (ctr[2]), claimed from ctr[1], of which
 // those that hold a NaN go on to fb (ctr[6]).
 constexpr int SP_DENSE_MID_MAX = 1024;  // bucket widths whose dense arrays also serve the mid-size buckets
 
@@ -2493,23 +2500,20 @@ __global__ __launch_bounds__(SP_NT) void k_sp_max_hot(SpRows rows, const int64_t
     uint32_t *vbest = reinterpret_cast<uint32_t *>(max_lds + ((size_t)8 << rows.S));
     const int nhot = ctr[0], nmid = mid_too ? ctr[2] : 0;
     if ((int)blockIdx.x >= nhot + nmid) return;  // no bucket left for this workgroup (see k_sp_accum_few)
-    for (;;) {
-        __syncthreads();  // the previous bucket is done with the LDS arrays
-        if (threadIdx.x == 0) {
-            int c = atomicAdd(&ctr[1], 1);
-            if (c >= nhot && nmid > 0) c = nhot + atomicAdd(&ctr[3], 1);
-            claim = c;
-            nan_seen = 0;
-        }
+    for (int ci = (int)blockIdx.x;;) {  // its own number first, then claims
+        if (threadIdx.x == 0) nan_seen = 0;
         __syncthreads();
-        const int ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
-        if (ci >= nhot + nmid) break;
         const int64_t slot = ci < nhot ? hot_list[ci] : mid_list[ci - nhot];
         const int64_t r = slot / rows.NB, bk = slot - r * rows.NB;
         int64_t start, end;
         sp_bucket_range(rows, base, r, bk, &start, &end);
         sp_max_hot_one(rows, start, end - start, slot, (int32_t)(bk << rows.S), dst_arr, val_arr, tie_arr, raw_local,
                        out_count, vbest, tbest, bits, wpre, scan_lds, &nan_seen, ci < nhot ? nullptr : fb, ctr + 6);
+        __syncthreads();  // the bucket is done with the LDS arrays
+        if (threadIdx.x == 0) claim = (int)gridDim.x + atomicAdd(&ctr[1], 1);
+        __syncthreads();
+        ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
+        if (ci >= nhot + nmid) break;
     }
 }
 
@@ -3460,45 +3464,13 @@ __device__ __forceinline__ float block_tree_sum(float v, float *red) {
 // (flashlog.cpp:1561-1565).  The clamp is the GPU path's (flashlog.cu:2540):
 // d >= eps ? d : eps, so a NaN sum divides by eps.
 //   The chain of dependent adds bounds it.  The first wave does nothing else:
-// its first thread adds chunk c from LDS, the next 32 values on their way
-// while 32 are added, and the other waves bring in chunk c + 1 meanwhile.
+// its first thread adds chunk c from LDS and the other waves bring in chunk
+// c + 1 meanwhile.
 // The row's range is searched by the workgroup itself (row_ptr is kept for
 // the backward), so that the normalizer is one launch.
-//   Rows of 14,000 values: 87 us; with the chunk loaded by all
-// waves and each LDS round trip waited for 98 us.  Composing the adds of a
+//   Rows of 14,000 values: 85 us; with the chunk loaded by all waves 98 us.  Composing the adds of a
 // binade as maps of the mantissa's parity, in parallel, took as long (95 us).
 constexpr int NF_CHUNK = 2048;
-
-// sv[0 .. n) added to a, left to right; sv is 16-byte aligned.
-__device__ __forceinline__ float nf_fold(float a, const float *sv, int n) {
-    constexpr int U = 8;  // float4s on their way
-    const float4 *v4 = reinterpret_cast<const float4 *>(sv);
-    const int groups = n / (4 * U);
-    float4 x[U], y[U];
-    auto get = [&](float4 *d, int g) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) d[u] = v4[g * U + u];
-    };
-    auto add = [&](const float4 *d) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            a = fl_add(a, d[u].x);
-            a = fl_add(a, d[u].y);
-            a = fl_add(a, d[u].z);
-            a = fl_add(a, d[u].w);
-        }
-    };
-    int g = 0;
-    if (groups > 0) get(x, 0);
-    for (; g + 2 <= groups; g += 2) {
-        get(y, g + 1);
-        add(x);
-        get(x, min(g + 2, groups - 1));
-        add(y);
-    }
-    if (g < groups) add(x);
-    return sp_fold(a, sv, groups * 4 * U, n);
-}
 
 __global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl,
                                                    int64_t nnz, int64_t L, int64_t R, const float *__restrict__ v,
@@ -3533,7 +3505,7 @@ __global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ 
 #pragma unroll 4
             for (int i = t - FL_WAVE; i < len; i += NM_NT - FL_WAVE) cb[i] = v[base + NF_CHUNK + i];
         } else if (t == 0) {
-            acc = nf_fold(acc, (const float *)buf[c & 1], (int)((b - base) < NF_CHUNK ? (b - base) : NF_CHUNK));
+            acc = sp_fold(acc, (const float *)buf[c & 1], 0, (int)((b - base) < NF_CHUNK ? (b - base) : NF_CHUNK));
         }
         __syncthreads();
     }
