@@ -1222,39 +1222,53 @@ __global__ __launch_bounds__(RL_NT) void k_row_fill(const uint32_t *__restrict__
 // in CSR order (groups in order, each group's first `take` edges), 64 at a
 // time.  Lane j of a window holds group j; item k of the window belongs to
 // the first group whose inclusive take prefix exceeds k.  Each item's terms
-// (go*w)*m and (go*a)*m are formed in parallel; the contributing items are
-// then added one after another in position order -- the first term onto
-// acc, the second onto its group's partial, held by the group's lane -- so
-// the additions are those of a sequential walk.  MAX: only positions that
+// (go*w)*m and (go*a)*m are formed in parallel and put into the wave's LDS
+// (tl), -0, which leaves every sum as it is, for the items that do not
+// contribute; they are then added one after another in position order -- the
+// first term onto acc, by every lane alike, the second onto its group's
+// partial, by the group's lane -- so the additions are those of a sequential
+// walk.  (Terms passed from lane to lane, 14 instructions an item, kept the
+// wave issuing: 96,000 pairs, 41,000 entities, 149 -> 101 us.  The max's few
+// winners are passed so: 190 us against 206 through LDS.)  MAX: only positions that
 // won their destination (arg[row, dst] == p) contribute, as in the
 // winner-only backward (flashlog.cu:699-710); a winning position is always a
 // kept one.  Group partials go to the pair's row of relation columns in LDS
 // (pgl, written where take > 0).
+//   A wave is a chain of dependent loads, and its few items leave nothing to
+// hide them behind: the pair's threshold, its group ranges and the first
+// window of both sides are requested together before either side is walked,
+// and the row is found 64 candidates a step (96,000 pairs, 164 -> 149 us).
+struct BwdWindow {
+    int rel;
+    int32_t start, count;
+};
+__device__ __forceinline__ BwdWindow bwd_window(const fl_side &s, int64_t g, int64_t g1) {
+    BwdWindow x{0, 0, 0};
+    if (g < g1) {
+        x.rel = s.group_rel[g];
+        x.start = s.group_start[g];
+        x.count = s.group_count[g];
+    }
+    return x;
+}
+
 template <bool MAX>
-__device__ __forceinline__ float bwd_side(const fl_side &s, int64_t src, int64_t bl, int64_t BL, int64_t E,
-                                          int64_t n, int64_t off, int dir, float a, const float *__restrict__ w,
-                                          const float *__restrict__ grad, const int64_t *__restrict__ arg,
-                                          const float2 *__restrict__ PK, const int32_t *__restrict__ CUT,
-                                          float acc, float *pgl) {
+__device__ __forceinline__ float bwd_side(const fl_side &s, int64_t bl, int64_t E, int64_t n, int64_t off, float a,
+                                          const float *__restrict__ w, const float *__restrict__ grad,
+                                          const int64_t *__restrict__ arg, float th, int32_t cut, int64_t g0,
+                                          int64_t g1, BwdWindow x, float wv, float acc, float *pgl, float *tl) {
     const int lane = fl_lane();
-    const int64_t at = ((int64_t)dir * E + src) * BL + bl;
-    const float th = PK[at].y;
-    const int32_t cut = th > 0.0f ? CUT[at] : 0;
     const float *wr = w + bl * n + off;
     const float *gr = grad + bl * E;
     const int64_t *ar = MAX ? arg + bl * E : nullptr;
-    const int64_t g0 = s.row_group_ptr[src], g1 = s.row_group_ptr[src + 1];
     for (int64_t gb = g0; gb < g1; gb += FL_WAVE) {
-        const int64_t g = gb + lane;
-        int rel = 0;
-        int32_t start = 0, take = 0;
-        float wv = 0.0f;
-        if (g < g1) {
-            rel = s.group_rel[g];
-            wv = wr[rel];
-            start = s.group_start[g];
-            take = (int32_t)group_take(wv, th, cut, start, s.group_count[g]);
+        if (gb != g0) {  // x and wv hold the first window
+            x = bwd_window(s, gb + lane, g1);
+            wv = gb + lane < g1 ? wr[x.rel] : 0.0f;
         }
+        const int rel = x.rel;
+        const int32_t start = x.start;
+        const int32_t take = (int32_t)group_take(wv, th, cut, start, x.count);  // (0 past the end: wv is 0)
         // a source's kept edges on a side fit int32 (CSR positions are int32)
         const int32_t incl = fl_wave_incl_scan_i32(take);
         const int32_t total = __builtin_amdgcn_readlane(incl, FL_WAVE - 1);
@@ -1282,12 +1296,44 @@ __device__ __forceinline__ float bwd_side(const fl_side &s, int64_t src, int64_t
             const bool contrib = valid && win && m != 0.0f && go != 0.0f;
             const float t1 = fl_mul(fl_mul(go, wj), m);
             const float t2 = fl_mul(fl_mul(go, a), m);
-            for (uint64_t bal = __ballot(contrib); bal; bal &= bal - 1) {
-                const int i = __ffsll((long long)bal) - 1;
-                acc = fl_add(acc, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t1), i)));
-                const int gi = __builtin_amdgcn_readlane(j, i);
-                const float t2i = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t2), i));
-                if (lane == gi) gs = fl_add(gs, t2i);
+            uint64_t bal = __ballot(contrib);
+            if (bal == 0) continue;
+            if constexpr (MAX) {  // few items win
+                for (; bal; bal &= bal - 1) {
+                    const int i = __ffsll((long long)bal) - 1;
+                    acc = fl_add(acc, __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t1), i)));
+                    const int gi = __builtin_amdgcn_readlane(j, i);
+                    const float t2i = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(t2), i));
+                    if (lane == gi) gs = fl_add(gs, t2i);
+                }
+                continue;
+            }
+            fl_wave_sync();  // the terms before are added
+            tl[lane] = contrib ? t1 : -0.0f;
+            tl[FL_WAVE + lane] = contrib ? t2 : -0.0f;
+            fl_wave_sync();
+            // the pair's chain, the same in every lane
+            const int cnt = (int)(total - q0 < FL_WAVE ? total - q0 : FL_WAVE);
+            for (int i = 0; i < cnt; i += 16) {
+                float4 y[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) y[u] = reinterpret_cast<const float4 *>(tl)[i / 4 + u];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    acc = fl_add(acc, y[u].x);
+                    acc = fl_add(acc, y[u].y);
+                    acc = fl_add(acc, y[u].z);
+                    acc = fl_add(acc, y[u].w);
+                }
+            }
+            // the groups' chains, one in a lane: its items of these 64
+            const int lo = (int)max(incl - take - q0, 0), hi = (int)min(incl - q0, FL_WAVE);
+            for (int i = lo; i < hi; i += 4) {
+                float y[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) y[u] = i + u < hi ? tl[FL_WAVE + i + u] : -0.0f;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) gs = fl_add(gs, y[u]);
             }
         }
         if (take > 0) pgl[off + rel] = gs;
@@ -1310,26 +1356,41 @@ __global__ __launch_bounds__(BWD_NT) void k_bwd_pairs(
     const int32_t *__restrict__ rowlist, const int32_t *__restrict__ rowcnt, const int64_t *__restrict__ rowoff,
     int64_t pairs, float *__restrict__ gA, float *__restrict__ PG) {
     extern __shared__ float pg_lds[];  // [BWDP_WAVES][n]
+    __shared__ __align__(16) float terms[BWDP_WAVES][2 * FL_WAVE];
     const int lane = fl_lane();
     const int wid = fl_wave_id();
     const int64_t q = (int64_t)blockIdx.x * BWDP_WAVES + wid;
     if (q >= pairs || q >= rowoff[BL]) return;  // no block barrier follows
-    int64_t lo = 0, hi = BL;  // the row: rowoff[lo] <= q < rowoff[lo + 1]
-    while (hi - lo > 1) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (rowoff[mid] <= q) lo = mid;
-        else hi = mid;
+    // the row, the last with rowoff[row] <= q: 64 candidates a step
+    int64_t bl = 0;
+    for (int64_t len = BL; len > 1;) {
+        const int64_t step = (len + FL_WAVE - 1) / FL_WAVE, at = bl + lane * step;
+        const int below = __popcll(__ballot(at < bl + len && rowoff[at] <= q));  // at least lane 0
+        const int64_t skip = (below - 1) * step;
+        bl += skip;
+        len = len - skip < step ? len - skip : step;
     }
-    const int64_t bl = lo, k = q - rowoff[bl];
+    bl = fl_uniform_i64(bl);
+    const int64_t k = q - rowoff[bl];
     if (k >= rowcnt[bl]) return;
     const int64_t src = rowlist[bl * E + k];
+    const int64_t at_o = src * BL + bl, at_i = (E + src) * BL + bl;
     const float a = A[bl * E + src];
-    float *pgl = pg_lds + (int64_t)wid * n;
+    float acc = gA[bl * E + src];  // identity term written by k_bwd_identity
+    const float th_o = PK[at_o].y, th_i = PK[at_i].y;
+    const int32_t cut_o = CUT[at_o], cut_i = CUT[at_i];  // (read where the threshold is positive)
+    const int64_t o0 = ori.row_group_ptr[src], o1 = ori.row_group_ptr[src + 1];
+    const int64_t i0 = inv.row_group_ptr[src], i1 = inv.row_group_ptr[src + 1];
+    const BwdWindow xo = bwd_window(ori, o0 + lane, o1), xi = bwd_window(inv, i0 + lane, i1);
+    const float wo = o0 + lane < o1 ? w[bl * n + xo.rel] : 0.0f;
+    const float wi = i0 + lane < i1 ? w[bl * n + r_size + xi.rel] : 0.0f;
+    float *pgl = pg_lds + (int64_t)wid * n, *tl = terms[wid];
     for (int64_t r = lane; r < n; r += FL_WAVE) pgl[r] = 0.0f;
     fl_wave_sync();
-    float acc = gA[bl * E + src];  // identity term written by k_bwd_identity
-    acc = bwd_side<MAX>(ori, src, bl, BL, E, n, 0, 0, a, w, g_ori, arg_ori, PK, CUT, acc, pgl);
-    acc = bwd_side<MAX>(inv, src, bl, BL, E, n, r_size, 1, a, w, g_inv, arg_inv, PK, CUT, acc, pgl);
+    acc = bwd_side<MAX>(ori, bl, E, n, 0, a, w, g_ori, arg_ori, th_o, th_o > 0.0f ? cut_o : 0, o0, o1, xo, wo, acc,
+                        pgl, tl);
+    acc = bwd_side<MAX>(inv, bl, E, n, r_size, a, w, g_inv, arg_inv, th_i, th_i > 0.0f ? cut_i : 0, i0, i1, xi, wi,
+                        acc, pgl, tl);
     fl_wave_sync();
     float *pg = PG + q * n;
     for (int64_t r = lane; r < n; r += FL_WAVE) pg[r] = pgl[r];
@@ -1337,33 +1398,59 @@ __global__ __launch_bounds__(BWD_NT) void k_bwd_pairs(
 }
 
 // gw[row, r] for the relation columns r < 2*r_size: the pairs' partials in
-// ascending source order, GW_C pairs at a time through LDS.
-constexpr int GW_C = 32;
+// ascending source order.  A workgroup a row: the partials of a row are
+// contiguous, and come in GW_FLOATS at a time (whole pairs of n floats), the
+// next chunk on its way in registers while a thread a column adds this one
+// from LDS.  Few workgroups (one a row) leave it bound by the round trips to
+// memory, so the chunks are large: 1000 pairs a row of 75 columns, 24 us;
+// 32 pairs at a time, nothing on its way while they were added, 124 us.
+constexpr int GW_LOADS = 32;                     // floats per thread and chunk
+constexpr int GW_FLOATS = GW_LOADS * BWD_NT;
+constexpr int64_t GW_MAX_N = 512;                // (16 pairs a chunk at least)
 
 __global__ __launch_bounds__(BWD_NT) void k_bwd_gw(const float *__restrict__ PG, const int32_t *__restrict__ rowcnt,
                                                   const int64_t *__restrict__ rowoff, int64_t pairs, int64_t n,
                                                   int64_t nrel, float *__restrict__ gw) {
-    extern __shared__ float stage[];  // [GW_C][n]
+    __shared__ float stage[GW_FLOATS];
     const int64_t bl = blockIdx.x;
+    const int t = threadIdx.x;
     int64_t cnt = rowcnt[bl];
     if (rowoff[bl] + cnt > pairs) cnt = pairs - rowoff[bl] > 0 ? pairs - rowoff[bl] : 0;
     const float *pg = PG + rowoff[bl] * n;
+    const int un = (int)n;
+    const int rows = GW_FLOATS / un;  // pairs of a chunk
+    float x[GW_LOADS];
+    auto request = [&](int64_t k0) {
+        const int64_t left = cnt - k0;
+        const int m = (int)(left < rows ? left : rows) * un;
+        const float *src = pg + k0 * n;
+#pragma unroll
+        for (int j = 0; j < GW_LOADS; ++j) {
+            const int i = j * BWD_NT + t;
+            x[j] = i < m ? src[i] : 0.0f;
+        }
+    };
     float acc[4] = {0.f, 0.f, 0.f, 0.f};  // columns t, t+256, t+512, t+768
-    for (int64_t k0 = 0; k0 < cnt; k0 += GW_C) {
-        const int64_t kc = (cnt - k0 < GW_C) ? cnt - k0 : GW_C;
-        for (int64_t i = threadIdx.x; i < kc * n; i += BWD_NT) stage[i] = pg[k0 * n + i];
+    if (cnt > 0) request(0);
+    for (int64_t k0 = 0; k0 < cnt; k0 += rows) {
+        const int kc = (int)(cnt - k0 < rows ? cnt - k0 : rows);
+#pragma unroll
+        for (int j = 0; j < GW_LOADS; ++j) stage[j * BWD_NT + t] = x[j];
         __syncthreads();
+        if (k0 + rows < cnt) request(k0 + rows);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int64_t r = threadIdx.x + j * BWD_NT;
-            if (r < nrel)
-                for (int64_t k = 0; k < kc; ++k) acc[j] = fl_add(acc[j], stage[k * n + r]);
+            const int r = t + j * BWD_NT;
+            if (r < nrel) {
+#pragma unroll 8
+                for (int k = 0; k < kc; ++k) acc[j] = fl_add(acc[j], stage[k * un + r]);
+            }
         }
         __syncthreads();
     }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const int64_t r = threadIdx.x + j * BWD_NT;
+        const int64_t r = t + j * BWD_NT;
         if (r < nrel) gw[bl * n + r] = acc[j];
     }
 }
@@ -1599,7 +1686,7 @@ int dense_backward_impl(const char *name, void *stream, const fl_side *ori, cons
         return fl_fail(FL_ERR_ARG, "%s: w width too small for r_size", name);
     const int64_t nrel = 2 * r_size;
     if (nrel > 4 * BWD_NT) return fl_fail(FL_ERR_ARG, "%s: more than %d relation columns", name, 4 * BWD_NT);
-    if ((size_t)GW_C * n * sizeof(float) > 65536) return fl_fail(FL_ERR_ARG, "%s: w width too large", name);
+    if (n > GW_MAX_N) return fl_fail(FL_ERR_ARG, "%s: w width too large", name);
     if (pg_pairs < 0 || (pg_pairs > 0 && !pg)) return fl_fail(FL_ERR_ARG, "%s: bad partial buffer", name);
     if (!workspace || workspace_bytes < fl_dense_backward_workspace_bytes(ori, inv, BL, E))
         return fl_fail(FL_ERR_ARG, "%s: workspace too small", name);
@@ -1643,8 +1730,7 @@ int dense_backward_impl(const char *name, void *stream, const fl_side *ori, cons
             FL_LAUNCH("k_bwd_pairs", k_bwd_pairs<false>, dim3(nb), dim3(BWD_NT), plds, st, *ori, *inv, A, w,
                       grad_ori, grad_inv, (const int64_t *)nullptr, (const int64_t *)nullptr, BL, E, n, r_size,
                       ws.pk, ws.cut, rowlist, rowcnt, rowoff, pg_pairs, grad_A, pg);
-        const size_t lds = sizeof(float) * (size_t)(GW_C * n);
-        FL_LAUNCH("k_bwd_gw", k_bwd_gw, dim3((unsigned)BL), dim3(BWD_NT), lds, st, pg, rowcnt, rowoff, pg_pairs, n,
+        FL_LAUNCH("k_bwd_gw", k_bwd_gw, dim3((unsigned)BL), dim3(BWD_NT), 0, st, pg, rowcnt, rowoff, pg_pairs, n,
                   nrel, grad_w);
     }
     return fl_check_launch(name);
