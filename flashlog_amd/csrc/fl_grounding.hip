@@ -12,8 +12,9 @@
 //              (:112-449, 898-1027): attention-guided walks of rule_steps
 //              = 3 steps from every source, one wave per source task with
 //              the source's std::mt19937_64 in LDS (the walks of a source
-//              share one engine, so they run in order); a walk becomes a
-//              record (body key, ends at a positive target).
+//              share one engine: side by side from assumed positions in its
+//              words where every node's options are listed, else in order);
+//              a walk becomes a record (body key, ends at a positive target).
 //   count      per (head, fold) the records are sorted by body key (stable
 //              radix sort), runs give walk hits / source hits / positive
 //              walk and source hits; per length the rows are ranked by

@@ -3468,8 +3468,9 @@ __device__ __forceinline__ float block_tree_sum(float v, float *red) {
 // c + 1 meanwhile.
 // The row's range is searched by the workgroup itself (row_ptr is kept for
 // the backward), so that the normalizer is one launch.
-//   Rows of 14,000 values: 85 us; with the chunk loaded by all waves 98 us.  Composing the adds of a
-// binade as maps of the mantissa's parity, in parallel, took as long (95 us).
+//   Rows of 14,000 values: 85 us; with the chunk loaded by all waves 98 us.
+// Composing the adds of a binade as maps of the mantissa's parity, in
+// parallel, took 95 us.
 constexpr int NF_CHUNK = 2048;
 
 __global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl,

@@ -317,9 +317,10 @@ typedef struct fl_sparse_hop {
                                           when the backward reads no mask
                                           value or edge factor: the top-k
                                           sum (masked items are dropped)
-                                          with E > 8192, each side's mask
-                                          absent or given as mask_bits, and
-                                          no side carrying dscore.          */
+                                          over more than one bucket a row,
+                                          each side's mask absent or given
+                                          as mask_bits, and no side carrying
+                                          dscore.                           */
     int16_t *raw_col;                  /* with raw_local: [items] receives its
                                           attention column (ORI relation,
                                           r_size + INV relation, n - 1 for the
