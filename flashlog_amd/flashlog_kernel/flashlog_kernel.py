@@ -977,15 +977,19 @@ def dense_filtered_ranks_cuda(state, targets, filter_indices=None, use_eql=False
     targets = targets.long().contiguous()
     if targets.numel() != B:
         raise ValueError("dense_filtered_ranks_cuda: one target per query")
-    ranks = torch.empty(B, dtype=torch.float32, device=state.device)
-    if B == 0:
-        return ranks
+    if B and E == 0:
+        raise ValueError("dense_filtered_ranks_cuda: target out of range")
     fb = fe = None
     if filter_indices is not None:
         fb, fe = (x.to(state.device).long().contiguous() for x in filter_indices)
-        if fb.dim() != 1 or fb.shape != fe.shape:
-            raise ValueError("dense_filtered_ranks_cuda: filter indices must be equal 1D tensors")
+        if targets.dim() != 1 or fb.dim() != 1 or fb.shape != fe.shape:
+            raise ValueError("dense_filtered_ranks_cuda: targets and filter indices must be 1D, the latter equal")
     n = fb.numel() if fb is not None else 0
+    ranks = torch.empty(B, dtype=torch.float32, device=state.device)
+    if B == 0:
+        if n:
+            raise ValueError("dense_filtered_ranks_cuda: filter index out of range")
+        return ranks
     lib = _lib.lib()
     ws_bytes = lib.fl_dense_filtered_ranks_pairs_bytes(n, B)
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=state.device)

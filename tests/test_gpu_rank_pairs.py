@@ -38,3 +38,26 @@ def test_out_of_range(target, pair, message):
     with pytest.raises(ValueError, match=message + ".* out of range"):
         fk.dense_filtered_ranks_cuda(state, torch.tensor([1, target]).cuda(),
                                      (torch.tensor([pair[0]]).cuda(), torch.tensor([pair[1]]).cuda()))
+
+
+@pytest.mark.parametrize("B,E,pairs,message", [(0, 10, 1, "filter index out of range"), (2, 0, 0, "target out of range"),
+                                               (0, 0, 0, None), (0, 10, 0, None)])
+def test_empty_scores(B, E, pairs, message):
+    """No query or no entity: every index given is out of range."""
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    z = torch.zeros(pairs, dtype=torch.long, device="cuda")
+    args = torch.zeros(B, E, device="cuda"), torch.zeros(B, dtype=torch.long, device="cuda"), (z, z)
+    if message is None:
+        assert fk.dense_filtered_ranks_cuda(*args).shape == (0,)
+    else:
+        with pytest.raises(ValueError, match=message):
+            fk.dense_filtered_ranks_cuda(*args)
+
+
+def test_shapes_of_filter_and_targets():
+    """A filter needs flat targets and pairs of equal length."""
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    state, t = torch.rand(2, 10, device="cuda"), torch.zeros(2, dtype=torch.long, device="cuda")
+    for targets, pair in ((t[:, None], (t, t)), (t, (t, t[:1])), (t, (t[:, None], t[:, None]))):
+        with pytest.raises(ValueError, match="1D"):
+            fk.dense_filtered_ranks_cuda(state, targets, pair)
