@@ -187,8 +187,9 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
             return None
         idx = torch.empty((2, count), dtype=torch.int64, device=device)
         vals = torch.empty(count, dtype=torch.float32, device=device)
-        check(lib.fl_rule_collect_fill(st, ptr(total), nb, E, s0, ptr(ws), ptr(idx[0]), ptr(idx[1]), ptr(vals)),
-              "rule_collect")
+        if count:  # (a tensor of no elements has no address)
+            check(lib.fl_rule_collect_fill(st, ptr(total), nb, E, s0, ptr(ws), ptr(idx[0]), ptr(idx[1]), ptr(vals)),
+                  "rule_collect")
         parts.append((idx, vals))
     stats["chunks"] += len(chunks) * len(parts)
     stats["ground_calls"] += len(parts) * sum(max(lengths[lo:hi]) for lo, hi in chunks)

@@ -118,3 +118,15 @@ def test_source_outside():
     with pytest.raises(ValueError, match="out of range"):
         si._score_in_one_launch(torch.tensor([1, E]).cuda(), [(0, 1)], ops, [1], W, tc, R, E, 2, False, False, False,
                                 {"chunks": 0, "ground_calls": 0})
+
+
+@pytest.mark.parametrize("sources,block", [([0], None), ([0, 1, 5, 1], None), ([0, 1, 5, 0], 1), ([0, 5], 1)])
+def test_no_scores(sources, block):
+    """Bodies that begin at a source and end nowhere: calls, and blocks of a
+    call, without one scored entity."""
+    E, R = 50, 3
+    trip = _graph(E, [2], [([1], 2, [7])])
+    kw = {} if block is None else {"dense_budget_bytes": block * 2 * E * 4}
+    # (nodes 0 and 5 have no edge of relation 2, and no node has one of it twice)
+    _both(E, R, trip, sources, [[1, 2, 2], [0, R, 2, 2], [2]], **kw)
+    _both(E, R, trip, [0, 5], [[1, 2, 2], [2, 2]], **kw)
