@@ -1396,10 +1396,10 @@ def _grad_at_outputs(grad, out_indices, L, E):
     if out_indices.shape[0] == 2:  # [B, E]: one channel
         gi = (gi[0], torch.zeros_like(gi[0]), gi[1])
         q = (q[0], torch.zeros_like(q[0]), q[1])
-    check(_lib.lib().fl_sparse_gather(_stream(gv), ptr(gi[0].contiguous()), ptr(gi[1].contiguous()),
-                                      ptr(gi[2].contiguous()), ptr(gv), gv.numel(), ptr(q[0].contiguous()),
-                                      ptr(q[1].contiguous()), ptr(q[2].contiguous()), out.numel(), int(L), int(E),
-                                      ptr(out)), "sparse_gather")
+    # copies of strided rows live until the launch: one freed before the next is made would lend it its memory
+    gi, q = [x.contiguous() for x in gi], [x.contiguous() for x in q]
+    check(_lib.lib().fl_sparse_gather(_stream(gv), *(ptr(x) for x in gi), ptr(gv), gv.numel(), *(ptr(x) for x in q),
+                                      out.numel(), int(L), int(E), ptr(out)), "sparse_gather")
     return out.to(grad.dtype)
 
 

@@ -453,9 +453,10 @@ def _accumulate(state, W, dense, is_max, nb, E, boolean):
     lib = _lib.lib()
     ws_bytes = lib.fl_rule_accumulate_bytes(v.numel(), nb, C)
     ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=v.device)
-    check(lib.fl_rule_accumulate(fk._stream(v), ptr(ix[0].contiguous()), ptr(ix[1].contiguous()),
-                                 ptr(ix[2].contiguous()), ptr(v), v.numel(), ptr(W.contiguous()), W.shape[1], nb, C,
-                                 E, 1 if is_max else 0, ptr(dense), ptr(ws), ws_bytes), "rule_accumulate")
+    # copies of strided rows live until the launch: one freed before the next is made would lend it its memory
+    rows, W = [x.contiguous() for x in ix], W.contiguous()
+    check(lib.fl_rule_accumulate(fk._stream(v), *(ptr(x) for x in rows), ptr(v), v.numel(), ptr(W), W.shape[1],
+                                 nb, C, E, 1 if is_max else 0, ptr(dense), ptr(ws), ws_bytes), "rule_accumulate")
 
 
 def _finalize_normalized(dense, nb, E, s0, device):

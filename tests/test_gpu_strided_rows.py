@@ -1,0 +1,48 @@
+"""Index rows of a sparse gradient or state that are not contiguous (indices
+made as pairs and transposed) give what contiguous ones give."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _coo(shape, n, strided, seed=3):
+    """n distinct sorted entries, the index tensor's rows strided or not."""
+    g = torch.Generator().manual_seed(seed)
+    total = 1
+    for s in shape:
+        total *= s
+    flat = torch.randperm(total, generator=g)[:n].sort().values
+    cols = []
+    for s in reversed(shape):
+        cols.append(flat % s)
+        flat = flat // s
+    pairs = torch.stack(cols[::-1], 1).cuda()
+    idx = pairs.t() if strided else pairs.t().contiguous()
+    return torch.sparse_coo_tensor(idx, torch.rand(n, generator=g).cuda() + 0.5, shape, is_coalesced=True)
+
+
+@pytest.mark.parametrize("shape", [(5, 97), (4, 3, 97)])
+@pytest.mark.parametrize("strided_out", [False, True])
+@pytest.mark.parametrize("n", [1, 64, 257])
+def test_gradient_lookup(shape, strided_out, n):
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    grad = _coo(shape, n, True)
+    assert n == 1 or not grad._indices()[0].is_contiguous()
+    out = _coo(shape, 200, strided_out, seed=4)._indices()
+    got = fk._grad_at_outputs(grad, out, 1 if len(shape) == 2 else shape[1], shape[-1])
+    assert torch.equal(got, grad.to_dense()[tuple(out)])
+
+
+@pytest.mark.parametrize("is_max", [False, True])
+def test_rule_accumulation(is_max):
+    from flashlog_amd.rules import evaluate, shared_inference
+    nb, C, E = 4, 3, 97
+    W = torch.rand(2, C, device="cuda").t()
+    want = [torch.zeros(2, nb * E, device="cuda") for _ in range(2)]
+    got = [torch.zeros(2, nb * E, device="cuda") for _ in range(2)]
+    for dense, strided in ((want, False), (got, True)):
+        state = _coo((nb, C, E), 300, strided)
+        shared_inference._accumulate_chunk(state, W if strided else W.contiguous(), dense[0], is_max, nb, E)
+        evaluate._accumulate(state, W if strided else W.contiguous(), dense[1], is_max, nb, E, False)
+    assert bool(want[0].any()) and all(torch.equal(a, b) for a, b in zip(want, got))
