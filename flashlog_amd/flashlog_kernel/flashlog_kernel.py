@@ -1799,13 +1799,13 @@ def _normalize_forward(sp_b, sp_l, values, B, L, eps):
     coalesce(), and rows out of order give unspecified values without any
     access out of bounds."""
     _require_cuda(sp_b, sp_l, values)
-    values = values.contiguous().float()
+    # copies of the rows live until the launch: one freed before the next is made would lend it its memory
+    sp_b, sp_l, values = sp_b.long().contiguous(), sp_l.long().contiguous(), values.contiguous().float()
     R = B * L
     out = torch.empty_like(values)
     denom = torch.empty(max(R, 1), dtype=torch.float32, device=values.device)
     row_ptr, err = _sparse_rows_scratch(R, values.device)
-    check(_lib.lib().fl_sparse_normalize_forward(_stream(values), ptr(sp_b.long().contiguous()),
-                                                 ptr(sp_l.long().contiguous()), ptr(values), values.numel(),
+    check(_lib.lib().fl_sparse_normalize_forward(_stream(values), ptr(sp_b), ptr(sp_l), ptr(values), values.numel(),
                                                  B, L, ctypes.c_float(eps), ptr(out), ptr(denom), ptr(row_ptr),
                                                  ptr(err)), "sparse_normalize")
     return out, denom[:R], row_ptr

@@ -46,3 +46,26 @@ def test_rule_accumulation(is_max):
         shared_inference._accumulate_chunk(state, W if strided else W.contiguous(), dense[0], is_max, nb, E)
         evaluate._accumulate(state, W if strided else W.contiguous(), dense[1], is_max, nb, E, False)
     assert bool(want[0].any()) and all(torch.equal(a, b) for a, b in zip(want, got))
+
+
+def _rows(kind, x):
+    """The row as a program may hold it: every second element of a larger one, or 32-bit."""
+    if kind == "int32":
+        return x.to(torch.int32)
+    return torch.stack([x, torch.zeros_like(x)], 1)[:, 0]
+
+
+@pytest.mark.parametrize("kind", ["strided", "int32"])
+@pytest.mark.parametrize("L", [1, 3])
+def test_normalize_forward(kind, L):
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    mod = fk.get_module()
+    B, E = 5, 97
+    state = _coo((B, L, E), 300, False)
+    b, l, _ = state._indices()
+    want = mod.sparse3d_normalize_forward_cuda(b, l, state._values(), B, L, 1e-7)
+    got = mod.sparse3d_normalize_forward_cuda(_rows(kind, b), _rows(kind, l), state._values(), B, L, 1e-7)
+    assert all(torch.equal(x, y) for x, y in zip(got, want))
+    sums = torch.zeros(B * L, dtype=torch.float64, device="cuda").index_add_(0, b * L + l, state._values().double())
+    # at most 300 additions of one rounding each
+    torch.testing.assert_close(got[1].view(-1).double(), sums, rtol=300 * 2.0 ** -24, atol=0)
