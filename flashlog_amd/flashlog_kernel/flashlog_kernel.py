@@ -505,10 +505,10 @@ class _HipModule:
         if mask_values.dtype not in (torch.bool, torch.float32):
             raise RuntimeError("edge visibility mask must be bool or float32")
         has_w = weight is not None and weight.numel() > 0
-        check(_lib.lib().fl_apply_mask(_stream(out), ptr(mask_values.contiguous()),
-                                       1 if mask_values.dtype == torch.bool else 0, ptr(order),
-                                       ptr(weight.float().contiguous()) if has_w else None, ptr(out), nnz),
-              "apply_mask")
+        # copies live until the launch: one freed before the next is made would lend it its memory
+        mask, weight = mask_values.contiguous(), weight.float().contiguous() if has_w else None
+        check(_lib.lib().fl_apply_mask(_stream(out), ptr(mask), 1 if mask.dtype == torch.bool else 0, ptr(order),
+                                       ptr(weight), ptr(out), nnz), "apply_mask")
         return out
 
     @staticmethod

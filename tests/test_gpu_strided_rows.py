@@ -69,3 +69,24 @@ def test_normalize_forward(kind, L):
     sums = torch.zeros(B * L, dtype=torch.float64, device="cuda").index_add_(0, b * L + l, state._values().double())
     # at most 300 additions of one rounding each
     torch.testing.assert_close(got[1].view(-1).double(), sums, rtol=300 * 2.0 ** -24, atol=0)
+
+
+@pytest.mark.parametrize("weight_kind", ["strided", "float64", "contiguous", None])
+@pytest.mark.parametrize("mask_kind", ["strided", "contiguous", "strided bool"])
+def test_apply_mask(mask_kind, weight_kind):
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    n = 1000
+    g = torch.Generator().manual_seed(7)
+    mask = torch.rand(n, generator=g).cuda()
+    if mask_kind == "strided bool":
+        mask = mask < 0.5
+    weight = torch.randn(n, generator=g).cuda()
+    order = torch.randperm(n, generator=g).to(torch.int32).cuda()
+    mod = fk.get_module()
+    want = mod.apply_mask_cuda(mask, order, weight if weight_kind else None)
+    # the factor sigmoid(weight): expf (2 ulp), a sum, a division and the product, one rounding each
+    ref = mask[order.long()].double() * (torch.sigmoid(weight[order.long()].double()) if weight_kind else 1)
+    torch.testing.assert_close(want.double(), ref, rtol=8 * 2.0 ** -24, atol=0)
+    m = mask if mask_kind == "contiguous" else _rows("strided", mask)
+    w = {"strided": _rows("strided", weight), "float64": weight.double(), "contiguous": weight, None: None}[weight_kind]
+    assert torch.equal(mod.apply_mask_cuda(m, order, w), want)
