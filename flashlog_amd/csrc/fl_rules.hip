@@ -123,7 +123,10 @@ __global__ __launch_bounds__(RA_NT) void k_ra_sum(const int64_t *__restrict__ se
 // float sum of them is exact in any order, else the row reports RG_LIMIT and
 // the caller takes the general path, as it does for a row of more than
 // RG_ITEMS_MAX edges in a step (which the general path spreads over the
-// chip) and for a full pool.
+// chip) and for a full pool.  Chunks before that one are added and stay so;
+// later chunks are left, and so are listed rows that begin after the report.
+// (k_rg_rows reads the report as it was at its start: asked for past the L2
+// by every row, 1024 sources took 2732 us instead of 2435.)
 //   k_rg_rows    state in a hash table (RG_TAB slots, at most RG_CAP
 //                entities): five workgroups a CU;
 //   k_rg_dense   the rows that outgrow it, from a list: two dense arrays of
@@ -149,16 +152,20 @@ struct RgPool {
     float *val;               // [cap]
     int64_t cap;
     int32_t *over;            // rows for k_rg_dense
-    // [0] pool entries taken, [1] status, [2] listed rows, [3] next row to claim
+    // [0] pool entries taken, [1] status, [2] listed rows, [3] next row to claim, [4] the status at the launch's start
     unsigned long long *ctr;
 };
+constexpr int RG_CTR = 5;
 
+// status: [0] the worst report of the calls so far, [1] chunks added
 __global__ void k_rg_zero(unsigned long long *ctr, const unsigned long long *status) {
-    if (threadIdx.x < 4) ctr[threadIdx.x] = threadIdx.x == 1 ? *status : 0ull;
+    if (threadIdx.x < RG_CTR) ctr[threadIdx.x] = threadIdx.x == 1 || threadIdx.x == 4 ? *status : 0ull;
 }
 
 __global__ void k_rg_status(const unsigned long long *ctr, unsigned long long *status) {
-    if (threadIdx.x == 0) *status = ctr[1];
+    if (threadIdx.x != 0) return;
+    status[0] = ctr[1];
+    if (ctr[1] == 0) status[1] += 1;
 }
 
 // Expands n entries (get(i, node, count), count 0: no entry) through relation
@@ -227,6 +234,7 @@ __global__ __launch_bounds__(RG_NT) void k_rg_rows(fl_side ori, fl_side inv, con
     const int t = threadIdx.x;
     const int64_t row = blockIdx.x, b = row / C, r = row - b * C;
     const int64_t src = sources[b];
+    if (pool.ctr[4] != 0) return;  // uniform: nothing of this chunk is used
     if (src < 0 || src >= E) {  // uniform
         if (t == 0) {
             atomicMax(&pool.ctr[1], (unsigned long long)RG_SOURCE);
@@ -334,7 +342,11 @@ __global__ __launch_bounds__(RG_DENSE_NT) void k_rg_dense(fl_side ori, fl_side i
     if ((int)blockIdx.x >= rows) return;
     for (;;) {
         __syncthreads();  // the last row is done with the LDS arrays
-        if (t == 0) claim = (int)atomicAdd(&pool.ctr[3], 1ull);
+        if (t == 0) {
+            // (one thread asks: the report may come while this kernel runs)
+            const unsigned long long at = atomicAdd(&pool.ctr[3], 1ull);
+            claim = __hip_atomic_load(&pool.ctr[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ? rows : (int)at;
+        }
         __syncthreads();
         const int ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
         if (ci >= rows) break;
@@ -580,7 +592,7 @@ static size_t rg_layout(int64_t nb, int64_t C, int64_t cap, char *base, fl::RgPo
     size_t off = 0;
     auto take = [&](size_t b) { char *q = base ? base + off : nullptr; off += (b + 255) & ~(size_t)255; return q; };
     const int64_t rows = nb * C > 0 ? nb * C : 1;
-    p->ctr = (unsigned long long *)take(4 * sizeof(unsigned long long));
+    p->ctr = (unsigned long long *)take(fl::RG_CTR * sizeof(unsigned long long));
     p->seg = (fl::RgSeg *)take(sizeof(fl::RgSeg) * (size_t)rows);
     p->over = (int32_t *)take(sizeof(int32_t) * (size_t)rows);
     p->ent = (int32_t *)take(sizeof(int32_t) * (size_t)cap);
@@ -616,7 +628,7 @@ int fl_rule_ground(void *stream, const fl_side *ori, const fl_side *inv, const i
     RgPool p;
     (void)rg_layout(nb, C, pool, (char *)ws, &p);
     hipStream_t st = (hipStream_t)stream;
-    // (status, given by the caller and zeroed by it, holds the worst of the calls that share it)
+    // (status, given by the caller and zeroed by it, is that of all calls that share it)
     FL_LAUNCH("k_rg_zero", k_rg_zero, dim3(1), dim3(64), 0, st, p.ctr, (const unsigned long long *)status);
     FL_LAUNCH("k_rg_rows", k_rg_rows, dim3((unsigned)(nb * C)), dim3(RG_NT), 0, st, *ori, *inv, sources, operators,
               lengths, C, steps, E, r_size, boolean_paths, p);

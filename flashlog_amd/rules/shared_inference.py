@@ -19,7 +19,10 @@ None): ev.initial_rule_state and ev.vectorized_operation_sparse3d_fixed_relation
 with ev.advance_single_rule_state_memory_bounded after an out-of-memory
 step of one source and one rule.  A chunk whose grounding runs out of
 memory is retried with half as many rules (stats["oom_retries"]), down to
-one rule.  Grounded chunks are added into a dense [ranks, sources x
+one rule.  With this package's own hooks and few enough entities a chunk is
+grounded by one launch (fl_rule_ground) instead, up to the first chunk with a
+state beyond what that holds: it and the chunks after it take the steps.
+Grounded chunks are added into a dense [ranks, sources x
 entities] accumulator by fl_rule_accumulate (sums: per (source, entity) the
 chunk's rules in rule order, chunks in order; maxima: exact) and finalized
 by fl_rule_finalize.  Sources are taken in blocks sized so that the
@@ -145,23 +148,30 @@ def _grounds_in_one_launch(ev, csr, entities, device):
             and entities <= _lib.lib().fl_rule_ground_max_entities())
 
 
+def _progress():
+    """What _score_in_one_launch got done: ``parts``, the (indices, scores) of the finished blocks of sources, and of
+    the block that begins at ``source`` the accumulator ``dense`` with the rules before ``rule`` in it."""
+    return types.SimpleNamespace(parts=[], source=0, rule=0, dense=None)
+
+
 def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, relations, E, block, is_max, boolean_paths,
-                         final_max, stats):
-    """(rows, columns, scores) of the blocks of sources with every chunk of rules grounded by one launch
+                         final_max, stats, done=None):
+    """(indices, scores) of the blocks of sources with every chunk of rules grounded by one launch
     (fl_rule_ground) and the scored entities collected with one host read per block, or None when a state outgrew
-    what those kernels hold (the caller grounds step by step)."""
+    what those kernels hold (the caller grounds step by step from where ``done`` says)."""
     lib = _lib.lib()
     device = sources.device
     sides = fk._fixed_sides(csr)
     ranks = weights.shape[1]
     lengths_d = torch.tensor(lengths, dtype=torch.int32).to(device)
     st = fk._stream(sources)
-    parts = []
+    done = _progress() if done is None else done
     for s0 in range(0, sources.numel(), block):
         src = sources[s0:s0 + block]
         nb = src.numel()
         dense = torch.zeros((ranks, nb * E), dtype=torch.float32, device=device)
-        status = torch.zeros(1, dtype=torch.int64, device=device)
+        words = torch.zeros(4, dtype=torch.int64, device=device)
+        status, info = words[:2], words[2:]
         widest = max(hi - lo for lo, hi in chunks)
         pool = min(nb * widest * E, _POOL_ENTRIES)
         collect_bytes = lib.fl_rule_collect_bytes(nb, E)
@@ -177,22 +187,28 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
         total = torch.empty(nb * E, dtype=torch.float32, device=device)
         check(lib.fl_rule_finalize(st, ptr(dense), ranks, nb, E, 1 if final_max else 0, ptr(rowsum), ptr(total)),
               "rule_finalize")
-        info = torch.empty(2, dtype=torch.int64, device=device)
         check(lib.fl_rule_collect_plan(st, ptr(total), nb, E, ptr(status), ptr(ws), ws_bytes, ptr(info)),
               "rule_collect")
-        count, bad = info.tolist()
+        bad, added, count, _ = words.tolist()
         if bad == 1:
             raise ValueError("sparse state index out of range for shape (%d, %d, %d)" % (nb, widest, E))
+        stats["chunks"] += added
+        stats["ground_calls"] += sum(max(lengths[lo:hi]) for lo, hi in chunks[:added])
         if bad:
+            done.dense, done.rule = dense, chunks[added][0]
             return None
         idx = torch.empty((2, count), dtype=torch.int64, device=device)
         vals = torch.empty(count, dtype=torch.float32, device=device)
         if count:  # (a tensor of no elements has no address)
             check(lib.fl_rule_collect_fill(st, ptr(total), nb, E, s0, ptr(ws), ptr(idx[0]), ptr(idx[1]), ptr(vals)),
                   "rule_collect")
-        parts.append((idx, vals))
-    stats["chunks"] += len(chunks) * len(parts)
-    stats["ground_calls"] += len(parts) * sum(max(lengths[lo:hi]) for lo, hi in chunks)
+        done.parts.append((idx, vals))
+        done.source = s0 + nb
+    return _joined(done.parts)
+
+
+def _joined(parts):
+    """(indices, scores) of consecutive blocks of sources."""
     if len(parts) == 1:
         return parts[0]
     return torch.cat([i for i, _ in parts], 1), torch.cat([v for _, v in parts])
@@ -277,11 +293,12 @@ def score(ev, sources, rules, csr, relations, entities, chunk_size,
     stats["dense_accumulation"] = True
     stats["prefix_enabled"] = False
     is_max = reduction == "max"
+    done = _progress()
     if _grounds_in_one_launch(ev, csr, E, device):
         chunks = [(lo, min(lo + chunk_size, len(rules))) for lo in range(0, len(rules), chunk_size)]
         try:
             found = _score_in_one_launch(sources.contiguous(), chunks, operators, lengths, weights, csr, relations, E,
-                                         block, is_max, boolean_paths, final_max, stats)
+                                         block, is_max, boolean_paths, final_max, stats, done)
         except torch.cuda.OutOfMemoryError:
             found = None  # step by step, with chunks halved as far as needed
             torch.cuda.empty_cache()
@@ -314,12 +331,13 @@ def score(ev, sources, rules, csr, relations, entities, chunk_size,
             state = advance(state, ops[:, step].unsqueeze(0).expand(nb, -1), nb)
         return state
 
-    keys_out, vals_out = [], []
-    for s0 in range(0, batch, block):
+    for s0 in range(done.source, batch, block):
         src = sources[s0:s0 + block]
         nb = src.numel()
-        dense = torch.zeros((ranks, nb * E), dtype=torch.float32, device=device)
-        off, size = 0, chunk_size
+        dense, off, size = done.dense, done.rule, chunk_size
+        if dense is None:
+            dense = torch.zeros((ranks, nb * E), dtype=torch.float32, device=device)
+        done.dense, done.rule = None, 0
         while off < len(rules):
             hi = min(off + size, len(rules))
             try:
@@ -336,9 +354,6 @@ def score(ev, sources, rules, csr, relations, entities, chunk_size,
             off = hi
             stats["chunks"] += 1
         keys, vals = _finalize(dense, nb, E, final_max)
-        keys_out.append(keys + s0 * E)
-        vals_out.append(vals)
+        done.parts.append((torch.stack((keys // E + s0, keys % E)), vals))
         del dense
-    keys = torch.cat(keys_out)
-    return torch.sparse_coo_tensor(torch.stack((keys // E, keys % E)), torch.cat(vals_out), shape,
-                                   is_coalesced=True)
+    return torch.sparse_coo_tensor(*_joined(done.parts), shape, is_coalesced=True)

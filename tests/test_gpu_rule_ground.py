@@ -130,3 +130,70 @@ def test_no_scores(sources, block):
     # (nodes 0 and 5 have no edge of relation 2, and no node has one of it twice)
     _both(E, R, trip, sources, [[1, 2, 2], [0, R, 2, 2], [2]], **kw)
     _both(E, R, trip, [0, 5], [[1, 2, 2], [2, 2]], **kw)
+
+
+def _hub(E, n):
+    """Node 7 with n edges of relation 2; relation 1: node j to j + 1; relation 0: node 0 to two nodes."""
+    return _graph(E, [2], [(np.full(n, 7), 2, np.arange(n) % E)])
+
+
+def _counted_steps(monkeypatch):
+    """The calls of the step-by-step form, of this package's own hooks too."""
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    from flashlog_amd.rules import evaluate as ev
+    calls = []
+    real = fk.vectorized_operation_sparse3d_fixed_relation
+
+    def step(*a, **k):
+        calls.append(a[0].shape)
+        return real(*a, **k)
+
+    monkeypatch.setattr(fk, "vectorized_operation_sparse3d_fixed_relation", step)
+    monkeypatch.setattr(ev, "vectorized_operation_sparse3d_fixed_relation", step)
+    return calls
+
+
+@pytest.mark.parametrize("at", [0, 7, 19])
+@pytest.mark.parametrize("block", [None, 2])
+def test_what_was_grounded_before_a_limit_is_kept(monkeypatch, at, block):
+    """20 rules in chunks of 5, one of them with a row beyond the limits: the chunks (and blocks of sources) before it
+    are not grounded again."""
+    E, R = 3000, 3
+    h, r, t = _hub(E, (1 << 20) + 1)
+    tc = to_torch_csr(O.build_csr_structure(h, t, r, E), torch.device("cuda"))
+    bodies = [[1, 1]] * 20
+    bodies[at] = [2]
+    W = np.random.default_rng(9).random((20, 2)).astype(np.float32)
+    rules = [{"body": b, "rank_weights": [float(x) for x in w]} for b, w in zip(bodies, W)]
+    src = torch.tensor([3, 4, 5, 6, 7, 9]).cuda()  # node 7 in the third block of two
+    kw = {} if block is None else {"dense_budget_bytes": block * 2 * E * 4}
+    want_stats, stats = {}, {}
+    want = _score(_stepwise(), src, rules, tc, R, E, 5, stats=want_stats, **kw)
+    calls = _counted_steps(monkeypatch)
+    got = _score(None, src, rules, tc, R, E, 5, stats=stats, **kw)
+    assert torch.equal(got.indices(), want.indices()) and torch.equal(got.values(), want.values())
+    assert stats["chunks"] == want_stats["chunks"]
+    assert len(calls) == 2 * (4 - at // 5)  # (every chunk has a body of two steps)
+
+
+def test_rows_after_a_limit_are_left():
+    """Chunks behind one that outgrew the kernels are not walked."""
+    from flashlog_amd import _lib
+    E, R = 3000, 4
+    n = 1 << 19
+    h, r, t = _hub(E, (1 << 20) + 1)
+    h, r, t = np.concatenate([h, np.full(n, 7)]), np.concatenate([r, np.full(n, 3)]), np.concatenate([t, np.arange(n) % E])
+    tc = to_torch_csr(O.build_csr_structure(h, t, r, E), torch.device("cuda"))
+
+    def walked(bodies):
+        rules = [{"body": b, "rank_weights": [0.5]} for b in bodies]
+        run = lambda: _score(None, torch.tensor([7]).cuda(), rules, tc, R, E, 1)
+        run()
+        _lib.prof_enable(True)
+        try:
+            run()
+            return _lib.prof_read("k_rg_rows")[0] + _lib.prof_read("k_rg_dense")[0]
+        finally:
+            _lib.prof_enable(False)
+
+    assert walked([[2]] + [[3]] * 4) < walked([[3]])
