@@ -123,7 +123,8 @@ __global__ __launch_bounds__(RA_NT) void k_ra_sum(const int64_t *__restrict__ se
 // float sum of them is exact in any order, else the row reports RG_LIMIT and
 // the caller takes the general path, as it does for a row of more than
 // RG_ITEMS_MAX edges in a step (which the general path spreads over the
-// chip) and for a full pool.  Chunks before that one are added and stay so;
+// chip).  A chunk that overruns the pool reports how much it asks for.
+// Chunks before a report are added and stay so;
 // later chunks are left, and so are listed rows that begin after the report.
 // (k_rg_rows reads the report as it was at its start: asked for past the L2
 // by every row, 1024 sources took 2732 us instead of 2435.)
@@ -139,7 +140,7 @@ constexpr int RG_NT = 128, RG_TAB = 2048, RG_CAP = 1536;
 constexpr int RG_DENSE_NT = 512;
 constexpr int RG_ITEMS_MAX = 1 << 20;
 constexpr unsigned long long RG_PATHS_MAX = 1ull << 24;
-enum { RG_SOURCE = 1, RG_LIMIT = 2 };
+enum { RG_SOURCE = 1, RG_POOL = 2, RG_LIMIT = 3 };  // the larger report stands
 
 struct RgSeg {
     int64_t base;
@@ -157,15 +158,17 @@ struct RgPool {
 };
 constexpr int RG_CTR = 5;
 
-// status: [0] the worst report of the calls so far, [1] chunks added
+// status: [0] the worst report of the calls so far, [1] chunks added, [2] the
+// pool entries that the chunk of a first RG_POOL asks for
 __global__ void k_rg_zero(unsigned long long *ctr, const unsigned long long *status) {
     if (threadIdx.x < RG_CTR) ctr[threadIdx.x] = threadIdx.x == 1 || threadIdx.x == 4 ? *status : 0ull;
 }
 
 __global__ void k_rg_status(const unsigned long long *ctr, unsigned long long *status) {
     if (threadIdx.x != 0) return;
-    status[0] = ctr[1];
     if (ctr[1] == 0) status[1] += 1;
+    if (status[0] == 0) status[2] = ctr[0];
+    status[0] = ctr[1];
 }
 
 // Expands n entries (get(i, node, count), count 0: no entry) through relation
@@ -313,7 +316,7 @@ __global__ __launch_bounds__(RG_NT) void k_rg_rows(fl_side ori, fl_side inv, con
     if (t == 0) {
         base_lds = n > 0 ? atomicAdd(&pool.ctr[0], (unsigned long long)n) : 0;
         const bool fits = (int64_t)base_lds + n <= pool.cap;
-        if (!fits) atomicMax(&pool.ctr[1], (unsigned long long)RG_LIMIT);
+        if (!fits) atomicMax(&pool.ctr[1], (unsigned long long)RG_POOL);
         pool.seg[row] = {(int64_t)base_lds, fits ? (int64_t)n : 0};
     }
     __syncthreads();
@@ -345,7 +348,9 @@ __global__ __launch_bounds__(RG_DENSE_NT) void k_rg_dense(fl_side ori, fl_side i
         if (t == 0) {
             // (one thread asks: the report may come while this kernel runs)
             const unsigned long long at = atomicAdd(&pool.ctr[3], 1ull);
-            claim = __hip_atomic_load(&pool.ctr[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 ? rows : (int)at;
+            // (a chunk that only overran the pool is walked to its end, which tells how much it asks for)
+            const unsigned long long now = __hip_atomic_load(&pool.ctr[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            claim = now != 0 && now != RG_POOL ? rows : (int)at;
         }
         __syncthreads();
         const int ci = __builtin_amdgcn_readfirstlane(claim);  // uniform: scalar registers
@@ -399,7 +404,7 @@ __global__ __launch_bounds__(RG_DENSE_NT) void k_rg_dense(fl_side ori, fl_side i
             if (limit) atomicMax(&pool.ctr[1], (unsigned long long)RG_LIMIT);
             base_lds = n > 0 ? atomicAdd(&pool.ctr[0], (unsigned long long)n) : 0;
             const bool fits = (int64_t)base_lds + n <= pool.cap;
-            if (!fits) atomicMax(&pool.ctr[1], (unsigned long long)RG_LIMIT);
+            if (!fits) atomicMax(&pool.ctr[1], (unsigned long long)RG_POOL);
             pool.seg[row] = {(int64_t)base_lds, fits ? (int64_t)n : 0};
         }
         __syncthreads();

@@ -135,8 +135,11 @@ def _finalize(dense, nb, E, final_max):
     return keys, total[keys]
 
 
-# Room for the final states of a chunk in the one-launch grounding (8 bytes an entry).
+# Room for the final states of a chunk in the one-launch grounding (8 bytes an entry): where a chunk asks for more it
+# is made larger, up to _POOL_GROWTH times (the states of the steps take 28 bytes an entry and more).
 _POOL_ENTRIES = 1 << 25
+_POOL_GROWTH = 8
+_POOL_FULL = 2  # fl_rule_ground's report
 
 
 def _grounds_in_one_launch(ev, csr, entities, device):
@@ -166,36 +169,44 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
     lengths_d = torch.tensor(lengths, dtype=torch.int32).to(device)
     st = fk._stream(sources)
     done = _progress() if done is None else done
+    widest = max(hi - lo for lo, hi in chunks)
+    limit = _POOL_ENTRIES
     for s0 in range(0, sources.numel(), block):
         src = sources[s0:s0 + block]
         nb = src.numel()
         dense = torch.zeros((ranks, nb * E), dtype=torch.float32, device=device)
-        words = torch.zeros(4, dtype=torch.int64, device=device)
-        status, info = words[:2], words[2:]
-        widest = max(hi - lo for lo, hi in chunks)
-        pool = min(nb * widest * E, _POOL_ENTRIES)
-        collect_bytes = lib.fl_rule_collect_bytes(nb, E)
-        ws_bytes = max(lib.fl_rule_ground_bytes(nb, widest, pool), collect_bytes)
-        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-        for lo, hi in chunks:
-            check(lib.fl_rule_ground(st, ctypes.byref(sides.ori), ctypes.byref(sides.inv), ptr(src), nb,
-                                     ptr(operators[lo:hi]), ptr(lengths_d[lo:hi]), hi - lo, operators.shape[1],
-                                     int(relations), ptr(weights[lo:hi]), ranks, E, 1 if boolean_paths else 0,
-                                     1 if is_max else 0, ptr(dense), pool, ptr(ws), ws_bytes, ptr(status)),
-                  "rule_ground")
         rowsum = torch.empty(ranks * nb, dtype=torch.float32, device=device)
         total = torch.empty(nb * E, dtype=torch.float32, device=device)
-        check(lib.fl_rule_finalize(st, ptr(dense), ranks, nb, E, 1 if final_max else 0, ptr(rowsum), ptr(total)),
-              "rule_finalize")
-        check(lib.fl_rule_collect_plan(st, ptr(total), nb, E, ptr(status), ptr(ws), ws_bytes, ptr(info)),
-              "rule_collect")
-        bad, added, count, _ = words.tolist()
-        if bad == 1:
-            raise ValueError("sparse state index out of range for shape (%d, %d, %d)" % (nb, widest, E))
-        stats["chunks"] += added
-        stats["ground_calls"] += sum(max(lengths[lo:hi]) for lo, hi in chunks[:added])
+        collect_bytes = lib.fl_rule_collect_bytes(nb, E)
+        first = 0  # chunks before it are in dense
+        while True:
+            words = torch.zeros(5, dtype=torch.int64, device=device)
+            status, info = words[:3], words[3:]
+            pool = min(nb * widest * E, limit)
+            ws_bytes = max(lib.fl_rule_ground_bytes(nb, widest, pool), collect_bytes)
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
+            for lo, hi in chunks[first:]:
+                check(lib.fl_rule_ground(st, ctypes.byref(sides.ori), ctypes.byref(sides.inv), ptr(src), nb,
+                                         ptr(operators[lo:hi]), ptr(lengths_d[lo:hi]), hi - lo, operators.shape[1],
+                                         int(relations), ptr(weights[lo:hi]), ranks, E, 1 if boolean_paths else 0,
+                                         1 if is_max else 0, ptr(dense), pool, ptr(ws), ws_bytes, ptr(status)),
+                      "rule_ground")
+            check(lib.fl_rule_finalize(st, ptr(dense), ranks, nb, E, 1 if final_max else 0, ptr(rowsum), ptr(total)),
+                  "rule_finalize")
+            check(lib.fl_rule_collect_plan(st, ptr(total), nb, E, ptr(status), ptr(ws), ws_bytes, ptr(info)),
+                  "rule_collect")
+            bad, added, wanted, count, _ = words.tolist()
+            if bad == 1:
+                raise ValueError("sparse state index out of range for shape (%d, %d, %d)" % (nb, widest, E))
+            stats["chunks"] += added
+            stats["ground_calls"] += sum(max(lengths[lo:hi]) for lo, hi in chunks[first:first + added])
+            first += added
+            done.dense, done.rule = dense, chunks[first][0] if first < len(chunks) else chunks[-1][1]
+            if bad != _POOL_FULL or wanted > _POOL_GROWTH * _POOL_ENTRIES:
+                break
+            limit = min(max(wanted, 2 * limit), _POOL_GROWTH * _POOL_ENTRIES)
+            del ws
         if bad:
-            done.dense, done.rule = dense, chunks[added][0]
             return None
         idx = torch.empty((2, count), dtype=torch.int64, device=device)
         vals = torch.empty(count, dtype=torch.float32, device=device)
@@ -203,7 +214,7 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
             check(lib.fl_rule_collect_fill(st, ptr(total), nb, E, s0, ptr(ws), ptr(idx[0]), ptr(idx[1]), ptr(vals)),
                   "rule_collect")
         done.parts.append((idx, vals))
-        done.source = s0 + nb
+        done.source, done.dense, done.rule = s0 + nb, None, 0
     return _joined(done.parts)
 
 

@@ -594,12 +594,14 @@ int fl_rule_finalize(void *stream, const float *dense, int64_t K, int64_t B,
  * [C, steps] (ids as the fixed-relation step takes them), lengths [C] a
  * rule's operators; boolean_paths: every state 0 or 1.  pool: room for that
  * many final state entries, at most nb * C * E are needed.  At most
- * fl_rule_ground_max_entities() entities.  status (device int64[2], zeroed
+ * fl_rule_ground_max_entities() entities.  status (device int64[3], zeroed
  * by the caller before the first of the calls that share it): [0] receives 1
- * when a source is outside [0, E), 2 when a path count reached 2^24, a row
- * passed 2^20 edges in a step or the pool was too small, [1] the calls whose
- * chunks were added to dense.  After a report neither that call nor a later
- * one adds to dense: the caller takes the steps one by one from there on. */
+ * when a source is outside [0, E), 2 when the pool was too small, 3 when a
+ * path count reached 2^24 or a row passed 2^20 edges in a step; [1] the calls
+ * whose chunks were added to dense, [2] the pool entries that the first call
+ * with a report asked for (of use with 2).  After a report neither that call
+ * nor a later one adds to dense: the caller goes on from there with a larger
+ * pool or takes the steps one by one. */
 int64_t fl_rule_ground_max_entities(void);
 size_t fl_rule_ground_bytes(int64_t nb, int64_t C, int64_t pool);
 int fl_rule_ground(void *stream, const fl_side *ori, const fl_side *inv,

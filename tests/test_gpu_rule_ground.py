@@ -176,6 +176,22 @@ def test_what_was_grounded_before_a_limit_is_kept(monkeypatch, at, block):
     assert len(calls) == 2 * (4 - at // 5)  # (every chunk has a body of two steps)
 
 
+@pytest.mark.parametrize("entries,fits", [(1400, True), (700, True), (175, True), (174, False)])
+def test_pool_grows(monkeypatch, entries, fits):
+    """Two final states of 700 entities each: the pool is made as large as they ask for, up to eight times."""
+    from flashlog_amd.rules import shared_inference as si
+    E, R = 1700, 3
+    monkeypatch.setattr(si, "_POOL_ENTRIES", entries)
+    calls = _counted_steps(monkeypatch)
+    h, r, t = _graph(E, [700], [([5], 2, [6])])
+    tc = to_torch_csr(O.build_csr_structure(h, t, r, E), torch.device("cuda"))
+    rules = [{"body": b, "rank_weights": [0.5, 0.25]} for b in ([2], [2], [2], [2], [2], [0], [0])]
+    got = _score(None, torch.tensor([0, 5]).cuda(), rules, tc, R, E, 5)
+    assert (calls == []) == fits
+    want = _score(_stepwise(), torch.tensor([0, 5]).cuda(), rules, tc, R, E, 5)
+    assert torch.equal(got.indices(), want.indices()) and torch.equal(got.values(), want.values())
+
+
 def test_rows_after_a_limit_are_left():
     """Chunks behind one that outgrew the kernels are not walked."""
     from flashlog_amd import _lib
