@@ -143,7 +143,7 @@ constexpr unsigned long long RG_PATHS_MAX = 1ull << 24;
 enum { RG_SOURCE = 1, RG_POOL = 2, RG_LIMIT = 3 };  // the larger report stands
 
 struct RgSeg {
-    int64_t base;
+    int64_t base;  // n == 0: the step, from 1, that left the row empty
     int64_t n;
 };
 
@@ -159,16 +159,34 @@ struct RgPool {
 constexpr int RG_CTR = 5;
 
 // status: [0] the worst report of the calls so far, [1] chunks added, [2] the
-// pool entries that the chunk of a first RG_POOL asks for
+// pool entries that the chunk of a first RG_POOL asks for, [3] the steps that
+// the added chunks would take one by one: a chunk's longest body, or as many
+// as leave every row empty
 __global__ void k_rg_zero(unsigned long long *ctr, const unsigned long long *status) {
     if (threadIdx.x < RG_CTR) ctr[threadIdx.x] = threadIdx.x == 1 || threadIdx.x == 4 ? *status : 0ull;
 }
 
-__global__ void k_rg_status(const unsigned long long *ctr, unsigned long long *status) {
+__global__ __launch_bounds__(RB_NT) void k_rg_status(RgPool pool, const int32_t *__restrict__ lens, int64_t C,
+                                                     int64_t rows, unsigned long long *status) {
+    __shared__ int steps;
+    if (threadIdx.x == 0) steps = 0;
+    __syncthreads();
+    int mine = 0;
+    if (pool.ctr[0] > 0) {  // some row is left: to the end of the longest body
+        for (int64_t r = threadIdx.x; r < C; r += RB_NT) mine = max(mine, (int)lens[r]);
+    } else {
+        for (int64_t r = threadIdx.x; r < rows; r += RB_NT) mine = max(mine, (int)pool.seg[r].base);
+    }
+    if (mine > 0) atomicMax(&steps, mine);
+    __syncthreads();
     if (threadIdx.x != 0) return;
-    if (ctr[1] == 0) status[1] += 1;
-    if (status[0] == 0) status[2] = ctr[0];
-    status[0] = ctr[1];
+    const unsigned long long report = pool.ctr[1];
+    if (report == 0) {
+        status[1] += 1;
+        status[3] += steps;
+    }
+    if (status[0] == 0) status[2] = pool.ctr[0];
+    status[0] = report;
 }
 
 // Expands n entries (get(i, node, count), count 0: no entry) through relation
@@ -251,12 +269,13 @@ __global__ __launch_bounds__(RG_NT) void k_rg_rows(fl_side ori, fl_side inv, con
     }
     int n = 1;
     bool limit = false, over = false;
-    for (int step = 0; step < lens[r] && n > 0; ++step) {
+    int step = 0;
+    for (; step < lens[r] && n > 0; ++step) {
         const int64_t op = ops[r * steps + step];
         if (op == 2 * R) continue;  // the identity
         if (op < 0 || op > 2 * R) {
             n = 0;
-            break;
+            continue;
         }
         __syncthreads();  // the last step's list is made, and its table read
         for (int q = t; q < RG_TAB; q += RG_NT) {
@@ -314,14 +333,14 @@ __global__ __launch_bounds__(RG_NT) void k_rg_rows(fl_side ori, fl_side inv, con
         return;
     }
     if (t == 0) {
-        base_lds = n > 0 ? atomicAdd(&pool.ctr[0], (unsigned long long)n) : 0;
-        const bool fits = (int64_t)base_lds + n <= pool.cap;
+        base_lds = n > 0 ? atomicAdd(&pool.ctr[0], (unsigned long long)n) : (unsigned long long)step;
+        const bool fits = n == 0 || (int64_t)base_lds + n <= pool.cap;
         if (!fits) atomicMax(&pool.ctr[1], (unsigned long long)RG_POOL);
         pool.seg[row] = {(int64_t)base_lds, fits ? (int64_t)n : 0};
     }
     __syncthreads();
     const int64_t base = (int64_t)base_lds;
-    if (base + n > pool.cap) return;
+    if (n == 0 || base + n > pool.cap) return;
     for (int i = t; i < n; i += RG_NT) {
         pool.ent[base + i] = node_of[i];
         pool.val[base + i] = (float)count_of[i];
@@ -361,12 +380,13 @@ __global__ __launch_bounds__(RG_DENSE_NT) void k_rg_dense(fl_side ori, fl_side i
         __syncthreads();
         if (t == 0) cur[sources[b]] = 1;  // (k_rg_rows checked the source)
         bool limit = false, none = false;
-        for (int step = 0; step < lens[r]; ++step) {
+        int step = 0;
+        for (; step < lens[r] && !none; ++step) {
             const int64_t op = ops[r * steps + step];
             if (op == 2 * R) continue;
             if (op < 0 || op > 2 * R) {
                 none = true;
-                break;
+                continue;
             }
             if (t == 0) paths_lds = 0;
             __syncthreads();
@@ -385,6 +405,7 @@ __global__ __launch_bounds__(RG_DENSE_NT) void k_rg_dense(fl_side ori, fl_side i
             __syncthreads();
             limit = items > RG_ITEMS_MAX || (!boolean && paths_lds >= RG_PATHS_MAX);
             if (limit) break;  // uniform
+            none = items == 0;
             for (int e = t; e < E; e += RG_DENSE_NT) {
                 cur[e] = 0;
                 if (boolean && nxt[e] > 1) nxt[e] = 1;
@@ -402,8 +423,8 @@ __global__ __launch_bounds__(RG_DENSE_NT) void k_rg_dense(fl_side ori, fl_side i
         const int at = fl_block_excl_scan<RG_DENSE_NT>(mine, scan_lds, &n);
         if (t == 0) {
             if (limit) atomicMax(&pool.ctr[1], (unsigned long long)RG_LIMIT);
-            base_lds = n > 0 ? atomicAdd(&pool.ctr[0], (unsigned long long)n) : 0;
-            const bool fits = (int64_t)base_lds + n <= pool.cap;
+            base_lds = n > 0 ? atomicAdd(&pool.ctr[0], (unsigned long long)n) : (unsigned long long)step;
+            const bool fits = n == 0 || (int64_t)base_lds + n <= pool.cap;
             if (!fits) atomicMax(&pool.ctr[1], (unsigned long long)RG_POOL);
             pool.seg[row] = {(int64_t)base_lds, fits ? (int64_t)n : 0};
         }
@@ -645,7 +666,8 @@ int fl_rule_ground(void *stream, const fl_side *ori, const fl_side *inv, const i
               *ori, *inv, sources, operators, lengths, C, steps, (int)E, r_size, boolean_paths, p);
     FL_LAUNCH("k_rg_sum", is_max ? k_rg_sum<true> : k_rg_sum<false>, dim3((unsigned)nb, (unsigned)K), dim3(RA_NT),
               sizeof(float) * (size_t)E, st, p, W, K, nb, C, E, dense);
-    FL_LAUNCH("k_rg_status", k_rg_status, dim3(1), dim3(64), 0, st, p.ctr, (unsigned long long *)status);
+    FL_LAUNCH("k_rg_status", k_rg_status, dim3(1), dim3(RB_NT), 0, st, p, lengths, C, nb * C,
+              (unsigned long long *)status);
     return fl_check_launch("rule_ground");
 }
 

@@ -161,7 +161,8 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
                          final_max, stats, done=None):
     """(indices, scores) of the blocks of sources with every chunk of rules grounded by one launch
     (fl_rule_ground) and the scored entities collected with one host read per block, or None when a state outgrew
-    what those kernels hold (the caller grounds step by step from where ``done`` says)."""
+    what those kernels hold (the caller grounds step by step from where ``done`` says).  ``lengths`` are of the
+    rules' bodies; stats["ground_calls"] counts the steps that the step-by-step form takes."""
     lib = _lib.lib()
     device = sources.device
     sides = fk._fixed_sides(csr)
@@ -180,8 +181,8 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
         collect_bytes = lib.fl_rule_collect_bytes(nb, E)
         first = 0  # chunks before it are in dense
         while True:
-            words = torch.zeros(5, dtype=torch.int64, device=device)
-            status, info = words[:3], words[3:]
+            words = torch.zeros(6, dtype=torch.int64, device=device)
+            status, info = words[:4], words[4:]
             pool = min(nb * widest * E, limit)
             ws_bytes = max(lib.fl_rule_ground_bytes(nb, widest, pool), collect_bytes)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
@@ -195,11 +196,11 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
                   "rule_finalize")
             check(lib.fl_rule_collect_plan(st, ptr(total), nb, E, ptr(status), ptr(ws), ws_bytes, ptr(info)),
                   "rule_collect")
-            bad, added, wanted, count, _ = words.tolist()
+            bad, added, wanted, steps, count, _ = words.tolist()
             if bad == 1:
                 raise ValueError("sparse state index out of range for shape (%d, %d, %d)" % (nb, widest, E))
             stats["chunks"] += added
-            stats["ground_calls"] += sum(max(lengths[lo:hi]) for lo, hi in chunks[first:first + added])
+            stats["ground_calls"] += steps
             first += added
             done.dense, done.rule = dense, chunks[first][0] if first < len(chunks) else chunks[-1][1]
             if bad != _POOL_FULL or wanted > _POOL_GROWTH * _POOL_ENTRIES:

@@ -594,12 +594,13 @@ int fl_rule_finalize(void *stream, const float *dense, int64_t K, int64_t B,
  * [C, steps] (ids as the fixed-relation step takes them), lengths [C] a
  * rule's operators; boolean_paths: every state 0 or 1.  pool: room for that
  * many final state entries, at most nb * C * E are needed.  At most
- * fl_rule_ground_max_entities() entities.  status (device int64[3], zeroed
+ * fl_rule_ground_max_entities() entities.  status (device int64[4], zeroed
  * by the caller before the first of the calls that share it): [0] receives 1
  * when a source is outside [0, E), 2 when the pool was too small, 3 when a
  * path count reached 2^24 or a row passed 2^20 edges in a step; [1] the calls
  * whose chunks were added to dense, [2] the pool entries that the first call
- * with a report asked for (of use with 2).  After a report neither that call
+ * with a report asked for (of use with 2), [3] the steps that the added chunks
+ * take one by one, up to one that leaves no state.  After a report neither that call
  * nor a later one adds to dense: the caller goes on from there with a larger
  * pool or takes the steps one by one. */
 int64_t fl_rule_ground_max_entities(void);

@@ -172,7 +172,7 @@ def test_what_was_grounded_before_a_limit_is_kept(monkeypatch, at, block):
     calls = _counted_steps(monkeypatch)
     got = _score(None, src, rules, tc, R, E, 5, stats=stats, **kw)
     assert torch.equal(got.indices(), want.indices()) and torch.equal(got.values(), want.values())
-    assert stats["chunks"] == want_stats["chunks"]
+    assert stats == want_stats
     assert len(calls) == 2 * (4 - at // 5)  # (every chunk has a body of two steps)
 
 
@@ -213,3 +213,22 @@ def test_rows_after_a_limit_are_left():
             _lib.prof_enable(False)
 
     assert walked([[2]] + [[3]] * 4) < walked([[3]])
+
+
+@pytest.mark.parametrize("kw", [{}, {"reduction": "max"}])
+@pytest.mark.parametrize("block", [None, 1])
+def test_stats_are_those_of_the_steps(kw, block):
+    """Steps whose states are all empty are not counted, also where a row dies late, only in the dense form, or where a
+    chunk's longest body is not its last to die."""
+    E, R = 1700, 5
+    h, r, t = _graph(E, [1600, 3], [([0], 3, [7]), ([7], 4, [8])])
+    tc = to_torch_csr(O.build_csr_structure(h, t, r, E), torch.device("cuda"))
+    kw = dict(kw) if block is None else dict(kw, dense_budget_bytes=block * 2 * E * 4)
+    for bodies in ([[3, 3, 3]], [[3, 3, 3], [3]], [[3, 4, 4]], [[3], []], [[0, 0, 2]], [[0, 2, 3, 4]], [[0, 2], [3, 3, 3]],
+                   [[3, 2 * R, 3, 3]], [[3, 4]] * 5 + [[3, 3, 2]] * 5 + [[1]], [[3, 2 * R + 3, 0]]):
+        rules = [{"body": b, "rank_weights": [0.5, 0.25]} for b in bodies]
+        want, got = {}, {}
+        a = _score(_stepwise(), torch.tensor([0, 7]).cuda(), rules, tc, R, E, 5, stats=want, **kw)
+        b = _score(None, torch.tensor([0, 7]).cuda(), rules, tc, R, E, 5, stats=got, **kw)
+        assert torch.equal(a.indices(), b.indices()) and torch.equal(a.values(), b.values())
+        assert got == want, bodies
