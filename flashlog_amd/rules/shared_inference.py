@@ -314,6 +314,7 @@ def score(ev, sources, rules, csr, relations, entities, chunk_size,
         except torch.cuda.OutOfMemoryError:
             found = None  # step by step, with chunks halved as far as needed
             torch.cuda.empty_cache()
+            stats["oom_retries"] += 1
         if found is not None:
             return torch.sparse_coo_tensor(*found, shape, is_coalesced=True)
 

@@ -232,3 +232,18 @@ def test_stats_are_those_of_the_steps(kw, block):
         b = _score(None, torch.tensor([0, 7]).cuda(), rules, tc, R, E, 5, stats=got, **kw)
         assert torch.equal(a.indices(), b.indices()) and torch.equal(a.values(), b.values())
         assert got == want, bodies
+
+
+def test_out_of_memory_is_counted(monkeypatch):
+    from flashlog_amd.rules import shared_inference as si
+
+    def full(*a):
+        raise torch.cuda.OutOfMemoryError("full")
+
+    monkeypatch.setattr(si, "_score_in_one_launch", full)
+    E, R = 50, 3
+    h, r, t = _graph(E, [2])
+    tc = to_torch_csr(O.build_csr_structure(h, t, r, E), torch.device("cuda"))
+    stats = {}
+    got = _score(None, torch.tensor([0, 1]).cuda(), [{"body": [0], "rank_weights": [0.5]}], tc, R, E, 5, stats=stats)
+    assert got._nnz() == 2 and stats["oom_retries"] == 1
