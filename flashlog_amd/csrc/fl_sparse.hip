@@ -3477,16 +3477,29 @@ __device__ __forceinline__ float block_tree_sum(float v, float *red) {
 // values in entry (= output key) order, as the CPU path adds them
 // (flashlog.cpp:1561-1565).  The clamp is the GPU path's (flashlog.cu:2540):
 // d >= eps ? d : eps, so a NaN sum divides by eps.
-//   The chain of dependent adds bounds it.  The first wave does nothing else:
-// its first thread adds chunk c from LDS and the other waves bring in chunk
-// c + 1 meanwhile.
-// The row's range is searched by the workgroup itself (row_ptr is kept for
-// the backward), so that the normalizer is one launch.
-//   Rows of 14,000 values: 85 us; with the chunk loaded by all waves 98 us.
-// Composing the adds of a binade as maps of the mantissa's parity, in
-// parallel, took 95 us.
+//   Up to NF_SELF_ROWS rows (SELF) the chain of dependent adds bounds it.  The
+// first wave does nothing else: its first thread adds chunk c from LDS and the
+// other waves bring in chunk c + 1 meanwhile.  The row's range is searched by
+// the workgroup itself (row_ptr is kept for the backward), so that the
+// normalizer is one launch.  (Rows of 14,000 values: 85 us; with the chunk
+// loaded by all waves 98 us.  Composing the adds of a binade as maps of the
+// mantissa's parity, in parallel, took 95 us.)
+//   With more rows than twice the 2000 workgroups that run at a time the
+// others' work hides a workgroup's waits and the number of instructions
+// counts: k_norm_rows finds all rows first, a thread a row, and all waves load
+// each chunk.  (4000 rows of 4 values 43 us a call searched by the workgroups
+// against 48; 8000 of 200 73 against 46, 200,000 of 4 782 against 153, and 180
+// with the rows found first but the waves' work split.)
 constexpr int NF_CHUNK = 2048;
+constexpr int64_t NF_SELF_ROWS = 4096;
 
+__global__ void k_norm_rows(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl, int64_t nnz, int64_t L,
+                            int64_t R, int64_t *__restrict__ row_ptr) {
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r <= R) row_ptr[r] = sp_row_start(sb, sl, nnz, L, R, r);
+}
+
+template <bool SELF>
 __global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ sb, const int64_t *__restrict__ sl,
                                                    int64_t nnz, int64_t L, int64_t R, const float *__restrict__ v,
                                                    float eps, float *__restrict__ out, float *__restrict__ denom,
@@ -3496,33 +3509,40 @@ __global__ __launch_bounds__(NM_NT) void k_norm_fwd(const int64_t *__restrict__ 
     __shared__ int64_t range[2];
     const int64_t r = blockIdx.x;
     const int t = threadIdx.x;
-    if (t < 2) {
+    if (SELF && t < 2) {
         const int64_t p = sp_row_start(sb, sl, nnz, L, R, r + t);
         range[t] = p;
         if (t == 0 || r == R - 1) row_ptr[r + t] = p;
     }
     if (r == 0 && t == 0) *err = 0;
-    __syncthreads();
-    const int64_t a = range[0], b = range[1];
-    {
-        const int len = (int)((b - a) < NF_CHUNK ? (b - a) : NF_CHUNK);
-        float *cb = (float *)buf[0];
-        for (int i = t; i < len; i += NM_NT) cb[i] = v[a + i];
-    }
-    __syncthreads();
+    if (SELF) __syncthreads();
+    const int64_t a = SELF ? range[0] : row_ptr[r], b = SELF ? range[1] : row_ptr[r + 1];
     float acc = 0.0f;
     int c = 0;
-    for (int64_t base = a; base < b; base += NF_CHUNK, ++c) {
-        if (t >= FL_WAVE) {
-            const int64_t left = b - base - NF_CHUNK;
-            const int len = (int)(left < NF_CHUNK ? left : NF_CHUNK);  // (<= 0 behind the last chunk)
-            float *cb = (float *)buf[(c + 1) & 1];
-#pragma unroll 4
-            for (int i = t - FL_WAVE; i < len; i += NM_NT - FL_WAVE) cb[i] = v[base + NF_CHUNK + i];
-        } else if (t == 0) {
-            acc = sp_fold(acc, (const float *)buf[c & 1], 0, (int)((b - base) < NF_CHUNK ? (b - base) : NF_CHUNK));
-        }
+    if constexpr (SELF) {
+        const int len0 = (int)((b - a) < NF_CHUNK ? (b - a) : NF_CHUNK);
+        for (int i = t; i < len0; i += NM_NT) ((float *)buf[0])[i] = v[a + i];
         __syncthreads();
+        for (int64_t base = a; base < b; base += NF_CHUNK, ++c) {
+            if (t >= FL_WAVE) {
+                const int64_t left = b - base - NF_CHUNK;
+                const int len = (int)(left < NF_CHUNK ? left : NF_CHUNK);  // (<= 0 behind the last chunk)
+                float *cb = (float *)buf[(c + 1) & 1];
+#pragma unroll 4
+                for (int i = t - FL_WAVE; i < len; i += NM_NT - FL_WAVE) cb[i] = v[base + NF_CHUNK + i];
+            } else if (t == 0) {
+                acc = sp_fold(acc, (const float *)buf[c & 1], 0, (int)((b - base) < NF_CHUNK ? (b - base) : NF_CHUNK));
+            }
+            __syncthreads();
+        }
+    } else {
+        for (int64_t base = a; base < b; base += NF_CHUNK, ++c) {
+            const int len = (int)((b - base) < NF_CHUNK ? (b - base) : NF_CHUNK);
+            float *cb = (float *)buf[c & 1];
+            for (int i = t; i < len; i += NM_NT) cb[i] = v[base + i];
+            __syncthreads();
+            if (t == 0) acc = sp_fold(acc, cb, 0, len);
+        }
     }
     if (t == 0) {
         dsh = acc;
@@ -4460,9 +4480,12 @@ int fl_sparse_normalize_forward(void *stream, const int64_t *sp_b, const int64_t
     hipStream_t st = (hipStream_t)stream;
     // the reference's GPU path checks no order either (flashlog.cu:2594-2649):
     // row starts by binary search, err cleared
+    if (R > NF_SELF_ROWS)
+        FL_LAUNCH("k_norm_rows", k_norm_rows, dim3((unsigned)(R / 256 + 1)), dim3(256), 0, st, sp_b, sp_l, nnz, L, R,
+                  row_ptr);
     if (R > 0)
-        FL_LAUNCH("k_norm_fwd", k_norm_fwd, dim3((unsigned)R), dim3(NM_NT), 0, st, sp_b, sp_l, nnz, L, R, v, eps, out,
-                  denom, row_ptr, err);
+        FL_LAUNCH("k_norm_fwd", R > NF_SELF_ROWS ? k_norm_fwd<false> : k_norm_fwd<true>, dim3((unsigned)R),
+                  dim3(NM_NT), 0, st, sp_b, sp_l, nnz, L, R, v, eps, out, denom, row_ptr, err);
     else
         FL_LAUNCH("k_fill_i64", k_fill_i64, dim3(1), dim3(64), 0, st, row_ptr, (int64_t)1, (int64_t)0, err,
                   (int64_t)1);
