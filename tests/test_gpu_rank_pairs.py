@@ -61,3 +61,39 @@ def test_shapes_of_filter_and_targets():
     for targets, pair in ((t[:, None], (t, t)), (t, (t, t[:1])), (t, (t[:, None], t[:, None]))):
         with pytest.raises(ValueError, match="1D"):
             fk.dense_filtered_ranks_cuda(state, targets, pair)
+
+
+@pytest.mark.parametrize("order", ["in runs", "mixed"])
+def test_pairs_given_many_times(order):
+    """A few pairs, each given thousands of times, are counted once."""
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    B, E = 7, 300
+    g = torch.Generator().manual_seed(3)
+    scores = torch.randint(0, 5, (B, E), generator=g).float().cuda()
+    targets = torch.randint(0, E, (B,), generator=g).cuda()
+    fb, fe = torch.randint(0, B, (9,), generator=g), torch.randint(0, E, (9,), generator=g)
+    want = fk.dense_filtered_ranks_cuda(scores, targets, (fb.cuda(), fe.cuda()), True)
+    pick = torch.randint(0, 9, (20_000,), generator=g)
+    if order == "in runs":
+        pick = pick.sort().values
+    got = fk.dense_filtered_ranks_cuda(scores, targets, (fb[pick].cuda(), fe[pick].cuda()), True)
+    assert torch.equal(got, want)
+
+
+def test_one_pair_given_many_times_is_not_slow():
+    """Every one of 20,000 threads put the same pair into the table: 200 us of atomics on one word."""
+    from flashlog_amd import _lib
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    B, E = 509, 14500
+    scores = torch.rand(B, E, device="cuda")
+    targets = torch.zeros(B, dtype=torch.int64, device="cuda")
+    pair = torch.zeros(20_000, dtype=torch.int64, device="cuda")
+    fk.dense_filtered_ranks_cuda(scores, targets, (pair, pair))
+    _lib.prof_enable(True)
+    try:
+        for _ in range(10):
+            fk.dense_filtered_ranks_cuda(scores, targets, (pair, pair))
+        ms, launches = _lib.prof_read("k_dr_filter")
+    finally:
+        _lib.prof_enable(False)
+    assert launches == 10 and ms / launches < 0.07
