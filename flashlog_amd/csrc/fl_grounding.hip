@@ -1402,6 +1402,8 @@ struct GrWalkLayout {
     size_t hub_hdr, hub_cum, hub_opt, hub_list;  // byte offsets of the hub cache (ncombo > 0)
 };
 
+constexpr int64_t GR_HUB_SCRATCH = 256 << 20;
+
 GrWalkLayout gr_walk_layout(const fl_ground_graph *g, int64_t ntasks, int64_t nheads, int64_t ranks) {
     GrWalkLayout L{};
     L.pmax = 128;
@@ -1413,9 +1415,13 @@ GrWalkLayout gr_walk_layout(const fl_ground_graph *g, int64_t ntasks, int64_t nh
     L.hub_waves = 0;
     if (g->nhub > 0 && g->hub_options > 0 && nheads > 0 && ranks > 0) {
         // the lists are ranked by as many waves as the chip holds, whatever
-        // the number of tasks
+        // the number of tasks; where a node has so many groups that their
+        // scratch passes GR_HUB_SCRATCH, by as many as that holds or the
+        // tasks have (2 MB a wave at 32,767 groups, 16 GB for all)
         L.ncombo = nheads * 3 * ranks;
         L.hub_waves = L.ncombo * g->nhub < 8192 ? L.ncombo * g->nhub : 8192;
+        const int64_t room = GR_HUB_SCRATCH / (int64_t)L.stride > L.waves ? GR_HUB_SCRATCH / (int64_t)L.stride : L.waves;
+        if (L.hub_waves > room) L.hub_waves = room > 0 ? room : 1;
     }
     const int64_t strides = L.waves > L.hub_waves ? L.waves : L.hub_waves;
     L.bytes = L.stride * (size_t)(strides > 0 ? strides : 1);

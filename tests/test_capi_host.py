@@ -94,3 +94,17 @@ def test_pull_index_is_destination_major_in_position_order():
             assert np.array_equal(seg_start[segs], pp[d] + _lib().FL_SEG * np.arange(segs.size))
             sups = np.arange(hup[k], hup[k + 1])
             assert np.array_equal(sup_seg0[sups], hsp[k] + _lib().FL_SUP * np.arange(sups.size))
+
+
+@pytest.mark.parametrize("max_groups", [1, 200, 822, 32767])
+@pytest.mark.parametrize("ntasks", [1, 16, 8192, 20000])
+def test_ground_walk_scratch_is_bounded(max_groups, ntasks):
+    """Ranking the option lists asks for no more scratch than the tasks' own walks, or 256 MiB."""
+    L = _lib()
+    g = L.FlGroundGraph()
+    g.nodes, g.num_relations, g.max_groups = 1000, 40000, max_groups
+    heads, ranks = 16, 3
+    walks = L.lib().fl_ground_walk_bytes(ctypes.byref(g), ntasks, heads, ranks)  # without lists
+    g.nhub, g.hub_options = 1000, 50000
+    lists = 3 * heads * ranks * (24 * g.hub_options + 16 * g.nhub) + 4 * g.nhub + 5 * 256
+    assert L.lib().fl_ground_walk_bytes(ctypes.byref(g), ntasks, heads, ranks) <= max(walks, 256 << 20) + lists
