@@ -2531,6 +2531,36 @@ __global__ __launch_bounds__(SP_NT) void k_sp_max_hot(SpRows rows, const int64_t
     }
 }
 
+// The value keys of a bucket that holds a NaN.  As in a scan of a
+// destination's items (sp_max_one) a NaN that comes first stays, for no value
+// is above it, and a later one is above none: the first position of every
+// destination decides whether its key is the NaN's (tbest keeps that position
+// then, the smallest (tie key, position) there is) or the largest of the values.
+__device__ __forceinline__ void sp_max_hot_nan(int wmask, const int32_t *dst, const float *val, int64_t n,
+                                            uint32_t *vbest, unsigned long long *tbest) {
+    const uint32_t inf_key = fl_order_key(__uint_as_float(0x7F800000u));
+    const int t = threadIdx.x;
+    for (int q = t; q <= wmask; q += SP_NT) {
+        vbest[q] = 0u;
+        tbest[q] = ~0ull;
+    }
+    __syncthreads();
+    for (int64_t k = t; k < n; k += SP_NT)
+        if (dst[k] >= 0) atomicMin(&tbest[dst[k] & wmask], (unsigned long long)k);
+    __syncthreads();
+    for (int64_t k = t; k < n; k += SP_NT) {
+        if (dst[k] < 0) continue;
+        const int dl = dst[k] & wmask;
+        const float v = val[k];
+        if (v == v) atomicMax(&vbest[dl], fl_order_key(sp_canon(v)));
+        else if (tbest[dl] == (unsigned long long)k) atomicMax(&vbest[dl], fl_order_key(fabsf(v)));
+    }
+    __syncthreads();
+    for (int q = t; q <= wmask; q += SP_NT)
+        if (vbest[q] <= inf_key) tbest[q] = ~0ull;
+    __syncthreads();
+}
+
 __device__ __forceinline__ void sp_max_hot_one(SpRows rows, int64_t start, int64_t n, int64_t slot, int32_t dbase,
                                                int32_t *__restrict__ dst_arr, float *__restrict__ val_arr,
                                                const uint32_t *__restrict__ tie_arr, int32_t *__restrict__ raw_local,
@@ -2556,12 +2586,15 @@ __device__ __forceinline__ void sp_max_hot_one(SpRows rows, int64_t start, int64
         if (key > vbest[dl]) atomicMax(&vbest[dl], key);
         const uint32_t b = 1u << (dl & 31);
         if (!(bits[dl >> 5] & b)) atomicOr(&bits[dl >> 5], b);
-        if (fb && v != v) *nan_seen = 1;
+        if (v != v) *nan_seen = 1;
     }
     __syncthreads();
-    if (fb && *nan_seen) {  // uniform: a NaN among the items of a mid-size bucket
-        if (t == 0) fb[atomicAdd(fb_ctr, 1)] = (int32_t)slot;
-        return;
+    if (*nan_seen) {  // uniform: a NaN among the items
+        if (fb) {  // of a mid-size bucket
+            if (t == 0) fb[atomicAdd(fb_ctr, 1)] = (int32_t)slot;
+            return;
+        }
+        sp_max_hot_nan(wmask, dst_arr + start, val_arr + start, n, vbest, tbest);
     }
 #pragma unroll 4
     for (int64_t k = t; k < n; k += SP_NT) {
