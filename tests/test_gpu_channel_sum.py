@@ -140,3 +140,78 @@ def test_channel_max_special_values(seed):
     (got.values() * g).sum().backward()
     (ref.values() * g).sum().backward()
     assert torch.equal(vt.grad.view(torch.int32), vr.grad.view(torch.int32))
+
+
+def _channel_case(seed, ties=False):
+    dev = torch.device("cuda:0")
+    B, L, E = 4, 3, 60
+    b, l, e, v = _state(seed, B, L, E, 300)
+    if ties:
+        v = (np.random.default_rng(seed).integers(1, 6, b.size) / 8.0).astype(np.float32)
+    idx = torch.stack([torch.from_numpy(x).to(dev) for x in (b, l, e)])
+    return B, L, E, idx, torch.from_numpy(v).to(dev)
+
+
+@pytest.mark.parametrize("op", ["sum", "max"])
+@pytest.mark.parametrize("how", ["to_dense", "dense", "other pattern", "uncoalesced", "empty", "strided"])
+def test_gradients_of_other_forms(op, how):
+    """A gradient that is dense, or sparse with other entries than the output, gives what its value at every output
+    gives: 0 where it has none."""
+    fk = _fk()
+    B, L, E, idx, v = _channel_case(31, ties=op == "max")
+    reduce = fk.sum_sp_3d if op == "sum" else fk.max_sp_3d
+    g = torch.randn(B, E, generator=torch.Generator().manual_seed(5)).cuda()
+    if how == "other pattern":   # every third cell, and some that the output does not have
+        g = g * (torch.arange(B * E, device="cuda").view(B, E) % 3 == 0)
+        up = g.to_sparse()
+    elif how == "uncoalesced":   # halves, each cell twice: exact sums
+        half = (g * 0.5).to_sparse()
+        up = torch.sparse_coo_tensor(half.indices().repeat(1, 2), half.values().repeat(2), (B, E))
+    elif how == "empty":
+        g = torch.zeros_like(g)
+        up = g.to_sparse()
+    elif how == "strided":
+        full = g.to_sparse()
+        up = torch.sparse_coo_tensor(full.indices().t().contiguous().t(), full.values(), (B, E), is_coalesced=True)
+    vr = v.clone().requires_grad_(True)
+    ref = _torch_sum(idx[0], idx[2], vr, B, E, None) if op == "sum" else \
+        _reference_max_sp_3d(torch.sparse_coo_tensor(idx, vr, (B, L, E)))
+    want, = torch.autograd.grad(ref.values(), [vr], g[tuple(ref.indices())])
+    vt = v.clone().requires_grad_(True)
+    out = reduce(torch.sparse_coo_tensor(idx, vt, (B, L, E), is_coalesced=True))
+    if how == "to_dense":
+        got, = torch.autograd.grad(out.to_dense(), [vt], g)
+    elif how == "dense":
+        ctx_grad = fk._channel_grad(g, out.indices(), E)
+        assert torch.equal(ctx_grad, g[tuple(out.indices())])
+        return
+    else:
+        got, = torch.autograd.grad(out, [vt], up)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("op", ["sum", "max"])
+@pytest.mark.parametrize("form", ["values", "dense"])
+def test_second_derivative(op, form):
+    """A gradient with a graph of its own: its derivative by the upstream gradient."""
+    fk = _fk()
+    B, L, E, idx, v = _channel_case(32, ties=op == "max")
+    reduce = fk.Sparse3DChannelSumFunction if op == "sum" else fk.Sparse3DChannelMaxFunction
+    vt = v.clone().requires_grad_(True)
+    out = reduce.apply(*idx, vt, B, L, E)  # (torch's own backward of a sparse state's values is not differentiable)
+    y = out.values() if form == "values" else out.to_dense()
+    u = torch.randn_like(y.detach()).requires_grad_(True)
+    gv, = torch.autograd.grad(y, [vt], u, create_graph=True)
+    p = torch.randn_like(gv)
+    got, = torch.autograd.grad(gv, [u], p)
+    # gv is linear in u: its transpose, from the same backward on every unit of u in turn
+    at = out.indices() if form == "values" else None
+    vr = v.clone().requires_grad_(True)
+    dense = torch.zeros(B, L, E, dtype=torch.float64, device="cuda").index_put(tuple(idx), vr.double())
+    share = torch.autograd.grad(dense.sum(1) if op == "sum" else dense.amax(1), [vr],
+                                torch.ones(B, E, dtype=torch.float64, device="cuda"))[0].double()
+    want = torch.zeros(B, E, dtype=torch.float64, device="cuda").index_put((idx[0], idx[2]), share * p.double(),
+                                                                          accumulate=True)
+    want = want[tuple(at)] if at is not None else want
+    # at most three float32 products and additions
+    torch.testing.assert_close(got.double(), want, rtol=6 * 2.0 ** -24, atol=6 * 2.0 ** -24 * float(p.abs().max()))

@@ -97,3 +97,20 @@ def test_one_pair_given_many_times_is_not_slow():
     finally:
         _lib.prof_enable(False)
     assert launches == 10 and ms / launches < 0.07
+
+
+@pytest.mark.parametrize("B,E,n", [(1, 5, 0), (3, 257, 40), (64, 3001, 2000)])
+@pytest.mark.parametrize("use_eql", [False, True])
+def test_sorted_keys(B, E, n, use_eql):
+    """The C entry that takes the filter as sorted unique keys, targets among them."""
+    from flashlog_amd import _lib
+    from flashlog_amd.flashlog_kernel import flashlog_kernel as fk
+    g = torch.Generator().manual_seed(n)
+    state = (torch.randint(0, 6, (B, E), generator=g) / 4).float().cuda()
+    targets = torch.randint(0, E, (B,), generator=g).cuda()
+    fb, fe = torch.randint(0, B, (n,), generator=g).cuda(), torch.randint(0, E, (n,), generator=g).cuda()
+    keys = torch.unique(torch.cat([fb * E + fe, torch.arange(B, device="cuda") * E + targets]))
+    ranks = torch.empty(B, device="cuda")
+    _lib.check(_lib.lib().fl_dense_filtered_ranks(fk._stream(state), _lib.ptr(state), _lib.ptr(targets), _lib.ptr(keys),
+                                                  keys.numel(), B, E, 1 if use_eql else 0, _lib.ptr(ranks)), "ranks")
+    assert torch.equal(ranks, fk.dense_filtered_ranks_cuda(state, targets, (fb, fe), use_eql))
