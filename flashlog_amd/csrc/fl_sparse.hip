@@ -3152,8 +3152,7 @@ constexpr int64_t SP_ONE_MAX = SP_ONE_NT * SP_ONE_PER;
 
 template <typename Get, typename Put>
 __device__ __forceinline__ int64_t sp_one_scan(int64_t n, long long *w64, Get get, Put put) {
-    // exclusive prefix sums of get(i), i < n (their total fits 32 bits or the
-    // hop does not take this path)
+    // exclusive prefix sums of get(i), i < n, in 64 bits
     const int t = threadIdx.x;
     int64_t x[SP_ONE_PER], sum = 0;
 #pragma unroll
