@@ -170,22 +170,24 @@ __global__ __launch_bounds__(RB_NT) void k_rg_status(RgPool pool, const int32_t 
                                                      int64_t rows, unsigned long long *status) {
     __shared__ int steps;
     if (threadIdx.x == 0) steps = 0;
-    __syncthreads();
-    int mine = 0;
-    if (pool.ctr[0] > 0) {  // some row is left: to the end of the longest body
-        for (int64_t r = threadIdx.x; r < C; r += RB_NT) mine = max(mine, (int)lens[r]);
-    } else {
+    // (the words, which the common case needs, are requested together)
+    const unsigned long long taken = pool.ctr[0], report = pool.ctr[1];
+    const unsigned long long before = status[0], added = status[1], done = status[3];
+    int mine = 0;  // some row is left: to the end of the longest body
+    for (int64_t r = threadIdx.x; r < C; r += RB_NT) mine = max(mine, (int)lens[r]);
+    if (taken == 0) {
+        mine = 0;
         for (int64_t r = threadIdx.x; r < rows; r += RB_NT) mine = max(mine, (int)pool.seg[r].base);
     }
+    __syncthreads();
     if (mine > 0) atomicMax(&steps, mine);
     __syncthreads();
     if (threadIdx.x != 0) return;
-    const unsigned long long report = pool.ctr[1];
     if (report == 0) {
-        status[1] += 1;
-        status[3] += steps;
+        status[1] = added + 1;
+        status[3] = done + steps;
     }
-    if (status[0] == 0) status[2] = pool.ctr[0];
+    if (before == 0) status[2] = taken;
     status[0] = report;
 }
 
@@ -254,10 +256,11 @@ __global__ __launch_bounds__(RG_NT) void k_rg_rows(fl_side ori, fl_side inv, con
     __shared__ unsigned long long paths_lds, base_lds;
     const int t = threadIdx.x;
     const int64_t row = blockIdx.x, b = row / C, r = row - b * C;
+    // (both are requested before either is looked at)
+    const unsigned long long before = pool.ctr[4];
     const int64_t src = sources[b];
-    if (pool.ctr[4] != 0) return;  // uniform: nothing of this chunk is used
-    if (src < 0 || src >= E) {  // uniform
-        if (t == 0) {
+    if ((before != 0) | (src < 0) | (src >= E)) {  // uniform
+        if (before == 0 && t == 0) {               // else nothing of this chunk is used
             atomicMax(&pool.ctr[1], (unsigned long long)RG_SOURCE);
             pool.seg[row] = {0, 0};
         }

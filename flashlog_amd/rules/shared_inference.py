@@ -181,8 +181,8 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
         collect_bytes = lib.fl_rule_collect_bytes(nb, E)
         first = 0  # chunks before it are in dense
         while True:
-            words = torch.zeros(6, dtype=torch.int64, device=device)
-            status, info = words[:4], words[4:]
+            words = torch.zeros(6, dtype=torch.int64, device=device)  # fl_rule_ground's status, fl_rule_collect's info
+            status, info = ptr(words), ctypes.c_void_p(words.data_ptr() + 4 * 8)
             pool = min(nb * widest * E, limit)
             ws_bytes = max(lib.fl_rule_ground_bytes(nb, widest, pool), collect_bytes)
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
@@ -190,12 +190,11 @@ def _score_in_one_launch(sources, chunks, operators, lengths, weights, csr, rela
                 check(lib.fl_rule_ground(st, ctypes.byref(sides.ori), ctypes.byref(sides.inv), ptr(src), nb,
                                          ptr(operators[lo:hi]), ptr(lengths_d[lo:hi]), hi - lo, operators.shape[1],
                                          int(relations), ptr(weights[lo:hi]), ranks, E, 1 if boolean_paths else 0,
-                                         1 if is_max else 0, ptr(dense), pool, ptr(ws), ws_bytes, ptr(status)),
+                                         1 if is_max else 0, ptr(dense), pool, ptr(ws), ws_bytes, status),
                       "rule_ground")
             check(lib.fl_rule_finalize(st, ptr(dense), ranks, nb, E, 1 if final_max else 0, ptr(rowsum), ptr(total)),
                   "rule_finalize")
-            check(lib.fl_rule_collect_plan(st, ptr(total), nb, E, ptr(status), ptr(ws), ws_bytes, ptr(info)),
-                  "rule_collect")
+            check(lib.fl_rule_collect_plan(st, ptr(total), nb, E, status, ptr(ws), ws_bytes, info), "rule_collect")
             bad, added, wanted, steps, count, _ = words.tolist()
             if bad == 1:
                 raise ValueError("sparse state index out of range for shape (%d, %d, %d)" % (nb, widest, E))
