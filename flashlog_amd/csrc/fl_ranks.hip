@@ -263,10 +263,11 @@ constexpr int DR_NT = 256;
 // once: a pair is inserted into a hash table of keys b*E + e (at least twice
 // as many slots as pairs: the probing ends), and the thread that inserted it
 // adds its entity to the row's filtered counts.  Integer counts: any order
-// gives the same.  A wave's pairs equal to the one before are left out of the
-// table: 20,000 times one pair, 278 -> 51 us a call.  (A sort of the pairs and checks of their ranges by
-// reductions took 230 of the 285 us of a call with 509 x 40 pairs, most of
-// it launches and host reads.)  err: 1 a target out of range, 2 a pair.
+// gives the same.  A pair equal to the one of the lane before is left to that
+// lane (20,000 times one pair, 278 -> 51 us a call).  (A sort of the pairs and
+// checks of their ranges by reductions took 230 of the 285 us of a call with
+// 509 x 40 pairs, most of it launches and host reads.)  err: 1 a target out of
+// range, 2 a pair.
 constexpr unsigned long long DR_EMPTY = ~0ull;
 
 __global__ void k_dr_init(unsigned long long *table, int64_t slots, uint32_t *counts, int64_t ncounts,
